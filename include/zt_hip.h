@@ -571,6 +571,44 @@ long zt_q5_0_gpu_qs_offset(long nblk);
 long zt_q5_0_gpu_bytes(long nblk);
 void zt_q5_0_raw_to_gpu(const void* raw, long nblk, void* out);
 
+/* ---- Wide batches ------------------------------------------------------ */
+
+/* C[T, rows] = X[T, K] W[rows, K]^T for T tokens, X and C row-major by token:
+ * the shape of a prompt's prefill and of wide decode batches, where the
+ * reference dequantizes and runs a dense GEMM (matMulQ4BWeight,
+ * dequantSgemm, compute/gpu_engine.go:2115-2255; MatMulW4A16,
+ * compute/w4a16.go:64-119).  W is the layout batch 1 reads:
+ *   ZT_WIDE_W4A16    packed nibbles and szr (zt_w4a16_pack_szr), group_size %
+ *                    128 == 0, fp16 X;
+ *   ZT_WIDE_Q4_0     RawBytesGPU, offset1 = the data offset (zt_gemm_q4_f32);
+ *   ZT_WIDE_Q8_0     zt_q8_raw_to_gpu, offset1 = the data offset;
+ *   ZT_WIDE_Q8_GGUF  zt_q8gguf_raw_to_gpu, offset1 = the data offset;
+ *   ZT_WIDE_Q5_0     zt_q5_0_raw_to_gpu, offset1 / offset2 = the qh / qs offset;
+ *   ZT_WIDE_Q4_K, ZT_WIDE_Q5_K   the raw super-blocks;
+ *   ZT_WIDE_Q6_K     zt_q6k_split;
+ *   ZT_WIDE_IQ4_NL   zt_iq4nl_raw_to_gpu, offset1 = the data offset, fp16 or fp32 X.
+ * The others take fp32 X.  Weights enter as exact fp16 integers (IQ4_NL's
+ * codebook and Q6_K's scaled values as fp16 hi + lo), fp32 activations as
+ * fp16 hi + lo after a power-of-two scale per token, sums are fp32; every
+ * output is written once and repeats bit for bit.  K % 128 == 0 (K-quants:
+ * 256), K <= 32768, bulk data below 2^31 bytes; W, X, the offsets and the
+ * workspace 16-byte aligned.  The workspace holds the packed activations
+ * (zt_gemm_wide_workspace_bytes, -1 for a size or type the path does not
+ * take); other calls -> InvalidValue. */
+#define ZT_WIDE_W4A16 0
+#define ZT_WIDE_Q4_0 1
+#define ZT_WIDE_Q8_0 2
+#define ZT_WIDE_Q8_GGUF 3
+#define ZT_WIDE_Q5_0 4
+#define ZT_WIDE_Q4_K 5
+#define ZT_WIDE_Q5_K 6
+#define ZT_WIDE_Q6_K 7
+#define ZT_WIDE_IQ4_NL 8
+long zt_gemm_wide_workspace_bytes(int fmt, int x_fp16, int rows, int K, int T);
+int zt_gemm_wide_f32(int fmt, const void* W, long offset1, long offset2, const uint32_t* szr, int group_size,
+                     const void* X, int x_fp16, float* C, int rows, int K, int T, void* workspace,
+                     long workspace_bytes, zt_stream_t stream);
+
 /* ---- int4 / int8 GEMMs with fp32 activations -------------------------- */
 
 /* The reference's group-quantized int4 and plain int8 GEMMs

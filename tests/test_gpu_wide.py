@@ -1,0 +1,222 @@
+"""The wide-batch GEMM (zt_gemm_wide_f32 and the engine's batches past 16
+tokens) against the oracle's dequantizers and a float64 product.
+
+Bar per output: |y - ref| <= (K / 32 + 24) 2^-24 sum |w x| + 2^-38 max|x| sum|w|.
+The sums are K / 32 block sums added in fp32, each an fp32 sum inside the
+MFMAs (16 roundings), and the operand splits add up to 2^-22 sum |w x| (fp16
+hi + lo of the activations and of IQ4_NL's codebook) and the split's absolute
+floor of 2^-39 of the token's largest value.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from ztensor_amd import _lib, storage as st, synth  # noqa: E402
+from ztensor_amd.engine import ROCmEngine  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+G = st.GGMLType
+FORMATS = ["gptq", "awq", "q4_0", "q8_0", "q5_0", "q4_k", "q5_k", "q6_k", "iq4_nl", "iq4_nl_f16",
+           "mmap_q4_0", "mmap_q8_0", "mmap_q5_0", "mmap_q4_k", "mmap_q5_k", "mmap_q6_k"]
+
+
+@pytest.fixture(scope="module")
+def eng():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return ROCmEngine()
+
+
+def weights(fmt, rows, K, seed, orc, group=128):
+    """(storage, the oracle's dequantized matrix in float64)"""
+    n = rows * K
+    if fmt in ("gptq", "awq"):
+        w = synth.w4a16(rows, K, seed, group)
+        z = np.random.default_rng(seed).integers(3, 13, w.zeros.shape).astype(np.float16).view(np.uint16)
+        if fmt == "gptq":
+            s = st.GPTQStorage.from_raw(w.packed, w.scales, z, n, group, 4)
+        else:
+            s = st.AWQStorage(np.ascontiguousarray(w.packed).reshape(-1).view("<u4"), w.scales, z, n, group)
+        d = orc.gptq_dequant(np.ascontiguousarray(w.packed).reshape(-1), w.scales, z, n, group)
+    elif fmt in ("q4_0", "mmap_q4_0"):
+        raw = synth.q4_0(rows, K, seed).raw
+        s, d = st.Q4Storage.from_raw(raw, n), orc.q4_dequant(raw, n)
+        s = s if fmt == "q4_0" else st.MmapStorage(raw, n, G.Q4_0)
+    elif fmt == "q8_0":
+        raw = synth.q8_0(rows, K, seed).raw
+        s, d = st.Q8Storage(raw, n), orc.q8_dequant(raw, n)
+    elif fmt == "mmap_q8_0":
+        raw = synth.gguf_q8_0(rows, K, seed)
+        s, d = st.MmapStorage(raw, n, G.Q8_0), orc.gguf_q8_0_dequant(raw, n)
+    elif fmt.startswith("iq4"):
+        raw = synth.iq4nl(rows, K, seed).raw
+        s, d = st.IQ4NLStorage.from_raw(raw, n), orc.iq4nl_dequant(raw, n)
+    else:
+        name = fmt.replace("mmap_", "")
+        raw = synth.kquant(name, rows, K, seed).raw
+        d = orc.q5_0_dequant(raw, n) if name == "q5_0" else orc.kq_dequant(name, raw, n)
+        kind = {"q5_0": st.Q5_0Storage, "q4_k": st.Q4KStorage, "q5_k": st.Q5KStorage, "q6_k": st.Q6KStorage}[name]
+        g = {"q5_0": G.Q5_0, "q4_k": G.Q4_K, "q5_k": G.Q5_K, "q6_k": G.Q6_K}[name]
+        s = st.MmapStorage(raw, n, g) if fmt.startswith("mmap") else kind.from_raw(raw, n)
+    return s, np.asarray(d, np.float64).reshape(rows, K)
+
+
+def half(fmt):
+    return fmt in ("gptq", "awq", "iq4_nl_f16")
+
+
+def activations(fmt, T, K, seed):
+    x = np.random.default_rng(seed).standard_normal((T, K)).astype(np.float32)
+    return x.astype(np.float16) if half(fmt) else x
+
+
+def check(y, x, w):
+    """y [T, rows] against x [T, K] w [rows, K]^T, by the module's bound."""
+    y, x = np.asarray(y, np.float64), np.asarray(x, np.float64)
+    K = x.shape[1]
+    bound = ((K / 32 + 24) * 2.0**-24 * (np.abs(x) @ np.abs(w).T) +
+             2.0**-38 * np.abs(x).max(axis=1, keepdims=True) * np.abs(w).sum(axis=1))
+    bad = np.abs(y - x @ w.T) > bound
+    assert not bad.any(), (int(bad.sum()), float((np.abs(y - x @ w.T) / np.maximum(bound, 1e-300)).max()))
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("rows,K,T", [(1, 256, 17), (37, 768, 33), (200, 1280, 100), (129, 3328, 65)])
+def test_wide_matmul_both_sides(eng, orc, fmt, rows, K, T):
+    """Tile edges and ragged rows, tokens and K units, in every format and on both operand sides."""
+    s, w = weights(fmt, rows, K, rows + T, orc)
+    x = activations(fmt, T, K, T)
+    xd = torch.from_numpy(x).cuda()
+    y = eng.matmul(xd, st.Tensor((K, rows), s))
+    assert y.shape == (T, rows) and y.is_contiguous()
+    check(y.cpu().numpy(), x, w)
+    z = eng.matmul(st.Tensor((rows, K), s), xd.t().contiguous())
+    assert z.shape == (rows, T)
+    if T > 32:  # on this side the wide path starts past two 16-column chunks
+        assert torch.equal(z.t(), y)
+    else:
+        check(z.t().cpu().numpy(), x, w)
+    # a transposed activation, three dimensions and an unaligned base give the same bits
+    assert torch.equal(eng.matmul(xd.t().contiguous().t(), st.Tensor((K, rows), s)), y)
+    assert torch.equal(eng.matmul(xd.reshape(1, T, K), st.Tensor((K, rows), s)), y.reshape(1, T, rows))
+    off = torch.empty(T * K + 1, dtype=xd.dtype, device="cuda")[1:].view(T, K).copy_(xd)
+    assert torch.equal(eng.matmul(off, st.Tensor((K, rows), s)), y)
+
+
+@pytest.mark.parametrize("fmt", ["gptq", "q4_0", "q4_k", "q6_k"])
+@pytest.mark.parametrize("rows,T", [(2304, 17), (4100, 20), (4100, 40), (4100, 100), (4100, 200), (4100, 300),
+                                    (4100, 520), (9000, 500), (9000, 1030), (20000, 900)])
+def test_wide_every_tile(eng, orc, fmt, rows, T):
+    """Every tile of the dispatch, by rows and tokens; a few tokens are checked."""
+    K = 512
+    s, w = weights(fmt, rows, K, 7, orc)
+    x = activations(fmt, T, K, 8)
+    y = eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, rows), s)).cpu().numpy()
+    pick = np.unique(np.r_[0, 15, 16, T // 2, T - 17, T - 2, T - 1])
+    check(y[pick], x[pick], w)
+
+
+def test_wide_long_k(eng, orc):
+    """The longest rows the packing holds, and a K past them (the other paths)."""
+    for K in (16512, 32768, 33024):
+        s, w = weights("q4_0", 24, K, 3, orc)
+        x = activations("q4_0", 18, K, 4)
+        y = eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, 24), s)).cpu().numpy()
+        if K <= 32768:
+            check(y, x, w)
+        else:
+            assert np.max(np.abs(y - x.astype(np.float64) @ w.T)) <= 1e-5 * np.max(np.abs(x.astype(np.float64) @ w.T))
+
+
+@pytest.mark.parametrize("K,group", [(768, 256), (640, 64)])
+def test_wide_w4a16_groups(eng, orc, K, group):
+    """A group of several 128-K units; a group the wide path does not take."""
+    s, w = weights("gptq", 40, K, 5, orc, group)
+    x = activations("gptq", 35, K, 6)
+    y = eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, 40), s)).cpu().numpy()
+    assert np.max(np.abs(y - x.astype(np.float64) @ w.T)) <= 1e-5 * np.max(np.abs(x.astype(np.float64) @ w.T))
+
+
+def test_wide_w4a16_zeros_of_any_value(eng, orc):
+    """Zeros that are no whole numbers, and large ones, in some groups."""
+    rows, K, T = 70, 1024, 50
+    w = synth.w4a16(rows, K, 11)
+    z = np.full(w.zeros.shape, 8.0, np.float16)
+    z.reshape(-1)[::5] = 7.3
+    z.reshape(-1)[3::11] = -0.125
+    z.reshape(-1)[6::31] = 3000.5
+    zb = z.view(np.uint16)
+    s = st.GPTQStorage.from_raw(w.packed, w.scales, zb, rows * K, 128, 4)
+    d = np.asarray(orc.gptq_dequant(np.ascontiguousarray(w.packed).reshape(-1), w.scales, zb, rows * K, 128), np.float64)
+    x = activations("gptq", T, K, 12)
+    y = eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, rows), s)).cpu().numpy().astype(np.float64)
+    x, d = x.astype(np.float64), d.reshape(rows, K)
+    # the whole part and the rest of a zero are summed apart: (|q| + |zero|) |s x| instead of |w x|
+    sc = w.scales.view(np.float16).astype(np.float64).repeat(128).reshape(rows, K)
+    mag = np.abs(x) @ (np.abs(d) + 15 * sc + np.abs(z.astype(np.float64)).repeat(128).reshape(rows, K) * sc).T
+    assert np.all(np.abs(y - x @ d.T) <= (K / 32 + 24) * 2.0**-24 * mag)
+
+
+def test_wide_token_scales_and_special_values(eng, orc):
+    """Tokens far apart in scale, all-zero tokens, and infinities and NaN, which stay in their tokens."""
+    rows, K, T = 48, 512, 40
+    s, w = weights("q8_0", rows, K, 21, orc)
+    x = activations("q8_0", T, K, 22)
+    x *= (10.0 ** np.linspace(-30, 30, T)).astype(np.float32)[:, None]
+    x[7] = 0.0
+    x[9, 5] = np.inf
+    x[11, 3] = np.nan
+    x[13] = np.float32(1e-42)  # subnormal
+    y = eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, rows), s)).cpu().numpy()
+    fine = [t for t in range(T) if t not in (9, 11, 13)]
+    check(y[fine], x[fine], w)
+    assert np.all(y[7] == 0.0) and np.all(np.isnan(y[11]))
+    with np.errstate(invalid="ignore"):
+        ref = x[9].astype(np.float64) @ w.T
+    assert np.array_equal(np.isnan(y[9]), np.isnan(ref)) and np.array_equal(y[9][np.isinf(ref)], ref[np.isinf(ref)])
+    assert np.allclose(y[13], x[13].astype(np.float64) @ w.T, rtol=1e-5, atol=3e-45)
+
+
+def test_wide_in_a_captured_graph(eng, orc):
+    """A captured call replays as the eager one, also after wider eager calls of the same engine."""
+    stream = torch.cuda.Stream()
+    eng = ROCmEngine(stream=stream)
+    s, _ = weights("q4_k", 300, 1024, 31, orc)
+    big, _ = weights("q8_0", 500, 2048, 32, orc)
+    t = st.Tensor((1024, 300), s)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):  # all work in the engine's stream order
+        x = torch.from_numpy(activations("q4_k", 24, 1024, 33)).cuda()
+        eng.matmul(x, t)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            y = eng.matmul(x, t)
+        for i in range(3):
+            x.copy_(torch.from_numpy(activations("q4_k", 24, 1024, 40 + i)))
+            want = eng.matmul(x, t).clone()
+            eng.matmul(torch.randn(700, 2048, device="cuda"), st.Tensor((2048, 500), big))
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)
+
+
+def test_wide_arguments(eng):
+    lib, need = eng.lib, eng.lib.zt_gemm_wide_workspace_bytes
+    assert need(1, 0, 64, 256, 20) > 0
+    for bad in [(-1, 0, 64, 256, 20), (9, 0, 64, 256, 20), (1, 1, 64, 256, 20), (0, 0, 64, 256, 20), (1, 0, 64, 160, 20),
+                (5, 0, 64, 384, 20), (1, 0, 64, 32896, 20), (2, 0, 1 << 16, 32768, 20), (1, 0, 0, 256, 20)]:
+        assert need(*bad) == -1, bad
+    b = torch.zeros(1 << 20, dtype=torch.uint8, device="cuda")
+    p, s = b.data_ptr(), torch.cuda.current_stream().cuda_stream
+    ws = need(1, 0, 64, 256, 20)
+
+    def call(w=p, o1=1024, x=p, c=p + (1 << 19), k=256, t=20, wsp=p + (1 << 18), wsb=ws, rows=64):
+        return lib.zt_gemm_wide_f32(1, w, o1, 0, 0, 0, x, 0, c, rows, k, t, wsp, wsb, s)
+
+    assert call() == 0 and call(rows=0) == 0 and call(t=0) == 0
+    for bad in (dict(w=0), dict(x=0), dict(c=0), dict(wsp=0), dict(wsb=ws - 1), dict(w=p + 8), dict(x=p + 4),
+                dict(o1=1032), dict(o1=-16), dict(c=p + 2), dict(wsp=p + 8), dict(k=-128), dict(t=-1), dict(k=96)):
+        assert call(**bad) == _lib.HIP_ERROR_INVALID_VALUE, bad
+    torch.cuda.synchronize()

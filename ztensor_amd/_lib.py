@@ -126,6 +126,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "zt_dequant_awq4_f32": (I, [P, L, P, L, I, I, P]),
     "zt_dequant_fp8_f32": (I, [P, L, P, L, I, P]),
     "zt_dequant_iq3s_f32": (I, [P, L, P, L, P]),
+    "zt_gemm_wide_workspace_bytes": (L, [I, I, I, I, I]),
+    "zt_gemm_wide_f32": (I, [I, P, L, L, P, I, P, I, P, I, I, I, P, L, P]),
     "zt_gemm_int8_f32": (I, [P, P, P, I, I, I, P]),
     "zt_gemm_int4_f32": (I, [P, P, P, P, P, I, I, I, I, P]),
     "zt_gemm_int4_f32_rmul": (I, [P, P, P, P, P, I, I, I, I, P]),

@@ -257,16 +257,77 @@ class ROCmEngine:
             x = b
             if x.shape[0] != k:
                 raise ValueError(f"matmul: A is [{rows},{k}] but B has {x.shape[0]} rows")
+            if x.dim() == 2 and _wide_tokens(x.shape[1], transposed=True):
+                ct = self._wide_times(a.storage, rows, k, x.t())
+                if ct is not None:
+                    return ct.t().contiguous()
             return self._weight_times(a.storage, rows, k, x.contiguous())
         if isinstance(b, Tensor):
             k, nout = b.shape[-2], b.shape[-1]
             if a.shape[-1] != k:
                 raise ValueError(f"matmul: A has {a.shape[-1]} columns but B is [{k},{nout}]")
             m = a.numel() // k
+            if _wide_tokens(m):
+                ct = self._wide_times(b.storage, nout, k, a.reshape(m, k))
+                if ct is not None:
+                    return ct.reshape(*a.shape[:-1], nout)
             xt = a.reshape(m, k).t().contiguous()  # [K, M]
             ct = self._weight_times(b.storage, nout, k, xt)  # [Nout, M]
             return ct.t().contiguous().reshape(*a.shape[:-1], nout)
         raise TypeError("matmul: neither operand is a quantized weight Tensor")
+
+    def _wide_times(self, s: Any, rows: int, k: int, x: torch.Tensor) -> torch.Tensor | None:
+        """x[T, k] @ dequant(W)[rows, k]^T -> fp32 [T, rows] on the wide-batch
+        GEMM, which reads the layout batch 1 reads and the activations as they
+        are: no tiled copy, no 16-column chunks, no transposes.  None for a
+        storage, type or size it does not take (the caller goes on to the
+        other paths).  The packed activations live in a temporary of this
+        call, which a captured graph keeps in its own pool."""
+        if x.device != self.device:
+            raise ValueError("activations must be on the engine's device")
+        mm = s.qtype if isinstance(s, MmapStorage) else None
+        half = x.dtype == torch.float16
+        if isinstance(s, (GPTQStorage, AWQStorage)):
+            fmt = _WIDE["w4a16"]
+            if s.group_size % 128 != 0 or k % s.group_size != 0:
+                return None
+        elif isinstance(s, Q4Storage) or mm == GGMLType.Q4_0:
+            fmt = _WIDE["q4_0"]
+            if half and mm is None:
+                x, half = x.float(), False  # widens exactly, as for the other Q4_0 batches
+        elif isinstance(s, IQ4NLStorage):
+            fmt = _WIDE["iq4_nl"]
+        elif mm is not None:
+            fmt = _WIDE_MMAP.get(mm, -1)
+        else:
+            fmt = _WIDE_STORAGE.get(type(s), -1)
+        if x.dtype not in (torch.float32, torch.float16):
+            return None
+        t = x.shape[0]
+        nbytes = self.lib.zt_gemm_wide_workspace_bytes(fmt, int(half), rows, k, t)
+        if nbytes < 0:
+            return None
+        self.upload_weights([s])
+        buf = s.gpu_ptr()
+        w, o1, o2, szr, group = buf.tensor, buf.data_offset, 0, 0, 0
+        if fmt == _WIDE["w4a16"]:
+            if s._gpu_szr is None:
+                return None
+            szr, group = _p(s._gpu_szr), s.group_size
+        elif fmt == _WIDE["q5_0"]:
+            o1, o2 = ((s._gpu_offsets["qh_offset"], s._gpu_offsets["qs_offset"]) if mm is not None
+                      else (s.gpu_qh_offset(), s.gpu_qs_offset()))
+        elif fmt == _WIDE["q6_k"]:
+            w = self._q6k_split_copy(s, _p(buf.tensor), rows, k)
+            if w is None:
+                return None
+        x = x.contiguous()
+        x = x if _p(x) % 16 == 0 else x.clone()
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        c = torch.empty((t, rows), dtype=torch.float32, device=self.device)
+        self.lib.call("zt_gemm_wide_f32", fmt, _p(w), o1, o2, szr, group, _p(x), int(half), _p(c), rows, k, t, _p(ws),
+                      nbytes, self._s)
+        return c
 
     def _w4a16_tiled(self, s: Any, rows: int, k: int) -> tuple[torch.Tensor, torch.Tensor]:
         """The tiled copy of uploaded W4A16 weights for batches of 4-16
@@ -379,21 +440,29 @@ class ROCmEngine:
         32-bit offsets or x's alignment do not allow it, when the engine was
         made with q6k_split=False, and when building the copy would leave less
         than split_reserve_bytes of device memory free."""
+        sp = self._q6k_split_copy(s, raw_ptr, rows, k) if _p(x) % 16 == 0 else None
+        if sp is None:
+            self.lib.call("zt_gemv_q6k_f32", raw_ptr, _p(x), _p(c), rows, k, self._s)
+            return
+        self.lib.call("zt_gemv_q6ks_f32", _p(sp), _p(x), _p(c), rows, k, self._s)
+
+    def _q6k_split_copy(self, s: Any, raw_ptr: int, rows: int, k: int) -> torch.Tensor | None:
+        """The split copy of uploaded Q6_K super-blocks, built on first use,
+        or None where it may not be built."""
         key = ("q6ks", rows, k, raw_ptr)
         cached = getattr(s, "_gpu_split", None)
         if cached is not None and cached[0] != key:
             s._gpu_split = cached = None  # type: ignore[attr-defined]  # a stale copy goes before a new one
         nbytes = self.lib.zt_q6k_split_bytes(rows, k)
-        if (rows * (k // 256) * 210 >= 1 << 31 or _p(x) % 16 != 0 or not self.q6k_split
+        if (rows * (k // 256) * 210 >= 1 << 31 or not self.q6k_split
                 or (cached is None and torch.cuda.mem_get_info(self.device)[0] < nbytes + self.split_reserve_bytes)):
-            self.lib.call("zt_gemv_q6k_f32", raw_ptr, _p(x), _p(c), rows, k, self._s)
-            return
+            return None
         if cached is None:
             sp = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
             self.lib.call("zt_q6k_split", raw_ptr, rows, k, _p(sp), self._s)
             cached = (key, sp)
             s._gpu_split = cached  # type: ignore[attr-defined]
-        self.lib.call("zt_gemv_q6ks_f32", _p(cached[1]), _p(x), _p(c), rows, k, self._s)
+        return cached[1]
 
     def _q5_0_tiled(self, s: Any, buf: GPUBuffer, rows: int, k: int, qh: int, qs: int) -> tuple:
         """The tiled copy of uploaded Q5_0 weights (nibbles and scales in the
@@ -817,6 +886,21 @@ def _block_wide(fmt: str, rows: int, k: int, n: int) -> bool:
         return n >= 128
     return n >= 128 or (n >= 32 and rows >= 8192) or (n >= 64 and k > 8192)
 
+
+def _wide_tokens(t: int, transposed: bool = False) -> bool:
+    """Whether a batch of t tokens goes to the wide-batch GEMM: past the 16
+    columns of the tiled and row-block GEMMs, which take wider batches in
+    chunks of 16 (32 tokens of 14336 x 4096 (rows x K): Q4_0 26 us against
+    2 x 13 us and the copies of the chunks, GPTQ 18 against 2 x 13); past two
+    chunks where the activations and the result are also to be transposed
+    (a weight on the A side)."""
+    return t > (32 if transposed else 16)
+
+
+# zt_gemm_wide_f32 formats (ZT_WIDE_*)
+_WIDE = {"w4a16": 0, "q4_0": 1, "q8_0": 2, "q8_gguf": 3, "q5_0": 4, "q4_k": 5, "q5_k": 6, "q6_k": 7, "iq4_nl": 8}
+_WIDE_STORAGE = {Q8Storage: 2, Q5_0Storage: 4, Q4KStorage: 5, Q5KStorage: 6, Q6KStorage: 7}
+_WIDE_MMAP = {GGMLType.Q8_0: 3, GGMLType.Q5_0: 4, GGMLType.Q4_K: 5, GGMLType.Q5_K: 6, GGMLType.Q6_K: 7}
 
 _TILED_BATCHES = (4, 8, 12, 16)  # batch sizes on the tiled layouts (W4A16, IQ4_NL, Q4_0, Q8_0, Q4_K, Q5_K, Q5_0)
 
