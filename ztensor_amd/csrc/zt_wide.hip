@@ -39,6 +39,9 @@ enum Order { kUnit, kHalves, kOctets };
 constexpr Order order_of(Fmt f) { return f == W4A16 ? kUnit : f == IQ4_NL ? kOctets : kHalves; }
 constexpr bool has_mins(Fmt f) { return f == Q4_K || f == Q5_K; }
 
+// Load instructions of one row tile and 128-K unit (Weights::load).
+constexpr int loads_of(Fmt f) { return f == Q6_K ? 5 : f == Q5_K ? 4 : f == Q5_0 || f == Q8_0 || f == Q8_GGUF ? 3 : 2; }
+
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 
 // x = p[0] + p[1] + p[2] in bf16 bits (the last two truncations are exact).
@@ -215,8 +218,10 @@ struct WideArgs {
 
 // One wave's direct global -> LDS copy of 1 KB: lane l's 16 bytes at
 // base + off go to lds + 16 l.  The caller waits for vmcnt before a barrier.
+// (s_nop: 5 wait states between a vector write of the base's registers, which
+// the compiler may have put right before, and the load's read of them.)
 __device__ __forceinline__ void dma_1k(const void* base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
                  : "memory");
 }
 
@@ -277,6 +282,7 @@ struct Weights {
         }
     }
     __device__ __forceinline__ void load(Raw& r, const Off& o, int u, int gu) const {
+        u = __builtin_amdgcn_readfirstlane(u);  // a scalar offset, or the loads loop over the lanes
         const int sb = u >> 1, h = u & 1;
         if constexpr (F == W4A16) {
             r.a = __builtin_amdgcn_raw_buffer_load_b128(rw, o.w, 64 * u, 0);
@@ -548,8 +554,13 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideAr
         for (int h = 0; h < H; h++) {
             const int buf = (t * H + h) & 1;
             // this stage's activations have landed, and the weights; the other buffer's readers are done
-            __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            // (a unit's later stages leave the next unit's weight loads, issued after their own, in flight)
+            if (h > 0 && u + WK < nu) {
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NT * loads_of(F)) : "memory");
+            } else {
+                __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
             if (h + 1 < H) {
                 if (u < nu) stage(u, h + 1, buf ^ 1);
             } else if (u + WK < nu) {
@@ -754,33 +765,42 @@ hipError_t launch_tile(const WideArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// The tile.  A workgroup's time hardly depends on its tile while the main
-// loop waits for memory, so the smallest tile whose workgroups still fit the
-// 256 CUs at once wins (4096 rows, K = 4096, us for 32 x 16 / 32 x 32 /
-// 32 x 64 / 64 x 64 / 64 x 128 tokens x rows: W4A16 32 tokens 9.9 / 12.4 /
-// 17 / 22 / 31, 64 tokens 16.7 / 13.1 / 18 / 22 / 31, 512 tokens - / - / 51 /
-// 44 / 37; Q4_0 32 tokens 15.6 / 18.8 / 25 / 37 / -, 512 tokens - / - / 74 /
-// 75 / 62).  Past one round the tile that decodes a weight for most MFMAs
-// wins: 128 x 128 for one activation part and for Q6_K's longer decode, 64 x
-// 128 in workgroups of 4 waves, two or more a CU, for two parts (14336 x 4096
-// rows x K at 1024 tokens: W4A16 128 x 128 171, 64 x 128 176; Q4_0 341 / 272;
-// Q6_K 408 / 408; Q4_K 385 / 314).
+// The tile.  While one round of workgroups covers the matrix, its time is
+// the chain of loads and barriers along K, so the smallest tile whose
+// workgroups still fit the 256 CUs wins, with as many waves along K as the
+// registers and LDS allow (16 waves against 8 in 64 x 128 tiles, K = 4096 /
+// 14336, 512 tokens of 4096 rows: Q4_0 54 / 159 us against 61 / 179, Q4_K
+// 64 / 183 against 78 / 234, W4A16 35 / 91 against 37 / 106; Q6_K's decode
+// would spill there and stays at 8 waves).  Past one round the tile that
+// feeds most MFMAs a decoded weight and stage wins, as long as its last round
+// is full enough: 128 x 256 in 8 waves (14336 x 4096 rows x K, us against 64
+// x 128 in 4 waves: 512 tokens W4A16 76 / 104, Q4_0 147 / 152, Q6_K 183 /
+// 239; 1024 tokens 144 / 179, 235 / 274, 356 / 415).
 template <Fmt F, int P>
 hipError_t launch_gemm(const WideArgs& a, hipStream_t st) {
-    auto fits = [&](int tokens, int rows, long most) { return (long)ceil_div(a.T, tokens) * ceil_div(a.rows, rows) <= most; };
-    if (a.T <= 16 && fits(16, 32, 256)) return launch_tile<F, P, 1, 2, 1, 8>(a, st);
-    if (fits(32, 16, 256)) return launch_tile<F, P, 2, 1, 1, 8>(a, st);
-    if (fits(32, 32, 256)) return launch_tile<F, P, 2, 2, 1, 8>(a, st);
-    if (fits(32, 64, 256)) return launch_tile<F, P, 2, 2, 2, 4>(a, st);
-    if (fits(64, 64, 256)) return launch_tile<F, P, 4, 2, 2, 4>(a, st);
-    if constexpr (P == 1 || F == Q6_K) {
-        if (fits(64, 128, 256)) return launch_tile<F, P, 4, 2, 4, 2>(a, st);
-        if (!fits(128, 128, 256) && fits(128, 128, 512)) return launch_tile<F, P, 8, 2, 4, 1>(a, st);
-        return launch_tile<F, P, 8, 2, 4, 2>(a, st);
-    } else {
-        if (fits(64, 128, 512)) return launch_tile<F, P, 4, 2, 4, 2>(a, st);
-        return launch_tile<F, P, 4, 2, 4, 1>(a, st);
+    auto tiles = [&](int tokens, int rows) { return (long)ceil_div(a.T, tokens) * ceil_div(a.rows, rows); };
+    auto fits = [&](int tokens, int rows) { return tiles(tokens, rows) <= 256; };
+    // whether rounds of 256 workgroups are at least this full on average
+    auto full = [&](int tokens, int rows, double share) {
+        const long t = tiles(tokens, rows);
+        return (double)t >= share * 256.0 * (double)((t + 255) / 256);
+    };
+    constexpr bool KQ = has_mins(F);
+    if (a.T <= 16 && fits(16, 32)) return launch_tile<F, P, 1, 2, 1, 8>(a, st);
+    if (fits(32, 16)) return launch_tile<F, P, 2, 1, 1, 8>(a, st);
+    if (fits(32, 32)) return launch_tile<F, P, 2, 2, 1, 8>(a, st);
+    if (fits(32, 64)) return launch_tile<F, P, 2, 2, 2, 8>(a, st);
+    if (fits(64, 64)) return launch_tile<F, P, 4, 2, 2, 4>(a, st);
+    if (fits(64, 128)) return launch_tile<F, P, 4, 2, 4, F == Q6_K ? 2 : 4>(a, st);
+    // (two parts without minima: 64 x 256 tiles, two workgroups a CU, hold their rate below 128 x 256)
+    if constexpr (P == 1 || KQ || F == Q6_K) {
+        if (fits(128, 128)) return launch_tile<F, P, 8, 2, 4, 2>(a, st);
     }
+    if (full(128, 256, P == 1 || F == Q6_K ? 0.65 : 0.85)) return launch_tile<F, P, 8, 2, 8, 1>(a, st);
+    if constexpr (!(P == 1 || KQ || F == Q6_K)) {
+        if (full(64, 256, 0.8)) return launch_tile<F, P, 4, 2, 8, 1>(a, st);
+    }
+    return launch_tile<F, P, 4, 2, 4, 1>(a, st);
 }
 
 // Bytes of the packed activations of T tokens (whole 128-token tiles: the
