@@ -118,3 +118,49 @@ def test_invalid_arguments(eng):
     assert lib.zt_dequant_w4_f16(0, 0, 0, 0, 64, 48, None) == 1  # group % 32
     assert lib.zt_dequant_w4_f16(0x1008, 0x2000, 0, 0x3000, 64, 32, None) == 1  # W_packed alignment
     assert lib.zt_dequant_q4_f16(0x1001, 0x3000, 32, 16, None) == 1  # odd base
+
+
+@pytest.mark.parametrize("n,g,off", [(96, 96, 0), (32, 32, 1), (8192 + 128, 128, 3), (288 * 37, 288, 1), (1 << 16, 1 << 15, 0)])
+@pytest.mark.parametrize("half", [True, False])
+def test_w4_pieces_groups_and_unaligned_outputs(eng, orc, n, g, off, half):
+    """Groups that are and are not a power of two, partial last workgroups,
+    and outputs aligned to their element only: bit for bit."""
+    rng = np.random.default_rng(n)
+    packed = rng.integers(0, 256, n // 2, dtype=np.uint8)
+    scales = synth.f16_bits(rng.standard_normal(n // g).astype(np.float32) * 0.1)
+    zeros = synth.f16_bits(rng.random(n // g).astype(np.float32) * 15)
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x).view(np.uint8)).cuda()  # noqa: E731
+    pd, sd, zd = dev(packed), dev(scales), dev(zeros)
+    buf = torch.full((n + 2 * off + 8,), 7.0, dtype=torch.float16 if half else torch.float32, device="cuda")
+    out = buf[off:off + n]
+    lib = _lib.load()
+    lib.call("zt_dequant_w4_f16" if half else "zt_dequant_w4_f32", pd.data_ptr(), sd.data_ptr(), zd.data_ptr(),
+             out.data_ptr(), n, g, torch.cuda.current_stream().cuda_stream)
+    ref = np.asarray(orc.gptq_dequant(packed, scales, zeros, n, g, 4), np.float32)
+    if half:
+        assert np.array_equal(out.cpu().numpy().view(np.uint16), f16_bits_of(ref))
+    else:
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+    assert torch.all(buf[:off] == 7.0) and torch.all(buf[off + n:] == 7.0)
+
+
+@pytest.mark.parametrize("n,off", [(1, 0), (31, 1), (32 * 300 + 13, 3), (1 << 15, 0)])
+@pytest.mark.parametrize("half", [True, False])
+def test_q4_0_pieces_partial_blocks_and_unaligned_outputs(eng, orc, n, off, half):
+    """Lengths that end inside a piece or a block, outputs aligned to their element only: bit for bit."""
+    nblk = -(-n // 32)
+    raw = synth.q4_0(nblk, 32, n).raw
+    lib = _lib.load()
+    host = np.empty(lib.zt_q4_gpu_bytes(nblk), np.uint8)
+    lib.zt_q4_raw_to_gpu(raw.ctypes.data, nblk, host.ctypes.data)
+    a = torch.from_numpy(host).cuda()
+    buf = torch.full((n + 2 * off + 8,), 7.0, dtype=torch.float16 if half else torch.float32, device="cuda")
+    out = buf[off:off + n]
+    lib.call("zt_dequant_q4_f16" if half else "zt_dequant_q4_f32", a.data_ptr(), out.data_ptr(), n,
+             lib.zt_q4_gpu_data_offset(nblk), torch.cuda.current_stream().cuda_stream)
+    ref = np.asarray(orc.q4_dequant(raw, n), np.float32)
+    if half:
+        assert np.array_equal(out.cpu().numpy().view(np.uint16), f16_bits_of(ref))
+    else:
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+    assert torch.all(buf[:off] == 7.0) and torch.all(buf[off + n:] == 7.0)

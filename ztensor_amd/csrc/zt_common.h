@@ -48,6 +48,18 @@ __device__ __forceinline__ float out_cvt<float>(float v) { return v; }
 template <>
 __device__ __forceinline__ uint16_t out_cvt<uint16_t>(float v) { return __half_as_ushort(__float2half_rn(v)); }
 
+// One 16-byte store of 4 fp32 or 8 fp16 values; out has the alignment of its type only.
+__device__ __forceinline__ void store16(float* out, const float (&v)[4]) {
+    const u32x4 w = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+    __builtin_memcpy(out, &w, 16);
+}
+__device__ __forceinline__ void store16(uint16_t* out, const uint16_t (&v)[8]) {
+    u32x4 w;
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = (uint32_t)v[2 * i] | (uint32_t)v[2 * i + 1] << 16;
+    __builtin_memcpy(out, &w, 16);
+}
+
 // 128-bit streaming load of weight data that is read exactly once: the
 // nontemporal hint keeps it from evicting the reused activations.
 __device__ __forceinline__ uint4 ld_stream(const uint4* p) {
