@@ -275,3 +275,33 @@ def test_engine_on_a_side_stream_runs_torch_work_on_that_stream(orc):
     assert rel_err(c_t.cpu().numpy().T.reshape(-1), ref8.reshape(-1)) <= TOL
     assert rel_err(ys[0].cpu().numpy(), ref4.reshape(8, rows)[0]) <= TOL
     torch.cuda.synchronize()
+
+
+def test_engine_stream_is_current_or_switched_to(orc):
+    """A call from the engine's own stream and one from another give the same
+    bits, and the caller's current stream is what it was; a weight whose
+    upload was dropped is uploaded again."""
+    rows, K = 48, 512
+    w = synth.q4_0(rows, K, 71)
+    s = Q4Storage.from_raw(w.raw, rows * K)
+    side = torch.cuda.Stream()
+    eng = ROCmEngine(stream=side)
+    x = torch.from_numpy(synth.x_f32(K, 71).reshape(1, K)).cuda()
+    torch.cuda.synchronize()
+    before = torch.cuda.current_stream()
+    assert not eng._is_current()
+    y = eng.matmul(x, Tensor((K, rows), s))
+    assert torch.cuda.current_stream() == before and y.shape == (1, rows)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        assert eng._is_current()
+        z = eng.matmul(x, Tensor((K, rows), s))
+        assert torch.cuda.current_stream() == side
+    side.synchronize()
+    s.set_gpu_ptr(None)
+    v = eng.matmul(x.reshape(1, 1, K), Tensor((K, rows), s))
+    torch.cuda.synchronize()
+    assert v.shape == (1, 1, rows)
+    assert torch.equal(y, z) and torch.equal(y, v.reshape(1, rows))
+    ref = np.asarray(orc.gemm_f32_q4_nt(synth.x_f32(K, 71), w.raw, 1, rows, K)).reshape(1, rows)
+    assert np.max(np.abs(y.cpu().numpy() - ref)) <= 1e-5 * np.max(np.abs(ref))

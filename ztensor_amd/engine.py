@@ -61,9 +61,13 @@ def _on_engine_stream(fn):
     one of them to other work while a kernel on the engine stream still uses
     it.  Inputs made on another stream must be ready before the call, and
     outputs used on another stream must wait for the engine stream, as with
-    any stream-ordered library."""
+    any stream-ordered library.  Where the caller's current stream is the
+    engine's own already, there is nothing to switch (a call on 1024 x 4096
+    Q4_0 weights spent 6 of its 24 us on the two switches)."""
 
     def wrapped(self, *args, **kwargs):
+        if self._is_current():
+            return fn(self, *args, **kwargs)
         with torch.cuda.stream(self.stream):
             return fn(self, *args, **kwargs)
 
@@ -99,6 +103,12 @@ class ROCmEngine:
     @property
     def _s(self) -> int:
         return self.stream.cuda_stream
+
+    def _is_current(self) -> bool:
+        """Whether the engine's stream is torch's current stream, on its own device."""
+        d = self.device.index
+        return (torch.cuda.current_device() == d and self.stream.device_index == d
+                and torch._C._cuda_getCurrentRawStream(d) == self.stream.cuda_stream)
 
     def _workspace(self, nbytes: int) -> tuple[int, int]:
         """Scratch for the split-K partials of the tiled GEMMs: one buffer per
@@ -271,6 +281,8 @@ class ROCmEngine:
                 ct = self._wide_times(b.storage, nout, k, a.reshape(m, k))
                 if ct is not None:
                     return ct.reshape(*a.shape[:-1], nout)
+            if m == 1:  # a vector is its own transpose
+                return self._weight_times(b.storage, nout, k, a.reshape(k, 1)).reshape(*a.shape[:-1], nout)
             xt = a.reshape(m, k).t().contiguous()  # [K, M]
             ct = self._weight_times(b.storage, nout, k, xt)  # [Nout, M]
             return ct.t().contiguous().reshape(*a.shape[:-1], nout)
@@ -307,7 +319,8 @@ class ROCmEngine:
         nbytes = self.lib.zt_gemm_wide_workspace_bytes(fmt, int(half), rows, k, t)
         if nbytes < 0:
             return None
-        self.upload_weights([s])
+        if s.gpu_ptr() is None:
+            self.upload_weights([s])
         buf = s.gpu_ptr()
         w, o1, o2, szr, group = buf.tensor, buf.data_offset, 0, 0, 0
         if fmt == _WIDE["w4a16"]:
@@ -506,7 +519,8 @@ class ROCmEngine:
                 xp[:, :m] = xs[:, j0:j0 + m]
                 outs.append(self._weight_times(s, rows, k, xp)[:, :m])
             return torch.cat(outs, dim=1)
-        self.upload_weights([s])
+        if getattr(s, "_gpu", None) is None:
+            self.upload_weights([s])
         c = torch.empty((rows, n), dtype=torch.float32, device=self.device)
         buf = s.gpu_ptr() if hasattr(s, "gpu_ptr") else None  # ternary: resident per shape, below
         if isinstance(s, MmapStorage):
