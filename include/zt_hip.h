@@ -590,8 +590,9 @@ void zt_q5_0_raw_to_gpu(const void* raw, long nblk, void* out);
  * The others take fp32 X.  Weights enter as exact fp16 integers (IQ4_NL's
  * codebook and Q6_K's scaled values as fp16 hi + lo), fp32 activations as
  * fp16 hi + lo after a power-of-two scale per token, sums are fp32; every
- * output is written once and repeats bit for bit.  K % 128 == 0 (K-quants:
- * 256), K <= 32768, bulk data below 2^31 bytes; W, X, the offsets and the
+ * output is written once and repeats bit for bit.  Up to 16 tokens of fp16 X
+ * are multiplied as they are, in one launch; the others are packed first.  K
+ * % 128 == 0 (K-quants: 256), K <= 32768, bulk data below 2^31 bytes; W, X, the offsets and the
  * workspace 16-byte aligned.  The workspace holds the packed activations
  * (zt_gemm_wide_workspace_bytes, -1 for a size or type the path does not
  * take); other calls -> InvalidValue. */

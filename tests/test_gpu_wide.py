@@ -118,6 +118,28 @@ def test_wide_every_tile(eng, orc, fmt, rows, T):
     check(y[pick], x[pick], w)
 
 
+@pytest.mark.parametrize("fmt", ["gptq", "iq4_nl_f16", "q4_0", "q5_k", "q6_k"])
+@pytest.mark.parametrize("rows,K,T", [(1, 256, 2), (33, 768, 5), (100, 1280, 16), (4096, 512, 3), (4100, 2304, 16),
+                                      (8200, 1024, 13), (24600, 512, 7), (50, 8448, 8)])
+def test_few_tokens(eng, orc, fmt, rows, K, T):
+    """2 to 16 tokens: one to all of a tile's tokens, K of whole and partial 512-value quads, every workgroup shape."""
+    s, w = weights(fmt, rows, K, rows + T, orc)
+    x = activations(fmt, T, K, T)
+    y = eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, rows), s))
+    check(y.cpu().numpy(), x, w)
+    assert torch.equal(eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, rows), s)), y)
+
+
+def test_few_tokens_special_values(eng, orc):
+    """Infinities and NaN stay in their tokens."""
+    s, w = weights("gptq", 40, 640, 3, orc)
+    x = activations("gptq", 6, 640, 4)
+    x[1, 7], x[3, 600] = np.inf, np.nan
+    y = eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((640, 40), s)).cpu().numpy()
+    check(y[[0, 2, 4, 5]], x[[0, 2, 4, 5]], w)
+    assert np.all(np.isnan(y[3])) and not np.any(np.isfinite(y[1]))
+
+
 def test_wide_long_k(eng, orc):
     """The longest rows the packing holds, and a K past them (the other paths)."""
     for K in (16512, 32768, 33024):
@@ -131,17 +153,19 @@ def test_wide_long_k(eng, orc):
 
 
 @pytest.mark.parametrize("K,group", [(768, 256), (640, 64)])
-def test_wide_w4a16_groups(eng, orc, K, group):
+@pytest.mark.parametrize("T", [6, 35])
+def test_wide_w4a16_groups(eng, orc, K, group, T):
     """A group of several 128-K units; a group the wide path does not take."""
     s, w = weights("gptq", 40, K, 5, orc, group)
-    x = activations("gptq", 35, K, 6)
+    x = activations("gptq", T, K, 6)
     y = eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, 40), s)).cpu().numpy()
     assert np.max(np.abs(y - x.astype(np.float64) @ w.T)) <= 1e-5 * np.max(np.abs(x.astype(np.float64) @ w.T))
 
 
-def test_wide_w4a16_zeros_of_any_value(eng, orc):
+@pytest.mark.parametrize("T", [11, 50])
+def test_wide_w4a16_zeros_of_any_value(eng, orc, T):
     """Zeros that are no whole numbers, and large ones, in some groups."""
-    rows, K, T = 70, 1024, 50
+    rows, K = 70, 1024
     w = synth.w4a16(rows, K, 11)
     z = np.full(w.zeros.shape, 8.0, np.float16)
     z.reshape(-1)[::5] = 7.3

@@ -751,6 +751,217 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideAr
         }
 }
 
+// ------------------------------------------------------------ few tokens
+//
+// Up to 16 tokens of fp16 activations on 4-bit weights of 16 bytes a block,
+// one launch on the upload layout.  Bound by memory: a wave needs many bytes
+// in flight, in long runs (operands read straight from the rows, 16 rows of 64
+// bytes an instruction, took 12.8 us where this takes 8.7 us, W4A16 1024 x
+// 8192 rows x K, 16 tokens).  The waves of a workgroup lie along K and work
+// alone up to the final sum.  A wave takes 512 values of K, a quad of units,
+// at a time: a load instruction reads 256 bytes of each of 4 rows (or tokens),
+// and a private LDS region turns rows into operands: lane l writes piece
+// l % 16 of row 4 v + l / 16 at position piece ^ row, and lane 16 g + i reads
+// piece 4 u + g of row i, both without bank conflicts.  A quad's registers are
+// free once it is written to LDS, so the next quad's loads are in flight
+// while this one is multiplied.
+template <Fmt F, int NT, int WK>
+__global__ void __launch_bounds__(64 * WK, 2) few_gemm_kernel(const WideArgs p) {
+    static_assert(F == W4A16 || F == IQ4_NL, "16-byte blocks, fp16 activations");
+    constexpr int PW = parts_of(F), SD = F == W4A16 ? 1 : 2;  // 16-byte scale loads of a row and quad
+    constexpr int RB = 4096 * (1 + NT);                       // LDS of a wave: one activation unit, NT weight quads
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const int n0 = blockIdx.x * 16 * NT, nu = p.K / 128, nq = (nu + 3) / 4;
+    const __amdgpu_buffer_rsrc_t rw = Weights<F>::rsrc(p.w, p.wb), rs = Weights<F>::rsrc(p.s, p.sb),
+                                 rx = Weights<F>::rsrc(p.xp, (uint32_t)p.T * (uint32_t)p.K * 2u);
+    uint32_t wo[NT][4], so[NT], xo[4];
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            wo[j][v] = (uint32_t)min(n0 + 16 * j + 4 * v + lg, p.rows - 1) * (uint32_t)(p.K / 2) + 16u * li;
+        so[j] = (uint32_t)min(n0 + 16 * j + li, p.rows - 1) * (uint32_t)(F == W4A16 ? p.K / 128 / p.gu * 4 : p.K / 16);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) xo[v] = (uint32_t)min(4 * v + lg, p.T - 1) * (uint32_t)p.K * 2u + 16u * li;
+    char* xs = smem + kg * RB;
+    char* ws = xs + 4096;
+    uint32_t put[4], get[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        put[v] = (4 * v + lg) * 256 + ((li ^ (4 * v + lg)) * 16);
+        get[v] = li * 256 + (((4 * v + lg) ^ li) * 16);
+    }
+    u32x4 w[NT][4], x[4][4], sn[NT][SD];
+    // past the last unit the loads read other rows or zeros, and nothing uses them
+    auto load_w = [&](int q) {
+        q = __builtin_amdgcn_readfirstlane(q);
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) w[j][v] = __builtin_amdgcn_raw_buffer_load_b128(rw, wo[j][v], 256 * q, 2);  // nontemporal
+            if (F == W4A16 && p.gu > 1) {
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    sn[j][0][v] = __builtin_amdgcn_raw_buffer_load_b32(rs, so[j], 4 * ((4 * q + v) / p.gu), 0);
+            } else {
+#pragma unroll
+                for (int d = 0; d < SD; d++) sn[j][d] = __builtin_amdgcn_raw_buffer_load_b128(rs, so[j], 16 * (SD * q + d), 0);
+            }
+        }
+    };
+    auto load_x = [&](int q, int v) {
+        const int u = __builtin_amdgcn_readfirstlane(4 * q + v);
+#pragma unroll
+        for (int t = 0; t < 4; t++) x[v][t] = __builtin_amdgcn_raw_buffer_load_b128(rx, xo[t], 256 * u, 0);
+    };
+    // between a wave's own LDS writes and reads: its LDS operations run in
+    // order, so only the compiler has to keep theirs
+    auto order = [] { asm volatile("" ::: "memory"); };
+    // IQ4_NL adds a block at a time: two chains of sums, half as long each
+    float4v acc[NT], ac2[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[j] = ac2[j] = (float4v){0.f, 0.f, 0.f, 0.f};
+    bool odd = false;  // a W4A16 zero that is no whole number was seen
+    if (kg < nq) {
+        load_w(kg);
+#pragma unroll
+        for (int v = 0; v < 4; v++) load_x(kg, v);
+    }
+    for (int q = kg; q < nq; q += WK) {
+        u32x4 sc[NT][SD];
+        order();
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) *reinterpret_cast<u32x4*>(ws + j * 4096 + put[v]) = w[j][v];
+#pragma unroll
+            for (int d = 0; d < SD; d++) sc[j][d] = sn[j][d];
+        }
+        const bool more = q + WK < nq;
+        if (more) load_w(q + WK);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            order();
+#pragma unroll
+            for (int t = 0; t < 4; t++) *reinterpret_cast<u32x4*>(xs + put[t]) = x[v][t];
+            order();
+            if (more) load_x(q + WK, v);
+            __builtin_amdgcn_sched_barrier(0);
+            if (4 * q + v < nu) {
+                half8v ao[4];
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const u32x4 o = *reinterpret_cast<const u32x4*>(xs + get[b]);
+                    const u32x4 e = F == W4A16
+                        ? (u32x4){__builtin_amdgcn_perm(o[2], o[0], 0x05040100u), __builtin_amdgcn_perm(o[2], o[0], 0x07060302u),
+                                  __builtin_amdgcn_perm(o[3], o[1], 0x05040100u), __builtin_amdgcn_perm(o[3], o[1], 0x07060302u)}
+                        : (u32x4){__builtin_amdgcn_perm(o[1], o[0], 0x05040100u), __builtin_amdgcn_perm(o[3], o[2], 0x05040100u),
+                                  __builtin_amdgcn_perm(o[1], o[0], 0x07060302u), __builtin_amdgcn_perm(o[3], o[2], 0x07060302u)};
+                    ao[b] = __builtin_bit_cast(half8v, e);
+                }
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    Raw r;
+                    r.a = *reinterpret_cast<const u32x4*>(ws + j * 4096 + get[v]);
+                    transpose4(r.a);
+                    half2v z1 = splat2(0.f), z2 = z1;
+                    float s = 0.f;
+                    if constexpr (F == W4A16) {
+                        const float z = h2f((uint16_t)(sc[j][0][v] >> 16)), zi = whole_zero(z);
+                        z1 = splat2(-1024.0f - zi);
+                        z2 = splat2(-64.0f - zi);
+                        s = h2f((uint16_t)sc[j][0][v]);
+                        odd |= z != zi;
+                    } else {
+#pragma unroll
+                        for (int d = 0; d < 2; d++) r.s[d] = sc[j][v >> 1][2 * (v & 1) + d];
+                    }
+                    float4v d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int b = 0; b < 4; b++) {
+                        half8v bo[PW];
+                        decode<F>(r, b, 0, lg, z1, z2, bo);
+                        if constexpr (F == W4A16) {
+                            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ao[b], bo[0], d, 0, 0, 0);
+                        } else {
+                            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ao[b], bo[0], (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ao[b], bo[PW - 1], d, 0, 0, 0);
+                            const float t = block_scale<F>(r, b, 0);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) {
+                                float4v& sum = b & 1 ? ac2[j] : acc[j];
+                                sum[e] = __builtin_fmaf(t, d[e], sum[e]);
+                            }
+                        }
+                    }
+                    if constexpr (F == W4A16) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[j][e] = __builtin_fmaf(s, d[e], acc[j][e]);
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (F == W4A16) {
+        // (after the walk: a branch in it, between an MFMA and the first use of
+        // its result, compiled to a read of the result before it was there)
+        // the rests of such zeros: s * rest * sum x off, a unit at a time (all-ones B operands give sum x)
+        if (__builtin_expect(__any(odd), 0)) {
+            const half2v one = splat2(1.0f);
+            const half8v ones = join(one, one, one, one);
+            const uint32_t xr = (uint32_t)min(li, p.T - 1) * (uint32_t)p.K * 2u + 16u * lg;
+            for (int q = kg; q < nq; q += WK)
+                for (int u = 4 * q; u < min(4 * q + 4, nu); u++) {
+                    const int us = __builtin_amdgcn_readfirstlane(u);
+                    float4v sx = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int b = 0; b < 4; b++)
+                        sx = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            __builtin_bit_cast(half8v, __builtin_amdgcn_raw_buffer_load_b128(rx, xr + 64 * b, 256 * us, 0)),
+                            ones, sx, 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < NT; j++) {
+                        const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(rs, so[j], 4 * (us / p.gu), 0);
+                        const float z = h2f((uint16_t)(v >> 16)), m = -h2f((uint16_t)v) * (z - whole_zero(z));
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[j][e] = __builtin_fmaf(m, sx[e], acc[j][e]);
+                    }
+                }
+        }
+    }
+    // the waves' sums, over the whole stage: every wave is past its last read of it
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) red[(kg * NT + j) * 256 + e * 64 + lane] = acc[j][e] + ac2[j][e];
+    __syncthreads();
+    for (int o = threadIdx.x; o < NT * 256; o += 64 * WK) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int g = 0; g < WK; g++) sum += red[g * (NT * 256) + o];
+        const int ln = o & 63, tok = 4 * (ln >> 4) + ((o >> 6) & 3), row = n0 + (o >> 8) * 16 + (ln & 15);
+        if (tok < p.T && row < p.rows) p.c[(long)tok * p.rows + row] = sum;
+    }
+}
+
+template <Fmt F, int NT, int WK>
+hipError_t launch_few(const WideArgs& a, hipStream_t st) {
+    constexpr int shm = WK * 4096 * (1 + NT);
+    if constexpr (shm > 65536) {
+        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_gemm_kernel<F, NT, WK>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+        if (set != hipSuccess) return set;
+    }
+    few_gemm_kernel<F, NT, WK><<<ceil_div(a.rows, 16 * NT), 64 * WK, shm, st>>>(a);
+    return hipGetLastError();
+}
+
 template <Fmt F, int P, int MT, int NT, int WN, int WK>
 hipError_t launch_tile(const WideArgs& a, hipStream_t st) {
     constexpr int xb = 2 * WK * MT * steps_of(P) * P * 1024, rb = WK > 1 ? WK / 2 * WN * MT * NT * 1024 : 0;
@@ -803,6 +1014,18 @@ hipError_t launch_gemm(const WideArgs& a, hipStream_t st) {
     return launch_tile<F, P, 4, 2, 4, 1>(a, st);
 }
 
+// One 16-row tile a wave and 8 waves along K while that gives the CUs one
+// workgroup each, two tiles up to 8192 rows (8192 x 8192, 16 tokens, W4A16:
+// 15.2 us, 19.8 with one tile), then shorter workgroups, several a CU (18944 x
+// 3584 rows x K, 8 tokens, IQ4_NL: 23.9 us with 4 waves, 30.8 with 8).
+template <Fmt F>
+hipError_t launch_few_gemm(const WideArgs& a, hipStream_t st) {
+    if (a.rows <= 4096) return launch_few<F, 1, 8>(a, st);
+    if (a.rows <= 8192) return launch_few<F, 2, 8>(a, st);
+    if (F == W4A16 && a.rows > 24576) return launch_few<F, 2, 2>(a, st);
+    return launch_few<F, 1, 4>(a, st);
+}
+
 // Bytes of the packed activations of T tokens (whole 128-token tiles: the
 // largest tile's reads stay inside), of the token scales and of the block sums.
 long padded(int T) { return (long)(T + 127) / 128 * 128; }
@@ -821,6 +1044,13 @@ hipError_t launch_fmt(const WideArgs& a, const void* X, hipStream_t st) {
     constexpr bool S = has_mins(F);
     using XT = std::conditional_t<P == 2, float, uint16_t>;
     const XT* x = static_cast<const XT*>(X);
+    if constexpr (P == 1) {
+        if (a.T <= 16) {  // the activations as they are
+            WideArgs b = a;
+            b.xp = reinterpret_cast<const char*>(x);
+            return launch_few_gemm<F>(b, st);
+        }
+    }
     const int ni = ceil_div(S ? (a.K + 1023) & ~1023 : a.K, 8 * kPackThreads);
     if (ni <= 1) launch_pack<O, XT, S, 1>(a, x, st);
     else if (ni <= 2) launch_pack<O, XT, S, 2>(a, x, st);

@@ -277,7 +277,7 @@ class ROCmEngine:
             if a.shape[-1] != k:
                 raise ValueError(f"matmul: A has {a.shape[-1]} columns but B is [{k},{nout}]")
             m = a.numel() // k
-            if _wide_tokens(m):
+            if _wide_tokens(m) or _few_tokens(b.storage, nout, k, m):
                 ct = self._wide_times(b.storage, nout, k, a.reshape(m, k))
                 if ct is not None:
                     return ct.reshape(*a.shape[:-1], nout)
@@ -909,6 +909,27 @@ def _wide_tokens(t: int, transposed: bool = False) -> bool:
     chunks where the activations and the result are also to be transposed
     (a weight on the A side)."""
     return t > (32 if transposed else 16)
+
+
+def _few_tokens(s: Any, rows: int, k: int, t: int) -> bool:
+    """Whether 2 to 16 tokens go to the token-major GEMM too, which spares
+    the two transposes (about 4 us each) and, for counts that are no multiple
+    of 4, the padding (five small launches).  W4A16 and IQ4_NL (one launch
+    without packing, for fp16 activations): while the matrix is small enough
+    that this weighs more than the tiled layout gives, and every padded count
+    (W4A16, 8 tokens 8192 x 8192 14.7 us against 13.2 + 7.3, 28672 x 8192 41
+    against 29 + 8, 16 tokens 4096 x 4096 6.4 against 6.4 + 7; IQ4_NL, 8 tokens
+    3584 x 3584 7.5 against 7.9 + 7.4, 18944 x 3584 23.9 against 19.4 + 8.6).
+    The formats that pack fp32 activations first: padded counts of small
+    matrices (a layer of 2048 x 5632 matrices, Q4_0, 2 tokens 107 -> 76 us;
+    Llama-3-8B's, whose MLP matrices stay tiled here, would go from 157 to
+    150 in Q4_0 at 6 tokens but from 162 to 193 in Q4_K / Q6_K at 3)."""
+    if not 2 <= t <= 16:
+        return False
+    if isinstance(s, (GPTQStorage, AWQStorage, IQ4NLStorage)):
+        # 12 and 16 tokens past 4096 rows have a tiled copy of their own
+        return t % 4 != 0 or (rows * k <= 1 << 27 and (t <= 8 or rows <= 4096))
+    return t % 4 != 0 and rows * k <= 1 << 24 and k <= 4096
 
 
 # zt_gemm_wide_f32 formats (ZT_WIDE_*)
