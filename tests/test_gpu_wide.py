@@ -130,6 +130,76 @@ def test_few_tokens(eng, orc, fmt, rows, K, T):
     assert torch.equal(eng.matmul(torch.from_numpy(x).cuda(), st.Tensor((K, rows), s)), y)
 
 
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("rows,K", [(1, 256), (37, 768), (130, 1280), (2060, 3328), (16400, 5120)])
+def test_tiled_tokens_are_the_columns(eng, orc, monkeypatch, fmt, rows, K):
+    """The token-major calls on the tiled copies give the column-major calls' bits: every token count, one and
+    several K ranges and chunks, ragged rows, an unaligned and a transposed X."""
+    if rows > 3000 and fmt not in ("gptq", "q4_0", "q6_k", "iq4_nl_f16"):
+        pytest.skip("one format of each kernel on the large matrix")
+    import ztensor_amd.engine as E
+
+    # the columns on the tiled copy too
+    monkeypatch.setattr(E, "_block_rowblock", lambda *a: False)
+    monkeypatch.setattr(E, "_w4a16_rowblock", lambda *a: False)
+    if fmt in ("iq4_nl", "iq4_nl_f16"):
+        fmt, K = "iq4_nl_f16", K + 8192  # past 8192 they always are
+    s, _ = weights(fmt, rows, K, rows + K, orc)
+    for T in range(2, 17) if rows < 3000 else (3, 8, 11, 16):
+        x = torch.from_numpy(activations(fmt, T, K, T)).cuda()
+        y = eng._tiled_tokens(s, rows, K, x)
+        n = -(-T // 4) * 4
+        xp = torch.zeros((K, n), dtype=x.dtype, device="cuda")
+        xp[:, :T] = x.t()
+        assert torch.equal(y, eng._weight_times(s, rows, K, xp)[:, :T].t()), T
+        off = torch.empty(T * K + 1, dtype=x.dtype, device="cuda")[1:].view(T, K).copy_(x)
+        assert torch.equal(eng._tiled_tokens(s, rows, K, off), y)
+        assert torch.equal(eng._tiled_tokens(s, rows, K, x.t().contiguous().t()), y)
+
+
+@pytest.mark.parametrize("fmt,rows,K,T", [("gptq", 100, 8192, 5), ("q4_0", 100, 512, 4), ("q8_0", 300, 1024, 3),
+                                          ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6),
+                                          ("iq4_nl_f16", 64, 5120, 8)])
+def test_tiled_tokens_build_a_copy_only_at_no_risk(eng, orc, fmt, rows, K, T):
+    """Where the columns need no tiled copy the tokens make one, but neither in a capture nor at the memory limit;
+    both ways give the result."""
+    s, w = weights(fmt, rows, K, rows + T, orc)
+    x = activations(fmt, T, K, T)
+    xd = torch.from_numpy(x).cuda()
+    careful = ROCmEngine(split_reserve_bytes=1 << 60)
+    check(careful.matmul(xd, st.Tensor((K, rows), s)).cpu().numpy(), x, w)
+    assert getattr(s, "_gpu_tiled", None) is None
+    side = torch.cuda.Stream()
+    cap = ROCmEngine(stream=side)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side), torch.cuda.graph(g, stream=side):
+        y = cap.matmul(xd, st.Tensor((K, rows), s))
+    assert getattr(s, "_gpu_tiled", None) is None
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            g.replay()
+        torch.cuda.synchronize()
+        check(y.cpu().numpy(), x, w)
+    z = eng.matmul(xd, st.Tensor((K, rows), s))
+    assert s._gpu_tiled is not None
+    check(z.cpu().numpy(), x, w)
+    assert torch.equal(careful.matmul(xd, st.Tensor((K, rows), s)), z)  # the copy is there
+
+
+def test_tiled_tokens_entry_point_errors(eng):
+    lib, p = eng.lib, 1 << 20
+    for t in (0, 17):
+        assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p, p, 16, 128, t, 0, 0, 0) == 1
+        assert lib.zt_gemm_w4a16t_tokens_f32(p, p, p, p, 16, 128, t, 128, 0, 0, 0) == 1
+        assert lib.zt_gemm_iq4nlt_tokens_f16(p, p, p, p, 16, 128, t, 0, 0, 0) == 1
+    assert lib.zt_gemm_blkt_tokens_f32(0, p, p, 0, p, p, 16, 128, 4, 0, 0, 0) == 1  # W4A16 and IQ4_NL have their own
+    assert lib.zt_gemm_blkt_tokens_f32(4, p, p, 0, p, p, 16, 128, 4, 0, 0, 0) == 1  # no fifth bits
+    assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p + 4, p, 16, 128, 4, 0, 0, 0) == 1  # X alignment
+    assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p, p, 16, 1 << 25, 4, 0, 0, 0) == 1
+    assert lib.zt_gemm_w4a16t_tokens_f32(p, p, p, p, 16, 1 << 26, 4, 128, 0, 0, 0) == 1
+
+
 def test_few_tokens_special_values(eng, orc):
     """Infinities and NaN stay in their tokens."""
     s, w = weights("gptq", 40, 640, 3, orc)

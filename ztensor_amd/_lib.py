@@ -39,6 +39,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "zt_iq4nl_tile": (I, [P, I, I, I, P, P, P]),
     "zt_gemm_iq4nlt_workspace_bytes": (L, [I, I, I]),
     "zt_gemm_iq4nlt_f16": (I, [P, P, P, P, I, I, I, P, L, P]),
+    "zt_gemm_iq4nlt_tokens_f16": (I, [P, P, P, P, I, I, I, P, L, P]),
     "zt_iq4nl_raw_to_gpu": (None, [P, L, P]),
     "zt_gemm_q8_f32": (I, [P, P, P, I, I, I, P]),
     "zt_gemm_q8sep_f32": (I, [P, P, P, I, I, I, L, P]),
@@ -68,6 +69,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "zt_w4a16_tile": (I, [P, P, P, I, I, I, P, P, P]),
     "zt_gemm_w4a16t_workspace_bytes": (L, [I, I, I]),
     "zt_gemm_w4a16t_f32": (I, [P, P, P, P, I, I, I, I, P, L, P]),
+    "zt_gemm_w4a16t_tokens_f32": (I, [P, P, P, P, I, I, I, I, P, L, P]),
     "zt_q4_tiled_bytes": (L, [I, I]),
     "zt_q4_tiled_scale_bytes": (L, [I, I]),
     "zt_q4_tile": (I, [P, I, I, I, P, P, P]),
@@ -102,6 +104,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "zt_q6k_tile": (I, [P, I, I, P, P, P]),
     "zt_gemm_q6kt_workspace_bytes": (L, [I, I, I]),
     "zt_gemm_q6kt_f32": (I, [P, P, P, P, I, I, I, P, L, P]),
+    "zt_gemm_blkt_tokens_f32": (I, [I, P, P, P, P, P, I, I, I, P, L, P]),
     "zt_ternary_gemv_f32": (I, [P, P, P, I, I, P]),
     "zt_ternary_gemv_i8": (I, [P, P, P, P, P, I, I, P]),
     "zt_dequant_ternary_f32": (I, [P, P, I, I, P]),

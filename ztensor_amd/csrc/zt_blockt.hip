@@ -259,18 +259,34 @@ __device__ __forceinline__ int blkt_lds_row(int r) {
     return (u << 7) + (g << 5) + (b << 3) + j;
 }
 
-template <BlkFmt F, int UPW, int N>
+// Token-major staging: LDS piece (lane group g, block b) of a unit holds the 8
+// elements above in the order of the A operand's halves.  They are two runs of
+// 4 in the block: run h's byte offset, and the half that element c of the two
+// runs goes to.
+template <BlkFmt F>
+__device__ __forceinline__ int blkt_token_off(int g, int h) {
+    return F == BlkFmt::Q8_0 ? 32 * g + 16 * h : 16 * g + 64 * h;
+}
+
+template <BlkFmt F>
+__device__ constexpr int blkt_token_slot(int c) {
+    if (F == BlkFmt::Q8_0 || F == BlkFmt::Q6_K) return c;
+    return (c & 1) * 4 + ((c & 3) >> 1) + ((c >> 2) << 1);
+}
+
+template <BlkFmt F, int UPW, int N, bool TM>
 __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict__ wt, const void* __restrict__ stl,
                                                         const uint32_t* __restrict__ aux, const float* __restrict__ x,
-                                                        int rows, int K, int gx, int gy, float* __restrict__ y,
+                                                        int rows, int K, int gx, int gy, int T, float* __restrict__ y,
                                                         float* __restrict__ ws) {
     constexpr int W = 4;
     constexpr int KC = 128 * UPW;
     constexpr int RW = 32 * W;
     constexpr int NPL = N <= 8 ? 1 : 2;                 // staged fp16 planes (hi/lo in columns, or two planes)
-    constexpr int XPB = mfma_chunk_xbytes(KC, 16);      // one plane: 16 fp16 columns, 2 pad rows per 32
+    constexpr int XPB = TM ? KC * 32 : mfma_chunk_xbytes(KC, 16);  // one plane: 16 fp16 columns, 2 pad rows per 32
     constexpr int PPR = N / 4;                          // 16-byte pieces per fp32 activation row
-    constexpr int XP = (KC * PPR + W * 64 - 1) / (W * 64);
+    // loads a thread: single 16-byte pieces, token-major in pairs (the 8 values of one LDS piece)
+    constexpr int XP = TM ? 2 * ((KC / 8 * N + W * 64 - 1) / (W * 64)) : (KC * PPR + W * 64 - 1) / (W * 64);
     constexpr bool QK = F == BlkFmt::Q4_K || F == BlkFmt::Q5_K;  // super-block headers: (d*scale, dmin*min)
     constexpr bool Q5 = F == BlkFmt::Q5_0 || F == BlkFmt::Q5_K;  // fifth-bit dwords in aux
     constexpr bool Q6 = F == BlkFmt::Q6_K;  // byte values, one scale per 16: two half-steps
@@ -299,12 +315,23 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
     const int ntiles = (rows + 15) / 16;
     const int npieces = (u1 - u0) * 128 * PPR;
     const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)u0 * 128 * N), (short)0, npieces * 16, 0x00020000);
+        TM ? __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, T * K * 4, 0x00020000)
+           : __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)u0 * 128 * N), (short)0, npieces * 16, 0x00020000);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)stl, (short)0, 0x7fffffff, 0x00020000);
     u32x4 xr[XP];
 #pragma unroll
-    for (int i = 0; i < XP; i++)
-        xr[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, (uint32_t)(tid + i * W * 64) * 16u, 0, 0);
+    for (int i = 0; i < XP; i++) {
+        uint32_t off = (uint32_t)(tid + i * W * 64) * 16u;
+        if constexpr (TM) {
+            // the halves of piece e of a token: block e / 4's lane group e % 4
+            // (past the tokens or the chunk's units: zeros)
+            const int p = tid + (i >> 1) * W * 64, t = p / (KC / 8), e = p % (KC / 8);
+            off = t < T && e < 16 * (u1 - u0)
+                      ? (uint32_t)t * (uint32_t)K * 4u + (uint32_t)(u0 * 512 + (e >> 2) * 128 + blkt_token_off<F>(e & 3, i & 1))
+                      : 0x80000000u;
+        }
+        xr[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0);
+    }
     u32x4 sr[SP];
 #pragma unroll
     for (int i = 0; i < SP; i++) {
@@ -364,31 +391,53 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
         sh = min(127, 15 - e2);
     }
     const float cs = ldexpf(1.0f, sh);
+    if constexpr (TM) {
+        // hi and lo rows of a token: planes of 16 rows, or (N <= 8) rows t and 8 + t of one plane
 #pragma unroll
-    for (int i = 0; i < XP; i++) {
-        const int p = tid + i * W * 64;
-        if (p < npieces) {
-            const int r = p / PPR, c4 = (p % PPR) * 4;
-            const float cr = cs;
-            const int base = mfma_xrow(blkt_lds_row<F>(r), 16);
-            uint32_t hv[2], lv[2];
+        for (int i = 0; i < XP; i += 2) {
+            const int p = tid + (i >> 1) * W * 64, t = p / (KC / 8), e = p % (KC / 8);
+            if (p < N * (KC / 8)) {
+                uint16_t h[8], l[8];
 #pragma unroll
-            for (int c = 0; c < 4; c += 2) {
-                const float v0 = __uint_as_float(xr[i][c]) * cr, v1 = __uint_as_float(xr[i][c + 1]) * cr;
-                const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
-                const _Float16 l0 = (_Float16)(v0 - (float)h0), l1 = (_Float16)(v1 - (float)h1);
-                hv[c / 2] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-                lv[c / 2] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
+                for (int c = 0; c < 8; c++) {
+                    const float v = __uint_as_float(xr[i + (c >> 2)][c & 3]) * cs;
+                    const _Float16 hv = (_Float16)v;
+                    h[blkt_token_slot<F>(c)] = __builtin_bit_cast(uint16_t, hv);
+                    l[blkt_token_slot<F>(c)] = __builtin_bit_cast(uint16_t, (_Float16)(v - (float)hv));
+                }
+                const int piece = (e & ~15) + 4 * (e & 3) + ((e >> 2) & 3);
+                *reinterpret_cast<short8v*>(smem + token_slot(t, piece, KC)) = __builtin_bit_cast(short8v, h);
+                *reinterpret_cast<short8v*>(smem + (NPL == 1 ? token_slot(8 + t, piece, KC) : XPB + token_slot(t, piece, KC))) =
+                    __builtin_bit_cast(short8v, l);
             }
-            const int lo_off = NPL == 1 ? 16 : XPB;
-            if (N % 8 != 0 && c4 == N - 4) {
-                // last piece of a row: it also zeroes the unused columns up to the
-                // next multiple of 8, so every lane of a transposing read reads data
-                *reinterpret_cast<uint4*>(smem + base + 2 * c4) = make_uint4(hv[0], hv[1], 0u, 0u);
-                *reinterpret_cast<uint4*>(smem + lo_off + base + 2 * c4) = make_uint4(lv[0], lv[1], 0u, 0u);
-            } else {
-                *reinterpret_cast<uint2*>(smem + base + 2 * c4) = make_uint2(hv[0], hv[1]);
-                *reinterpret_cast<uint2*>(smem + lo_off + base + 2 * c4) = make_uint2(lv[0], lv[1]);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < XP; i++) {
+            const int p = tid + i * W * 64;
+            if (p < npieces) {
+                const int r = p / PPR, c4 = (p % PPR) * 4;
+                const float cr = cs;
+                const int base = mfma_xrow(blkt_lds_row<F>(r), 16);
+                uint32_t hv[2], lv[2];
+#pragma unroll
+                for (int c = 0; c < 4; c += 2) {
+                    const float v0 = __uint_as_float(xr[i][c]) * cr, v1 = __uint_as_float(xr[i][c + 1]) * cr;
+                    const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
+                    const _Float16 l0 = (_Float16)(v0 - (float)h0), l1 = (_Float16)(v1 - (float)h1);
+                    hv[c / 2] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
+                    lv[c / 2] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
+                }
+                const int lo_off = NPL == 1 ? 16 : XPB;
+                if (N % 8 != 0 && c4 == N - 4) {
+                    // last piece of a row: it also zeroes the unused columns up to the
+                    // next multiple of 8, so every lane of a transposing read reads data
+                    *reinterpret_cast<uint4*>(smem + base + 2 * c4) = make_uint4(hv[0], hv[1], 0u, 0u);
+                    *reinterpret_cast<uint4*>(smem + lo_off + base + 2 * c4) = make_uint4(lv[0], lv[1], 0u, 0u);
+                } else {
+                    *reinterpret_cast<uint2*>(smem + base + 2 * c4) = make_uint2(hv[0], hv[1]);
+                    *reinterpret_cast<uint2*>(smem + lo_off + base + 2 * c4) = make_uint2(lv[0], lv[1]);
+                }
             }
         }
     }
@@ -429,6 +478,11 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
     // 4 qq + 3; mfma_xrow of that row is this lane base plus (136u + 8s) * 32.
     const int jq = li >> 2, qq = li & 3;
     const int lbase = (34 * lg + jq) * 32 + 8 * qq;
+    // token-major: piece 16u + 4 lg + s of row li (an unused column repeats a used one)
+    int pb[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+        pb[s] = token_slot(NPL == 1 ? (li & 8) + min(li & 7, N - 1) : min(li, N - 1), 4 * lg + s, KC);
     // -(base + off 2^10) in every A element: one MFMA a step gives that times
     // sum(x), the C input of both tiles' weight MFMAs, so each step's D is
     // 2^10 sum((q - off) x) (Q6_K: 2^9, Q8_0: 2^7).
@@ -465,6 +519,10 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
                 half8v bv[NPL];
 #pragma unroll
                 for (int pl = 0; pl < NPL; pl++) {
+                    if constexpr (TM) {
+                        bv[pl] = *reinterpret_cast<const half8v*>(smem + pb[s] + pl * XPB + 256 * u);
+                        continue;
+                    }
                     const int o = pl * XPB + (136 * u + 8 * s) * 32;
                     const short4v ba = tr_read_b64(smem, lbase + o), bb = tr_read_b64(smem, lbase + o + 128);
                     bv[pl] = __builtin_bit_cast(half8v, (short8v){ba[0], ba[1], ba[2], ba[3], bb[0], bb[1], bb[2], bb[3]});
@@ -601,27 +659,42 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = row0 + 16 * t + 4 * lg + i;
-                if (row < rows) y[(long)row * N + li] = acc[t][i];
+                if constexpr (TM) {
+                    if (row < rows && li < T) y[(long)li * rows + row] = acc[t][i];
+                } else {
+                    if (row < rows) y[(long)row * N + li] = acc[t][i];
+                }
             }
     }
 }
 
-template <BlkFmt F, int UPW, int N>
+template <BlkFmt F, int UPW, int N, bool TM>
 static void launch_blkt(dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux, const float* x,
-                        float* y, float* ws, int M, int K) {
+                        float* y, float* ws, int M, int K, int T) {
     constexpr int NPL = N <= 8 ? 1 : 2;
     constexpr int SB = F == BlkFmt::Q8_0 ? 4 : (F == BlkFmt::Q4_K || F == BlkFmt::Q5_K || F == BlkFmt::Q6_K) ? 8 : 2;  // LDS bytes per (row, block)
     const size_t lds = (size_t)NPL * mfma_chunk_xbytes(128 * UPW, 16) + 16 + (size_t)8 * UPW * 64 * SB;
-    blkt_mfma_kernel<F, UPW, N><<<g, 256, lds, st>>>(wt, sc, aux, x, M, K, (int)g.x, (int)g.y, y, ws);
+    blkt_mfma_kernel<F, UPW, N, TM><<<g, 256, lds, st>>>(wt, sc, aux, x, M, K, (int)g.x, (int)g.y, T, y, ws);
 }
 
-template <BlkFmt F, int N>
+template <BlkFmt F, int N, bool TM>
 static void launch_blkt_n(int upw, dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux,
-                          const float* x, float* y, float* ws, int M, int K) {
+                          const float* x, float* y, float* ws, int M, int K, int T) {
     if (upw >= 4)
-        launch_blkt<F, 4, N>(g, st, wt, sc, aux, x, y, ws, M, K);
+        launch_blkt<F, 4, N, TM>(g, st, wt, sc, aux, x, y, ws, M, K, T);
     else
-        launch_blkt<F, 2, N>(g, st, wt, sc, aux, x, y, ws, M, K);
+        launch_blkt<F, 2, N, TM>(g, st, wt, sc, aux, x, y, ws, M, K, T);
+}
+
+template <BlkFmt F, bool TM>
+static void launch_blkt_any(int upw, dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux,
+                            const float* x, float* y, float* ws, int M, int K, int N, int T) {
+    switch (N) {
+        case 4: launch_blkt_n<F, 4, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
+        case 8: launch_blkt_n<F, 8, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
+        case 12: launch_blkt_n<F, 12, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
+        default: launch_blkt_n<F, 16, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
+    }
 }
 
 // Grid of a tiled block GEMM: 128 rows by the largest K range per
@@ -649,7 +722,8 @@ static long blkt_ws_bytes(int M, int K, int N) {
 
 template <BlkFmt F>
 static int gemm_blkt(const void* W_tiled, const void* S_tiled, const float* B, float* C, int M, int K, int N,
-                     void* ws, long ws_bytes, hipStream_t stream, const void* aux = nullptr, int force_upw = 0) {
+                     void* ws, long ws_bytes, hipStream_t stream, const void* aux = nullptr, int force_upw = 0,
+                     int tokens = 0) {
     constexpr int KQ = (F == BlkFmt::Q4_K || F == BlkFmt::Q5_K || F == BlkFmt::Q6_K) ? 256 : 128;  // K-quants: whole super-blocks
     if (M < 0 || K < 0 || K % KQ != 0) return (int)hipErrorInvalidValue;
     if (N != 4 && N != 8 && N != 12 && N != 16) return (int)hipErrorInvalidValue;
@@ -671,13 +745,13 @@ static int gemm_blkt(const void* W_tiled, const void* S_tiled, const float* B, f
     if (need > 0 && (ws == nullptr || ws_bytes < need || ((uintptr_t)ws & 15))) return (int)hipErrorInvalidValue;
     const uint4* wt = static_cast<const uint4*>(W_tiled);
     float* wsf = static_cast<float*>(ws);
-    switch (N) {
-        case 4: launch_blkt_n<F, 4>(upw, g, stream, wt, S_tiled, static_cast<const uint32_t*>(aux), B, C, wsf, M, K); break;
-        case 8: launch_blkt_n<F, 8>(upw, g, stream, wt, S_tiled, static_cast<const uint32_t*>(aux), B, C, wsf, M, K); break;
-        case 12: launch_blkt_n<F, 12>(upw, g, stream, wt, S_tiled, static_cast<const uint32_t*>(aux), B, C, wsf, M, K); break;
-        default: launch_blkt_n<F, 16>(upw, g, stream, wt, S_tiled, static_cast<const uint32_t*>(aux), B, C, wsf, M, K); break;
-    }
-    if (g.y > 1) tiled_reduce(ws, C, M, N, (int)g.y, stream);
+    const uint32_t* ax = static_cast<const uint32_t*>(aux);
+    // tokens > 0: B[tokens][K] and C[tokens][M], N = tokens up to a multiple of 4
+    if (tokens > 0)
+        launch_blkt_any<F, true>(upw, g, stream, wt, S_tiled, ax, B, C, wsf, M, K, N, tokens);
+    else
+        launch_blkt_any<F, false>(upw, g, stream, wt, S_tiled, ax, B, C, wsf, M, K, N, tokens);
+    if (g.y > 1) tiled_reduce(ws, C, M, N, (int)g.y, stream, tokens);
     return (int)hipGetLastError();
 }
 
@@ -956,4 +1030,21 @@ ZT_EXPORT long zt_gemm_q6kt_workspace_bytes(int M, int K, int N) { return blkt_w
 ZT_EXPORT int zt_gemm_q6kt_f32(const void* W_tiled, const void* S_tiled, const float* B, float* C, int M, int K, int N,
                                void* workspace, long workspace_bytes, hipStream_t stream) {
     return gemm_blkt<BlkFmt::Q6_K>(W_tiled, S_tiled, B, C, M, K, N, workspace, workspace_bytes, stream);
+}
+
+ZT_EXPORT int zt_gemm_blkt_tokens_f32(int fmt, const void* W_tiled, const void* S_tiled, const void* aux,
+                                      const float* X, float* C, int M, int K, int T, void* ws, long ws_bytes,
+                                      hipStream_t stream) {
+    if (T < 1 || T > 16 || K >= 1 << 25) return (int)hipErrorInvalidValue;
+    const int N = (T + 3) & ~3;
+    switch (fmt) {
+        case ZT_WIDE_Q4_0: return gemm_blkt<BlkFmt::Q4_0>(W_tiled, S_tiled, X, C, M, K, N, ws, ws_bytes, stream, aux, 0, T);
+        case ZT_WIDE_Q8_0:
+        case ZT_WIDE_Q8_GGUF: return gemm_blkt<BlkFmt::Q8_0>(W_tiled, S_tiled, X, C, M, K, N, ws, ws_bytes, stream, aux, 0, T);
+        case ZT_WIDE_Q5_0: return gemm_blkt<BlkFmt::Q5_0>(W_tiled, S_tiled, X, C, M, K, N, ws, ws_bytes, stream, aux, 0, T);
+        case ZT_WIDE_Q4_K: return gemm_blkt<BlkFmt::Q4_K>(W_tiled, S_tiled, X, C, M, K, N, ws, ws_bytes, stream, aux, 0, T);
+        case ZT_WIDE_Q5_K: return gemm_blkt<BlkFmt::Q5_K>(W_tiled, S_tiled, X, C, M, K, N, ws, ws_bytes, stream, aux, 0, T);
+        case ZT_WIDE_Q6_K: return gemm_blkt<BlkFmt::Q6_K>(W_tiled, S_tiled, X, C, M, K, N, ws, ws_bytes, stream, aux, 0, T);
+        default: return (int)hipErrorInvalidValue;
+    }
 }

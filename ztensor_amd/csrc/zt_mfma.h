@@ -125,15 +125,30 @@ __device__ __forceinline__ void mfma_reduce_store(float4v (&acc)[kMfmaTiles], ch
 // zero fill, no atomics, and the same result on every run.  The workspace
 // holds splits * ntiles KB.  Partials are stored and loaded nontemporally:
 // they are read once, by the next kernel (with ordinary stores the GEMM
-// measured 10-15% slower at the Llama-3-8B shapes, batch 16).
+// measured 10-15% slower at the Llama-3-8B shapes, batch 16).  Token-major
+// calls (tokens > 0: C[tokens][rows]) write C in runs of 16 bytes.
 
 __device__ __forceinline__ void tiled_store_partial(const float4v& v, float* __restrict__ ws, int split, int ntiles,
                                                     int rt, int lane, int N) {
     if ((lane & 15) < N) __builtin_nontemporal_store(v, reinterpret_cast<float4v*>(ws + (((long)split * ntiles + rt) * 64 + lane) * 4));
 }
 
+// ---- token-major activations (tiled kernels)
+//
+// X[T][K], C[T][rows]: a K chunk of each token is a row of KC halves in LDS,
+// 16-byte piece c at position c ^ token within each 128-K unit's 16 pieces,
+// so the 16 columns' reads of one piece spread over all banks and need no
+// transposing read.  This spares the two transposes around a channel-major
+// call and the padding of T to a multiple of 4 (us, 3 / 16 tokens, with
+// those: W4A16 8192 x 8192 25.0 / 18.9 -> 11.6 / 13.3, 28672 x 8192 43.7 /
+// 40.2 -> 28.5 / 32.9; Q4_0 14336 x 4096 23.7 / 22.9 -> 12.3 / 17.8; Q6_K
+// 14336 x 4096 31.6 / 28.4 -> 18.5 / 23.5).
+__device__ __forceinline__ int token_slot(int row, int piece, int KC) {
+    return row * KC * 2 + ((piece & ~15) | ((piece ^ row) & 15)) * 16;
+}
+
 static __global__ void __launch_bounds__(64) tiled_reduce_kernel(const float* __restrict__ ws, float* __restrict__ y,
-                                                                 int rows, int N, int ntiles, int splits) {
+                                                                 int rows, int N, int ntiles, int splits, int tokens) {
     // thread = one output of a lane with column < N: (tile, lane 16g + i, element e),
     // consecutive threads on consecutive floats of the partial tiles
     const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -151,17 +166,22 @@ static __global__ void __launch_bounds__(64) tiled_reduce_kernel(const float* __
         for (int j = 0; j < 32; j++) s += v[j];
     }
     const long row = rt * 16 + 4 * lg + e;
-    if (row < rows) y[row * N + li] = s;
+    if (tokens > 0) {
+        if (row < rows && li < tokens) y[(long)li * rows + row] = s;
+    } else if (row < rows) {
+        y[row * N + li] = s;
+    }
 }
 
 __host__ __forceinline__ long tiled_ws_bytes(int rows, int splits) {
     return splits > 1 ? (long)splits * ((rows + 15) / 16) * 1024 : 0;
 }
 
-__host__ __forceinline__ void tiled_reduce(const void* ws, float* y, int rows, int N, int splits, hipStream_t st) {
+__host__ __forceinline__ void tiled_reduce(const void* ws, float* y, int rows, int N, int splits, hipStream_t st,
+                                               int tokens = 0) {
     const int ntiles = (rows + 15) / 16;
     tiled_reduce_kernel<<<(int)(((long)ntiles * 16 * N + 63) / 64), 64, 0, st>>>(
-        static_cast<const float*>(ws), y, rows, N, ntiles, splits);
+        static_cast<const float*>(ws), y, rows, N, ntiles, splits, tokens);
 }
 
 static __global__ void mfma_zero_kernel(float* __restrict__ y, long n) {

@@ -1617,18 +1617,18 @@ __global__ void iq4t_tile_kernel(const uint32_t* __restrict__ data, const uint16
 // 18944 x 3584, batch 8).  Each step's result is scaled by its block's fp16
 // scale in fp32.  The fp16-rounded table with one MFMA a step measured no
 // faster than the split.
-template <int UPW, int W, int N>
+template <int UPW, int W, int N, bool TM>
 __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __restrict__ wt,
                                                              const uint16_t* __restrict__ stl,
                                                              const uint16_t* __restrict__ x, int rows, int K, int nch,
-                                                             int gx, int gy, float* __restrict__ y,
+                                                             int gx, int gy, int T, float* __restrict__ y,
                                                              float* __restrict__ ws) {
     constexpr int KC = 128 * UPW;
     constexpr int RW = 32 * W;
     constexpr int XP = (KC * 2 * N / 16 + W * 64 - 1) / (W * 64);
     constexpr int SPC = RW / 16 * UPW * 128 / 16;  // 16-byte scale pieces of the workgroup
     constexpr int SP = (SPC + W * 64 - 1) / (W * 64);
-    constexpr int XB = mfma_chunk_xbytes(KC, N);
+    constexpr int XB = TM ? KC * 2 * N : mfma_chunk_xbytes(KC, N);
     extern __shared__ __attribute__((aligned(16))) char smem[];
     char* zero_area = smem + XB;
     uint2* tbl = reinterpret_cast<uint2*>(zero_area + 16);         // 256 x (hi pair, lo pair)
@@ -1655,12 +1655,20 @@ __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __rest
     if (ch > 0) asm volatile("s_barrier" ::: "memory");  // every wave is done with the previous chunk's LDS
     const int npieces = (u1 - u0) * 128 * 2 * N / 16;
     const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)u0 * 128 * N), (short)0, npieces * 16, 0x00020000);
+        TM ? __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, T * K * 2, 0x00020000)
+           : __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)u0 * 128 * N), (short)0, npieces * 16, 0x00020000);
+    // the 16 bytes of piece e: past the tokens or the chunk's units an offset
+    // past the buffer (zeros, which nothing uses)
+    auto xoff = [&](int e) -> uint32_t {
+        if constexpr (!TM) return (uint32_t)e * 16u;
+        const int t = e / (KC / 8), c = e % (KC / 8);
+        return t < T && c < 16 * (u1 - u0) ? (uint32_t)t * (uint32_t)K * 2u + (uint32_t)(u0 * 256 + c * 16) : 0x80000000u;
+    };
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)stl, (short)0, 0x7fffffff, 0x00020000);
     u32x4 xr[XP];
 #pragma unroll
     for (int i = 0; i < XP; i++)
-        xr[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, (uint32_t)(tid + i * W * 64) * 16u, 0, 0);
+        xr[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff(tid + i * W * 64), 0, 0);
     // scales: piece e = (tile in WG) * UPW * 8 + unit * 8 + q (8 pieces of 16 bytes a tile-unit)
     u32x4 sr[SP];
 #pragma unroll
@@ -1686,7 +1694,10 @@ __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __rest
 #pragma unroll
     for (int i = 0; i < XP; i++) {
         const int p = tid + i * W * 64;
-        if (p < npieces) {
+        if constexpr (TM) {
+            if (p < N * (KC / 8))
+                *reinterpret_cast<u32x4*>(smem + token_slot(p / (KC / 8), p % (KC / 8), KC)) = xr[i];
+        } else if (p < npieces) {
             const int off = p * 16;
             *reinterpret_cast<u32x4*>(smem + off + (off / (64 * N)) * (4 * N)) = xr[i];
         }
@@ -1701,12 +1712,20 @@ __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __rest
     // step s of unit u reads X rows 128u + 32s + 8lg + (li >> 2) (+ 4), whose
     // padded LDS offset is (8lg + (li >> 2)) 2N + (136u + 34s) 2N
     const int lbase = (8 * lg + (li >> 2)) * 2 * N + 8 * (li & 3);
+    // token-major: piece 16u + 4s + lg of token li (columns >= N repeat the last)
+    int pb[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) pb[s] = token_slot(min(li, N - 1), 4 * s + lg, KC);
 #pragma unroll
     for (int u = 0; u < UPW; u++) {
         if (u0 + u < u1) {
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                const u32x4 bw = __builtin_bit_cast(u32x4, mfma_b_pair(smem, lbase + (136 * u + 34 * s) * 2 * N, 8 * N));
+                u32x4 bw;
+                if constexpr (TM)
+                    bw = *reinterpret_cast<const u32x4*>(smem + pb[s] + 256 * u);
+                else
+                    bw = __builtin_bit_cast(u32x4, mfma_b_pair(smem, lbase + (136 * u + 34 * s) * 2 * N, 8 * N));
                 // activation pairs (x0 x1), (x2 x3) each twice: k slots of the
                 // A operand {entry(byte 0), entry(byte 1)} = Th0 Th1 Tl0 Tl1 Th2 Th3 Tl2 Tl3
                 const half8v b1 = __builtin_bit_cast(half8v, (u32x4){bw[0], bw[0], bw[1], bw[1]});
@@ -1742,26 +1761,41 @@ __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __rest
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = row0 + 16 * t + 4 * lg + i;
-                if (row < rows) y[(long)row * N + li] = acc[t][i];
+                if constexpr (TM) {
+                    if (row < rows && li < T) y[(long)li * rows + row] = acc[t][i];
+                } else {
+                    if (row < rows) y[(long)row * N + li] = acc[t][i];
+                }
             }
     }
 }
 
-template <int UPW, int N>
+template <int UPW, int N, bool TM>
 static void launch_iq4t(dim3 g, hipStream_t st, const uint4* wt, const uint16_t* sc, const uint16_t* x, float* y,
-                        float* ws, int M, int K, int nch) {
+                        float* ws, int M, int K, int nch, int T) {
     constexpr int W = 4;
     const size_t lds = (size_t)mfma_chunk_xbytes(128 * UPW, N) + 16 + 2048 + (size_t)2 * W * UPW * 64 * 2;
-    iq4nlt_mfma_kernel<UPW, W, N><<<g, W * 64, lds, st>>>(wt, sc, x, M, K, nch, (int)g.x, (int)g.y, y, ws);
+    iq4nlt_mfma_kernel<UPW, W, N, TM><<<g, W * 64, lds, st>>>(wt, sc, x, M, K, nch, (int)g.x, (int)g.y, T, y, ws);
 }
 
-template <int N>
+template <int N, bool TM>
 static void launch_iq4t_n(int upw, int nch, dim3 g, hipStream_t st, const uint4* wt, const uint16_t* sc,
-                          const uint16_t* x, float* y, float* ws, int M, int K) {
+                          const uint16_t* x, float* y, float* ws, int M, int K, int T) {
     if (upw == 4)
-        launch_iq4t<4, N>(g, st, wt, sc, x, y, ws, M, K, nch);
+        launch_iq4t<4, N, TM>(g, st, wt, sc, x, y, ws, M, K, nch, T);
     else
-        launch_iq4t<2, N>(g, st, wt, sc, x, y, ws, M, K, nch);
+        launch_iq4t<2, N, TM>(g, st, wt, sc, x, y, ws, M, K, nch, T);
+}
+
+template <bool TM>
+static void launch_iq4t_any(int upw, int nch, dim3 g, hipStream_t st, const uint4* wt, const uint16_t* sc,
+                            const uint16_t* x, float* y, float* ws, int M, int K, int N, int T) {
+    switch (N) {
+        case 4: launch_iq4t_n<4, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
+        case 8: launch_iq4t_n<8, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
+        case 12: launch_iq4t_n<12, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
+        default: launch_iq4t_n<16, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
+    }
 }
 
 // Grid of the tiled IQ4_NL GEMM: 128 rows a workgroup and the largest K
@@ -1814,8 +1848,9 @@ ZT_EXPORT long zt_gemm_iq4nlt_workspace_bytes(int M, int K, int N) {
     return tiled_ws_bytes(M, (int)iq4t_grid(M, K, upw, nch).y);
 }
 
-ZT_EXPORT int zt_gemm_iq4nlt_f16(const void* W_tiled, const void* S_tiled, const uint16_t* B, float* C, int M, int K,
-                                 int N, void* workspace, long workspace_bytes, hipStream_t stream) {
+// tokens > 0: B[tokens][K] and C[tokens][M], N = tokens up to a multiple of 4
+static int gemm_iq4nlt(const void* W_tiled, const void* S_tiled, const uint16_t* B, float* C, int M, int K, int N,
+                       int tokens, void* workspace, long workspace_bytes, hipStream_t stream) {
     if (M < 0 || K < 0 || K % 128 != 0) return (int)hipErrorInvalidValue;
     if (N != 4 && N != 8 && N != 12 && N != 16) return (int)hipErrorInvalidValue;
     if (M == 0 || K == 0) return (int)hipSuccess;
@@ -1831,12 +1866,21 @@ ZT_EXPORT int zt_gemm_iq4nlt_f16(const void* W_tiled, const void* S_tiled, const
     const uint4* wt = static_cast<const uint4*>(W_tiled);
     const uint16_t* sc = static_cast<const uint16_t*>(S_tiled);
     float* ws = static_cast<float*>(workspace);
-    switch (N) {
-        case 4: launch_iq4t_n<4>(upw, nch, g, stream, wt, sc, B, C, ws, M, K); break;
-        case 8: launch_iq4t_n<8>(upw, nch, g, stream, wt, sc, B, C, ws, M, K); break;
-        case 12: launch_iq4t_n<12>(upw, nch, g, stream, wt, sc, B, C, ws, M, K); break;
-        default: launch_iq4t_n<16>(upw, nch, g, stream, wt, sc, B, C, ws, M, K); break;
-    }
-    if (g.y > 1) tiled_reduce(workspace, C, M, N, (int)g.y, stream);
+    if (tokens > 0)
+        launch_iq4t_any<true>(upw, nch, g, stream, wt, sc, B, C, ws, M, K, N, tokens);
+    else
+        launch_iq4t_any<false>(upw, nch, g, stream, wt, sc, B, C, ws, M, K, N, tokens);
+    if (g.y > 1) tiled_reduce(workspace, C, M, N, (int)g.y, stream, tokens);
     return (int)hipGetLastError();
+}
+
+ZT_EXPORT int zt_gemm_iq4nlt_f16(const void* W_tiled, const void* S_tiled, const uint16_t* B, float* C, int M, int K,
+                                 int N, void* workspace, long workspace_bytes, hipStream_t stream) {
+    return gemm_iq4nlt(W_tiled, S_tiled, B, C, M, K, N, 0, workspace, workspace_bytes, stream);
+}
+
+ZT_EXPORT int zt_gemm_iq4nlt_tokens_f16(const void* W_tiled, const void* S_tiled, const uint16_t* X, float* C, int M,
+                                        int K, int T, void* workspace, long workspace_bytes, hipStream_t stream) {
+    if (T < 1 || T > 16 || K >= 1 << 26) return (int)hipErrorInvalidValue;
+    return gemm_iq4nlt(W_tiled, S_tiled, X, C, M, K, (T + 3) & ~3, T, workspace, workspace_bytes, stream);
 }

@@ -1091,6 +1091,12 @@ __global__ void w4t_sz_kernel(const uint16_t* __restrict__ scales, const uint16_
     sz[e] = (uint32_t)s | ((uint32_t)z << 16);
 }
 
+// 8 halves in the A operand's order of a dword's nibbles: e0 e4 e1 e5 e2 e6 e3 e7
+__device__ __forceinline__ u32x4 nibble_order(const u32x4& o) {
+    return (u32x4){__builtin_amdgcn_perm(o[2], o[0], 0x05040100u), __builtin_amdgcn_perm(o[2], o[0], 0x07060302u),
+                   __builtin_amdgcn_perm(o[3], o[1], 0x05040100u), __builtin_amdgcn_perm(o[3], o[1], 0x07060302u)};
+}
+
 // Small-batch W4A16 GEMM on the tiled layout (N in {4, 8, 12, 16}, K % 128 == 0,
 // group size % 128 == 0).  A workgroup of W waves owns 32 W rows (two 16-row
 // tiles a wave) and a K range of UPW 128-K units; K ranges are split across
@@ -1112,17 +1118,17 @@ __global__ void w4t_sz_kernel(const uint16_t* __restrict__ scales, const uint16_
 //  * Workgroups are mapped XCD-aware: workgroup id mod 8 selects the XCD,
 //    and every K range of a row block runs on one XCD, whose L2 then holds
 //    the row block's scale lines.
-template <int UPW, int W, int N>
+template <int UPW, int W, int N, bool TM>
 __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __restrict__ wt,
                                                              const uint32_t* __restrict__ szp,
                                                              const uint16_t* __restrict__ x, int rows, int K, int gs,
-                                                             int nch, int gx, int gy, float* __restrict__ y,
+                                                             int nch, int gx, int gy, int T, float* __restrict__ y,
                                                              float* __restrict__ ws) {
     constexpr int KC = 128 * UPW;
     constexpr int RW = 32 * W;
     constexpr int XP = (KC * 2 * N / 16 + W * 64 - 1) / (W * 64);
     constexpr int SP = (UPW * RW + W * 64 - 1) / (W * 64);
-    constexpr int XB = mfma_chunk_xbytes(KC, N);
+    constexpr int XB = TM ? KC * 2 * N : mfma_chunk_xbytes(KC, N);
     extern __shared__ __attribute__((aligned(16))) char smem[];
     char* zero_area = smem + XB;
     float2* szs = reinterpret_cast<float2*>(zero_area + 16);
@@ -1151,7 +1157,15 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
     if (ch > 0) asm volatile("s_barrier" ::: "memory");  // every wave is done with the previous chunk's LDS
     const int npieces = (u1 - u0) * 128 * 2 * N / 16;
     const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)u0 * 128 * N), (short)0, npieces * 16, 0x00020000);
+        TM ? __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, T * K * 2, 0x00020000)
+           : __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)u0 * 128 * N), (short)0, npieces * 16, 0x00020000);
+    // the 16 bytes that slot e of the staged chunk holds; past the tokens or
+    // the chunk's units nothing uses them (an offset past the buffer loads zeros)
+    auto xoff = [&](int e) -> uint32_t {
+        if constexpr (!TM) return (uint32_t)e * 16u;
+        const int t = e / (KC / 8), pos = e % (KC / 8), c = (pos & ~15) | ((pos ^ t) & 15);
+        return t < T && c < 16 * (u1 - u0) ? (uint32_t)t * (uint32_t)K * 2u + (uint32_t)(u0 * 256 + c * 16) : 0x80000000u;
+    };
     const __amdgpu_buffer_rsrc_t rsz = __builtin_amdgcn_make_buffer_rsrc((void*)szp, (short)0, 0x7fffffff, 0x00020000);
     // N = 16: a wave's 64 pieces of 16 bytes are one padded 32-row segment
     // (64 N bytes), so they go to LDS directly (buffer_load ... lds, the
@@ -1163,11 +1177,12 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
     for (int i = 0; i < XP; i++) {
         if constexpr (XDMA) {
             const int c = wave + i * W;  // segment of this wave's pieces
+            const uint32_t off = xoff(tid + i * W * 64);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rx, (__attribute__((address_space(3))) void*)(smem + c * 68 * N), 16,
-                (uint32_t)(tid + i * W * 64) * 16u, 0, 0, 0);
+                rx, (__attribute__((address_space(3))) void*)(smem + c * (TM ? 1024 : 68 * N)), 16,
+                off, 0, 0, 0);
         } else {
-            xr[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, (uint32_t)(tid + i * W * 64) * 16u, 0, 0);
+            xr[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff(tid + i * W * 64), 0, 0);
         }
     }
     uint32_t sr[SP];
@@ -1197,7 +1212,9 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
 #pragma unroll
     for (int i = 0; i < XP; i++) {
         const int p = tid + i * W * 64;
-        if (!XDMA && p < npieces) {
+        if constexpr (TM && !XDMA) {
+            if (p < N * (KC / 8)) *reinterpret_cast<u32x4*>(smem + p * 16) = nibble_order(xr[i]);
+        } else if (!XDMA && p < npieces) {
             const int off = p * 16;
             *reinterpret_cast<u32x4*>(smem + off + (off / (64 * N)) * (4 * N)) = xr[i];
         }
@@ -1222,6 +1239,10 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
     // step s of unit u reads X rows 128u + 32lg + 8s + offa (+ 2), whose
     // padded LDS offset is (34lg + offa) 2N + (136u + 8s) 2N
     const int lbase = (34 * lg + offa) * 2 * N + 8 * (li & 3);
+    // token-major: piece 16u + 4 lg + s of token li (columns >= N repeat the last)
+    int pb[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) pb[s] = token_slot(min(li, N - 1), 4 * lg + s, KC);
 #pragma unroll
     for (int u = 0; u < UPW; u++) {
         if (u0 + u < u1) {
@@ -1229,7 +1250,13 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
             d[0] = d[1] = (float4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                const half8v bv = mfma_b_pair(smem, lbase + (136 * u + 8 * s) * 2 * N, 4 * N);
+                half8v bv;
+                if constexpr (TM) {
+                    const u32x4 o = *reinterpret_cast<const u32x4*>(smem + pb[s] + 256 * u);
+                    bv = __builtin_bit_cast(half8v, XDMA ? nibble_order(o) : o);
+                } else {
+                    bv = mfma_b_pair(smem, lbase + (136 * u + 8 * s) * 2 * N, 4 * N);
+                }
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
                     const uint32_t dw = s == 0 ? w[u][t].x : s == 1 ? w[u][t].y : s == 2 ? w[u][t].z : w[u][t].w;
@@ -1263,28 +1290,43 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = row0 + 16 * t + 4 * lg + i;
-                if (row < rows) y[(long)row * N + li] = acc[t][i];
+                if constexpr (TM) {
+                    if (row < rows && li < T) y[(long)li * rows + row] = acc[t][i];
+                } else {
+                    if (row < rows) y[(long)row * N + li] = acc[t][i];
+                }
             }
     }
 }
 
-template <int UPW, int N>
+template <int UPW, int N, bool TM>
 static void launch_w4t(dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz, const uint16_t* x, float* y,
-                       float* ws, int M, int K, int gs, int nch) {
+                       float* ws, int M, int K, int gs, int nch, int T) {
     constexpr int W = 4;
     const size_t lds = (size_t)mfma_chunk_xbytes(128 * UPW, N) + 16 + 8 * UPW * 32 * W;
-    w4a16t_mfma_kernel<UPW, W, N><<<g, W * 64, lds, st>>>(wt, sz, x, M, K, gs, nch, (int)g.x, (int)g.y, y, ws);
+    w4a16t_mfma_kernel<UPW, W, N, TM><<<g, W * 64, lds, st>>>(wt, sz, x, M, K, gs, nch, (int)g.x, (int)g.y, T, y, ws);
 }
 
-template <int N>
+template <int N, bool TM>
 static void launch_w4t_n(int upw, int nch, dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz,
-                         const uint16_t* x, float* y, float* ws, int M, int K, int gs) {
+                         const uint16_t* x, float* y, float* ws, int M, int K, int gs, int T) {
     if (upw == 8)
-        launch_w4t<8, N>(g, st, wt, sz, x, y, ws, M, K, gs, nch);
+        launch_w4t<8, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
     else if (upw == 4)
-        launch_w4t<4, N>(g, st, wt, sz, x, y, ws, M, K, gs, nch);
+        launch_w4t<4, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
     else
-        launch_w4t<2, N>(g, st, wt, sz, x, y, ws, M, K, gs, nch);
+        launch_w4t<2, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
+}
+
+template <bool TM>
+static void launch_w4t_any(int upw, int nch, dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz,
+                           const uint16_t* x, float* y, float* ws, int M, int K, int N, int gs, int T) {
+    switch (N) {
+        case 4: launch_w4t_n<4, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
+        case 8: launch_w4t_n<8, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
+        case 12: launch_w4t_n<12, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
+        default: launch_w4t_n<16, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
+    }
 }
 
 // Grid of the tiled W4A16 GEMM: 128 rows a workgroup, and a K range of 8, 4
@@ -1342,8 +1384,9 @@ ZT_EXPORT long zt_gemm_w4a16t_workspace_bytes(int M, int K, int N) {
     return tiled_ws_bytes(M, (int)w4t_grid(M, K, upw, nch).y);
 }
 
-ZT_EXPORT int zt_gemm_w4a16t_f32(const void* W_tiled, const uint32_t* sz, const uint16_t* B, float* C, int M, int K,
-                                 int N, int group_size, void* workspace, long workspace_bytes, hipStream_t stream) {
+// tokens > 0: B[tokens][K] and C[tokens][M], N = tokens up to a multiple of 4
+static int gemm_w4a16t(const void* W_tiled, const uint32_t* sz, const uint16_t* B, float* C, int M, int K, int N,
+                       int tokens, int group_size, void* workspace, long workspace_bytes, hipStream_t stream) {
     if (M < 0 || K < 0 || K % 128 != 0 || group_size <= 0 || group_size % 128 != 0 || K % group_size != 0)
         return (int)hipErrorInvalidValue;
     if (N != 4 && N != 8 && N != 12 && N != 16) return (int)hipErrorInvalidValue;
@@ -1359,12 +1402,22 @@ ZT_EXPORT int zt_gemm_w4a16t_f32(const void* W_tiled, const uint32_t* sz, const 
         return (int)hipErrorInvalidValue;
     const uint4* wt = static_cast<const uint4*>(W_tiled);
     float* ws = static_cast<float*>(workspace);
-    switch (N) {
-        case 4: launch_w4t_n<4>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, group_size); break;
-        case 8: launch_w4t_n<8>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, group_size); break;
-        case 12: launch_w4t_n<12>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, group_size); break;
-        default: launch_w4t_n<16>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, group_size); break;
-    }
-    if (g.y > 1) tiled_reduce(workspace, C, M, N, (int)g.y, stream);
+    if (tokens > 0)
+        launch_w4t_any<true>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, N, group_size, tokens);
+    else
+        launch_w4t_any<false>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, N, group_size, tokens);
+    if (g.y > 1) tiled_reduce(workspace, C, M, N, (int)g.y, stream, tokens);
     return (int)hipGetLastError();
+}
+
+ZT_EXPORT int zt_gemm_w4a16t_f32(const void* W_tiled, const uint32_t* sz, const uint16_t* B, float* C, int M, int K,
+                                 int N, int group_size, void* workspace, long workspace_bytes, hipStream_t stream) {
+    return gemm_w4a16t(W_tiled, sz, B, C, M, K, N, 0, group_size, workspace, workspace_bytes, stream);
+}
+
+ZT_EXPORT int zt_gemm_w4a16t_tokens_f32(const void* W_tiled, const uint32_t* sz, const uint16_t* X, float* C, int M,
+                                        int K, int T, int group_size, void* workspace, long workspace_bytes,
+                                        hipStream_t stream) {
+    if (T < 1 || T > 16 || K >= 1 << 26) return (int)hipErrorInvalidValue;
+    return gemm_w4a16t(W_tiled, sz, X, C, M, K, (T + 3) & ~3, T, group_size, workspace, workspace_bytes, stream);
 }

@@ -277,8 +277,12 @@ class ROCmEngine:
             if a.shape[-1] != k:
                 raise ValueError(f"matmul: A has {a.shape[-1]} columns but B is [{k},{nout}]")
             m = a.numel() // k
-            if _wide_tokens(m) or _few_tokens(b.storage, nout, k, m):
-                ct = self._wide_times(b.storage, nout, k, a.reshape(m, k))
+            if m > 1:
+                x, ct = a.reshape(m, k), None
+                if _wide_tokens(m) or _few_tokens(b.storage, nout, k, x):
+                    ct = self._wide_times(b.storage, nout, k, x)
+                if ct is None and m <= 16:
+                    ct = self._tiled_tokens(b.storage, nout, k, x)
                 if ct is not None:
                     return ct.reshape(*a.shape[:-1], nout)
             if m == 1:  # a vector is its own transpose
@@ -340,6 +344,72 @@ class ROCmEngine:
         c = torch.empty((t, rows), dtype=torch.float32, device=self.device)
         self.lib.call("zt_gemm_wide_f32", fmt, _p(w), o1, o2, szr, group, _p(x), int(half), _p(c), rows, k, t, _p(ws),
                       nbytes, self._s)
+        return c
+
+    def _tiled_tokens(self, s: Any, rows: int, k: int, x: torch.Tensor) -> torch.Tensor | None:
+        """x[t, k] @ dequant(W)[rows, k]^T -> fp32 [t, rows] for 2 to 16 tokens
+        on the tiled copy, the token-major form of the tiled GEMMs: no
+        transposes and no padding around the call.  None for a type or size
+        that has no tiled copy; and where columns run without one (the
+        row-block GEMMs, padded counts of a mapped file), unless it is there or can be made at no risk: with
+        memory to spare, and not while a graph is captured, whose pool the
+        copy would be left in."""
+        t = x.shape[0]
+        n = -(-t // 4) * 4
+        mm = s.qtype if isinstance(s, MmapStorage) else None
+        half = x.dtype == torch.float16
+        if x.device != self.device or k % 128 != 0:
+            return None
+        rowblock = False
+        if isinstance(s, (GPTQStorage, AWQStorage)):
+            if not half or s.group_size % 128 != 0 or rows * (k // s.group_size) >= 1 << 29:
+                return None
+            f, rowblock = "w4a16", _w4a16_rowblock(rows, k, n)
+        elif isinstance(s, IQ4NLStorage):
+            if not half:
+                return None
+            f, rowblock = "iq4nl", k <= 8192 and (n <= 8 or rows <= 4096)
+        elif half and isinstance(s, Q4Storage):
+            x = x.float()  # exact
+            f, rowblock = "q4", _block_rowblock("q4", rows, k, n)
+        else:
+            f = _TILED_MMAP.get(mm) if mm is not None else _TILED_STORAGE.get(type(s))
+            if f is None or x.dtype != torch.float32 or (f in ("q4k", "q5k", "q6k") and k % 256 != 0):
+                return None
+            rowblock = f in ("q4", "q8", "q8gguf") and _block_rowblock(f[:2], rows, k, n)
+        if getattr(s, "_gpu", None) is None:
+            self.upload_weights([s])
+        buf = s.gpu_ptr()
+        if ((rowblock or (mm is not None and t != n)) and _tiled_cached(s, (f + "t", rows, k, _p(buf.tensor))) is None
+                and (torch.cuda.is_current_stream_capturing()
+                     or torch.cuda.mem_get_info(self.device)[0] < 2 * rows * k + self.split_reserve_bytes)):
+            return None
+        x = x.contiguous()
+        x = x if _p(x) % 16 == 0 else x.clone()
+        c = torch.empty((t, rows), dtype=torch.float32, device=self.device)
+        if f == "w4a16":
+            wt, sz = self._w4a16_tiled(s, rows, k)
+            ws, wsb = self._workspace(self.lib.zt_gemm_w4a16t_workspace_bytes(rows, k, n))
+            self.lib.call("zt_gemm_w4a16t_tokens_f32", _p(wt), _p(sz), _p(x), _p(c), rows, k, t, s.group_size, ws, wsb,
+                          self._s)
+            return c
+        if f == "iq4nl":
+            wt, st = self._iq4nl_tiled(s, buf, rows, k)
+            ws, wsb = self._workspace(self.lib.zt_gemm_iq4nlt_workspace_bytes(rows, k, n))
+            self.lib.call("zt_gemm_iq4nlt_tokens_f16", _p(wt), _p(st), _p(x), _p(c), rows, k, t, ws, wsb, self._s)
+            return c
+        if f in ("q4", "q8", "q8gguf"):
+            bufs = self._block_tiled(s, buf, rows, k, f)
+        elif f == "q5_0":
+            o = (s.gpu_qh_offset(), s.gpu_qs_offset()) if mm is None else (s._gpu_offsets["qh_offset"],
+                                                                           s._gpu_offsets["qs_offset"])
+            bufs = self._q5_0_tiled(s, buf, rows, k, *o)
+        else:
+            bufs = self._kq_tiled(s, buf, rows, k, f)
+        size_fmt = "q8" if f == "q8gguf" else f
+        ws, wsb = self._workspace(getattr(self.lib, f"zt_gemm_{size_fmt}t_workspace_bytes")(rows, k, n))
+        self.lib.call("zt_gemm_blkt_tokens_f32", _TILED_FORMATS[f], _p(bufs[0]), _p(bufs[1]),
+                      _p(bufs[2]) if len(bufs) > 2 else 0, _p(x), _p(c), rows, k, t, ws, wsb, self._s)
         return c
 
     def _w4a16_tiled(self, s: Any, rows: int, k: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -683,7 +753,7 @@ class ROCmEngine:
             ws, wsb = self._workspace(self.lib.zt_gemm_q4t_workspace_bytes(rows, k, n))
             self.lib.call("zt_gemm_q4t_f32", _p(wt), _p(st), _p(x), _p(c), rows, k, n, ws, wsb, self._s)
         elif q in (GGMLType.Q4_K, GGMLType.Q5_K, GGMLType.Q6_K) and tiled and k % 256 == 0:
-            self._kq_tiled_gemm(s, buf, rows, k, x, n, c, {GGMLType.Q4_K: "q4k", GGMLType.Q5_K: "q5k"}.get(q, "q6k"))
+            self._kq_tiled_gemm(s, buf, rows, k, x, n, c, _TILED_MMAP[q])
         elif q == GGMLType.Q8_0 and tiled and k % 128 == 0:
             wt, st = self._block_tiled(s, buf, rows, k, "q8gguf")
             ws, wsb = self._workspace(self.lib.zt_gemm_q8t_workspace_bytes(rows, k, n))
@@ -911,29 +981,34 @@ def _wide_tokens(t: int, transposed: bool = False) -> bool:
     return t > (32 if transposed else 16)
 
 
-def _few_tokens(s: Any, rows: int, k: int, t: int) -> bool:
-    """Whether 2 to 16 tokens go to the token-major GEMM too, which spares
-    the two transposes (about 4 us each) and, for counts that are no multiple
-    of 4, the padding (five small launches).  W4A16 and IQ4_NL (one launch
-    without packing, for fp16 activations): while the matrix is small enough
-    that this weighs more than the tiled layout gives, and every padded count
-    (W4A16, 8 tokens 8192 x 8192 14.7 us against 13.2 + 7.3, 28672 x 8192 41
-    against 29 + 8, 16 tokens 4096 x 4096 6.4 against 6.4 + 7; IQ4_NL, 8 tokens
-    3584 x 3584 7.5 against 7.9 + 7.4, 18944 x 3584 23.9 against 19.4 + 8.6).
-    The formats that pack fp32 activations first: padded counts of small
-    matrices (a layer of 2048 x 5632 matrices, Q4_0, 2 tokens 107 -> 76 us;
-    Llama-3-8B's, whose MLP matrices stay tiled here, would go from 157 to
-    150 in Q4_0 at 6 tokens but from 162 to 193 in Q4_K / Q6_K at 3)."""
-    if not 2 <= t <= 16:
+def _few_tokens(s: Any, rows: int, k: int, x: torch.Tensor) -> bool:
+    """Whether 2 to 16 tokens x[t, k] go to the token-major GEMM on the upload
+    layout before the tiled copy's is tried.  fp16 tokens (one launch, against
+    a GEMM and the sum of its K ranges): while K is short enough for one
+    workgroup's walk and the matrix small (us, against the tiled copy: W4A16
+    4096 x 4096 6.0 / 7.0, 8192 x 4096 8.1 / 8.6, 2048 x 8192 9.1 / 6.8, 14336
+    x 4096 14.4 / 12.9; IQ4_NL 8192 x 2048 8.5 / 9.0, 6144 x 4096 11.4 / 10.4),
+    and past 8 tokens up to 4096 rows (more have a tiled copy from the
+    columns).  fp32 tokens on IQ4_NL, which has no other kernel of that shape:
+    the counts the column kernel is slow at (14336 x 4096, us against it: 3
+    tokens 27 / 63, 4 28 / 21, 8 28 / 31, 16 28 / 56)."""
+    t = x.shape[0]
+    if not 2 <= t <= 16 or not isinstance(s, (GPTQStorage, AWQStorage, IQ4NLStorage)):
         return False
-    if isinstance(s, (GPTQStorage, AWQStorage, IQ4NLStorage)):
-        # 12 and 16 tokens past 4096 rows have a tiled copy of their own
-        return t % 4 != 0 or (rows * k <= 1 << 27 and (t <= 8 or rows <= 4096))
-    return t % 4 != 0 and rows * k <= 1 << 24 and k <= 4096
+    if x.dtype != torch.float16:
+        return isinstance(s, IQ4NLStorage) and (t % 4 != 0 or t > 8)
+    return (k <= 4096 and rows * k <= 1 << (24 if isinstance(s, IQ4NLStorage) else 25)
+            and (t <= 8 or rows <= 4096))
 
 
 # zt_gemm_wide_f32 formats (ZT_WIDE_*)
 _WIDE = {"w4a16": 0, "q4_0": 1, "q8_0": 2, "q8_gguf": 3, "q5_0": 4, "q4_k": 5, "q5_k": 6, "q6_k": 7, "iq4_nl": 8}
+# tiled copies: the ZT_WIDE_* format of each, and whose they are
+_TILED_FORMATS = {"q4": 1, "q8": 2, "q8gguf": 3, "q5_0": 4, "q4k": 5, "q5k": 6, "q6k": 7}
+_TILED_STORAGE = {Q4Storage: "q4", Q8Storage: "q8", Q5_0Storage: "q5_0", Q4KStorage: "q4k", Q5KStorage: "q5k",
+                  Q6KStorage: "q6k"}
+_TILED_MMAP = {GGMLType.Q4_0: "q4", GGMLType.Q8_0: "q8gguf", GGMLType.Q5_0: "q5_0", GGMLType.Q4_K: "q4k",
+               GGMLType.Q5_K: "q5k", GGMLType.Q6_K: "q6k"}
 _WIDE_STORAGE = {Q8Storage: 2, Q5_0Storage: 4, Q4KStorage: 5, Q5KStorage: 6, Q6KStorage: 7}
 _WIDE_MMAP = {GGMLType.Q8_0: 3, GGMLType.Q5_0: 4, GGMLType.Q4_K: 5, GGMLType.Q5_K: 6, GGMLType.Q6_K: 7}
 
