@@ -157,8 +157,25 @@ def test_tiled_tokens_are_the_columns(eng, orc, monkeypatch, fmt, rows, K):
         assert torch.equal(eng._tiled_tokens(s, rows, K, x.t().contiguous().t()), y)
 
 
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q5_0", "q4_k", "q5_k", "q6_k", "mmap_q8_0", "mmap_q4_k"])
+@pytest.mark.parametrize("rows,K", [(1, 256), (37, 768), (130, 1280), (2060, 3328)])
+def test_tiled_tokens_to_32(eng, orc, fmt, rows, K):
+    """Two column tiles: partial and whole second tiles, one and several K ranges, ragged rows; tokens of very
+    different sizes share a K range's power-of-two scale, whose absolute floor is 2^-39 of the largest value."""
+    s, w = weights(fmt, rows, K, rows + K, orc)
+    for T in (17, 18, 31, 32):
+        x = activations(fmt, T, K, T)
+        x[T - 1] *= 30.0
+        y = eng._tiled_tokens(s, rows, K, torch.from_numpy(x).cuda()).cpu().numpy()
+        assert y.shape == (T, rows)
+        floor = 2.0**-38 * np.abs(x).max() * np.abs(w).sum(axis=1)
+        bound = (K / 32 + 24) * 2.0**-24 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + floor
+        assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound), T
+        check(eng._wide_times(s, rows, K, torch.from_numpy(x).cuda()).cpu().numpy(), x, w)  # the other way
+
+
 @pytest.mark.parametrize("fmt,rows,K,T", [("gptq", 100, 8192, 5), ("q4_0", 100, 512, 4), ("q8_0", 300, 1024, 3),
-                                          ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6),
+                                          ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6), ("q4_k", 64, 512, 20),
                                           ("iq4_nl_f16", 64, 5120, 8)])
 def test_tiled_tokens_build_a_copy_only_at_no_risk(eng, orc, fmt, rows, K, T):
     """Where the columns need no tiled copy the tokens make one, but neither in a capture nor at the memory limit;
@@ -190,13 +207,18 @@ def test_tiled_tokens_build_a_copy_only_at_no_risk(eng, orc, fmt, rows, K, T):
 def test_tiled_tokens_entry_point_errors(eng):
     lib, p = eng.lib, 1 << 20
     for t in (0, 17):
-        assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p, p, 16, 128, t, 0, 0, 0) == 1
+        assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p, p, 16, 128, t and 33, 0, 0, 0) == 1
+        assert lib.zt_gemm_blkt_tokens_workspace_bytes(1, 16, 128, t and 33) == -1
         assert lib.zt_gemm_w4a16t_tokens_f32(p, p, p, p, 16, 128, t, 128, 0, 0, 0) == 1
         assert lib.zt_gemm_iq4nlt_tokens_f16(p, p, p, p, 16, 128, t, 0, 0, 0) == 1
     assert lib.zt_gemm_blkt_tokens_f32(0, p, p, 0, p, p, 16, 128, 4, 0, 0, 0) == 1  # W4A16 and IQ4_NL have their own
     assert lib.zt_gemm_blkt_tokens_f32(4, p, p, 0, p, p, 16, 128, 4, 0, 0, 0) == 1  # no fifth bits
     assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p + 4, p, 16, 128, 4, 0, 0, 0) == 1  # X alignment
-    assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p, p, 16, 1 << 25, 4, 0, 0, 0) == 1
+    assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p, p, 16, 1 << 24, 4, 0, 0, 0) == 1
+    # 32 tokens: two column tiles of partials
+    one, two = lib.zt_gemm_q8t_workspace_bytes(4096, 4096, 16), lib.zt_gemm_blkt_tokens_workspace_bytes(2, 4096, 4096, 17)
+    assert two == 2 * one > 0 and lib.zt_gemm_blkt_tokens_workspace_bytes(2, 4096, 4096, 16) == one
+    assert lib.zt_gemm_blkt_tokens_f32(2, p, p, 0, p, p, 4096, 4096, 17, p, two - 1, 0) == 1
     assert lib.zt_gemm_w4a16t_tokens_f32(p, p, p, p, 16, 1 << 26, 4, 128, 0, 0, 0) == 1
 
 

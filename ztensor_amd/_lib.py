@@ -104,6 +104,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "zt_q6k_tile": (I, [P, I, I, P, P, P]),
     "zt_gemm_q6kt_workspace_bytes": (L, [I, I, I]),
     "zt_gemm_q6kt_f32": (I, [P, P, P, P, I, I, I, P, L, P]),
+    "zt_gemm_blkt_tokens_workspace_bytes": (L, [I, I, I, I]),
     "zt_gemm_blkt_tokens_f32": (I, [I, P, P, P, P, P, I, I, I, P, L, P]),
     "zt_ternary_gemv_f32": (I, [P, P, P, I, I, P]),
     "zt_ternary_gemv_i8": (I, [P, P, P, P, P, I, I, P]),

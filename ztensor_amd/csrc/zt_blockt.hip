@@ -274,6 +274,12 @@ __device__ constexpr int blkt_token_slot(int c) {
     return (c & 1) * 4 + ((c & 3) >> 1) + ((c >> 2) << 1);
 }
 
+// TM: token-major activations (zt_mfma.h), there also 17 to 32 tokens: two
+// column tiles against each decoded A operand (us, 20 tokens, against the wide
+// GEMM on the upload layout: Q8_0 4096 x 14336 25.6 / 44.6, Q4_K 28672 x 8192
+// 80 / 109).  With wmax apart from the scales the K-quants' 80 KB of LDS left
+// one workgroup a CU: Q4_K 28672 x 8192 108 against 80, 4096 x 14336 32.7
+// against 25.7.
 template <BlkFmt F, int UPW, int N, bool TM>
 __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict__ wt, const void* __restrict__ stl,
                                                         const uint32_t* __restrict__ aux, const float* __restrict__ x,
@@ -283,7 +289,8 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
     constexpr int KC = 128 * UPW;
     constexpr int RW = 32 * W;
     constexpr int NPL = N <= 8 ? 1 : 2;                 // staged fp16 planes (hi/lo in columns, or two planes)
-    constexpr int XPB = TM ? KC * 32 : mfma_chunk_xbytes(KC, 16);  // one plane: 16 fp16 columns, 2 pad rows per 32
+    constexpr int NCT = N > 16 ? 2 : 1;                 // 16-column tiles (32 tokens: token-major only)
+    constexpr int XPB = TM ? KC * 32 * NCT : mfma_chunk_xbytes(KC, 16);  // one plane: 16 fp16 columns, 2 pad rows per 32
     constexpr int PPR = N / 4;                          // 16-byte pieces per fp32 activation row
     // loads a thread: single 16-byte pieces, token-major in pairs (the 8 values of one LDS piece)
     constexpr int XP = TM ? 2 * ((KC / 8 * N + W * 64 - 1) / (W * 64)) : (KC * PPR + W * 64 - 1) / (W * 64);
@@ -298,7 +305,9 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
     constexpr int WL = (F == BlkFmt::Q8_0 || F == BlkFmt::Q6_K) ? 2 : 1;  // 16-byte weight loads per lane per tile-unit
     extern __shared__ __attribute__((aligned(16))) char smem[];
     float* wmax = reinterpret_cast<float*>(smem + NPL * XPB);  // per-wave max |x|
-    char* ssm = smem + NPL * XPB + 16;                            // block scales
+    // block scales, after wmax; over it with 32 tokens, so that two workgroups
+    // of the K-quants (80 KB each) fit a CU
+    char* ssm = smem + NPL * XPB + (NCT == 2 ? 0 : 16);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, lg = lane >> 4;
     const int nunits = K / 128;
@@ -384,6 +393,7 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
     if (lane == 0) wmax[wave] = m;
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    if constexpr (NCT == 2) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // read by every wave
     int sh = 0;
     if (m > 0.0f && m <= 3.402823466e38f) {
         int e2;
@@ -497,8 +507,9 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
     uint32_t nmask = Q5 ? 0x01E001E0u : 0x03C003C0u,
              nexp = (Q5 || Q6 || F == BlkFmt::Q8_0) ? 0x78007800u : 0x74007400u;
     asm volatile("" : "+v"(nmask), "+s"(nexp));
-    float4v acc[2];
-    acc[0] = acc[1] = (float4v){0.f, 0.f, 0.f, 0.f};
+    float4v acc[NCT][2];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++) acc[ct][0] = acc[ct][1] = (float4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < UPW; u++) {
         if (u0 + u < u1) {
@@ -515,12 +526,14 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
                     for (int h = 0; h < SVR; h++)
                         sc[t][i][h] = reinterpret_cast<const SV*>(ssm)[(((2 * wave + t) * UPW + u) * 16 + 4 * lg + i) * SVR + h];
 #pragma unroll
-            for (int s = 0; s < 4; s++) {
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int ct = 0; ct < NCT; ct++) {
                 half8v bv[NPL];
 #pragma unroll
                 for (int pl = 0; pl < NPL; pl++) {
                     if constexpr (TM) {
-                        bv[pl] = *reinterpret_cast<const half8v*>(smem + pb[s] + pl * XPB + 256 * u);
+                        bv[pl] = *reinterpret_cast<const half8v*>(smem + pb[s] + ct * (32 * KC) + pl * XPB + 256 * u);
                         continue;
                     }
                     const int o = pl * XPB + (136 * u + 8 * s) * 32;
@@ -567,7 +580,7 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
                         for (int i = 0; i < 4; i++) {
                             const SV& pr = sc[t][i][s >> 1];  // groups 2s, 2s+1
                             const float s0 = (s & 1) ? pr.z : pr.x, s1 = (s & 1) ? pr.w : pr.y;
-                            acc[t][i] = fmaf(s0, d[0][i], fmaf(s1, d[1][i], acc[t][i]));
+                            acc[ct][t][i] = fmaf(s0, d[0][i], fmaf(s1, d[1][i], acc[ct][t][i]));
                         }
                     }
                     continue;
@@ -619,8 +632,8 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
                             // 2^10 (d sc sum(q x) - dmin mn sum(x)) = sv D + (mv 2^-4) dn
                             const SV& pr = sc[t][i][s >> 1];
                             const float sv = (s & 1) ? pr.z : pr.x, mv = (s & 1) ? pr.w : pr.y;
-                            acc[t][i] = fmaf(sv, d[i], fmaf(mv * (F == BlkFmt::Q5_K ? 0.03125f : 0.0625f), dn[i],
-                                                            acc[t][i]));
+                            acc[ct][t][i] = fmaf(sv, d[i], fmaf(mv * (F == BlkFmt::Q5_K ? 0.03125f : 0.0625f), dn[i],
+                                                            acc[ct][t][i]));
                         } else {
                             float sv;
                             if constexpr (F == BlkFmt::Q4_0 || F == BlkFmt::Q5_0) {  // fp16 scales
@@ -629,7 +642,7 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
                             } else {
                                 sv = s == 0 ? sc[t][i][0].x : s == 1 ? sc[t][i][0].y : s == 2 ? sc[t][i][0].z : sc[t][i][0].w;
                             }
-                            acc[t][i] = fmaf(sv, d[i], acc[t][i]);
+                            acc[ct][t][i] = fmaf(sv, d[i], acc[ct][t][i]);
                         }
                     }
                 }
@@ -640,29 +653,35 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
     // factor and the activation normalisation undone in one exact
     // power-of-two scaling
 #pragma unroll
+    for (int ct = 0; ct < NCT; ct++)
+#pragma unroll
     for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            float v = acc[t][i];
+            float v = acc[ct][t][i];
             if constexpr (NPL == 1) v += __shfl_xor(v, 8);  // hi columns n + lo columns 8 + n
-            acc[t][i] = ldexpf(v, (F == BlkFmt::Q8_0 ? -7 : Q6 ? -9 : -10) - sh);
+            acc[ct][t][i] = ldexpf(v, (F == BlkFmt::Q8_0 ? -7 : Q6 ? -9 : -10) - sh);
         }
     if (gy > 1) {
 #pragma unroll
+        for (int ct = 0; ct < NCT; ct++)
+#pragma unroll
         for (int t = 0; t < 2; t++) {
             const int rt = row0 / 16 + t;
-            if (rt < ntiles) tiled_store_partial(acc[t], ws, byi, ntiles, rt, lane, N);
+            if (rt < ntiles) tiled_store_partial(acc[ct][t], ws + (long)ct * gy * ntiles * 256, byi, ntiles, rt, lane, N);
         }
     } else if (li < N) {
+#pragma unroll
+        for (int ct = 0; ct < NCT; ct++)
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = row0 + 16 * t + 4 * lg + i;
                 if constexpr (TM) {
-                    if (row < rows && li < T) y[(long)li * rows + row] = acc[t][i];
+                    if (row < rows && 16 * ct + li < T) y[(long)(16 * ct + li) * rows + row] = acc[ct][t][i];
                 } else {
-                    if (row < rows) y[(long)row * N + li] = acc[t][i];
+                    if (row < rows) y[(long)row * N + li] = acc[0][t][i];
                 }
             }
     }
@@ -673,7 +692,14 @@ static void launch_blkt(dim3 g, hipStream_t st, const uint4* wt, const void* sc,
                         float* y, float* ws, int M, int K, int T) {
     constexpr int NPL = N <= 8 ? 1 : 2;
     constexpr int SB = F == BlkFmt::Q8_0 ? 4 : (F == BlkFmt::Q4_K || F == BlkFmt::Q5_K || F == BlkFmt::Q6_K) ? 8 : 2;  // LDS bytes per (row, block)
-    const size_t lds = (size_t)NPL * mfma_chunk_xbytes(128 * UPW, 16) + 16 + (size_t)8 * UPW * 64 * SB;
+    constexpr size_t lds =
+        (N > 16 ? (size_t)NPL * 128 * UPW * 64 : (size_t)NPL * mfma_chunk_xbytes(128 * UPW, 16) + 16) +
+        (size_t)8 * UPW * 64 * SB;
+    if constexpr (lds > 65536) {  // past the default dynamic LDS limit (gfx950 has 160 KB a CU)
+        static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void*>(&blkt_mfma_kernel<F, UPW, N, TM>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+        if (!raised) return;
+    }
     blkt_mfma_kernel<F, UPW, N, TM><<<g, 256, lds, st>>>(wt, sc, aux, x, M, K, (int)g.x, (int)g.y, T, y, ws);
 }
 
@@ -693,7 +719,9 @@ static void launch_blkt_any(int upw, dim3 g, hipStream_t st, const uint4* wt, co
         case 4: launch_blkt_n<F, 4, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
         case 8: launch_blkt_n<F, 8, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
         case 12: launch_blkt_n<F, 12, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
-        default: launch_blkt_n<F, 16, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
+        case 16: launch_blkt_n<F, 16, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
+        default:
+            if constexpr (TM) launch_blkt_n<F, 32, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T);
     }
 }
 
@@ -726,7 +754,7 @@ static int gemm_blkt(const void* W_tiled, const void* S_tiled, const float* B, f
                      int tokens = 0) {
     constexpr int KQ = (F == BlkFmt::Q4_K || F == BlkFmt::Q5_K || F == BlkFmt::Q6_K) ? 256 : 128;  // K-quants: whole super-blocks
     if (M < 0 || K < 0 || K % KQ != 0) return (int)hipErrorInvalidValue;
-    if (N != 4 && N != 8 && N != 12 && N != 16) return (int)hipErrorInvalidValue;
+    if (N != 4 && N != 8 && N != 12 && N != 16 && (N != 32 || tokens <= 0)) return (int)hipErrorInvalidValue;
     if (M == 0 || K == 0) return (int)hipSuccess;
     if (W_tiled == nullptr || S_tiled == nullptr || B == nullptr || C == nullptr) return (int)hipErrorInvalidValue;
     if (((uintptr_t)W_tiled & 15) || ((uintptr_t)S_tiled & 15) || ((uintptr_t)B & 15) || ((uintptr_t)C & 3))
@@ -741,7 +769,7 @@ static int gemm_blkt(const void* W_tiled, const void* S_tiled, const float* B, f
         upw = force_upw;
         g.y = ceil_div(K / 128, upw);
     }
-    const long need = tiled_ws_bytes(M, (int)g.y);
+    const long need = tiled_ws_bytes(M, (int)g.y) * (N > 16 ? 2 : 1);
     if (need > 0 && (ws == nullptr || ws_bytes < need || ((uintptr_t)ws & 15))) return (int)hipErrorInvalidValue;
     const uint4* wt = static_cast<const uint4*>(W_tiled);
     float* wsf = static_cast<float*>(ws);
@@ -1032,11 +1060,30 @@ ZT_EXPORT int zt_gemm_q6kt_f32(const void* W_tiled, const void* S_tiled, const f
     return gemm_blkt<BlkFmt::Q6_K>(W_tiled, S_tiled, B, C, M, K, N, workspace, workspace_bytes, stream);
 }
 
+static int token_columns(int T) { return T > 16 ? 32 : (T + 3) & ~3; }
+
+ZT_EXPORT long zt_gemm_blkt_tokens_workspace_bytes(int fmt, int M, int K, int T) {
+    if (T < 1 || T > 32 || K >= 1 << 24) return -1;
+    const int N = T > 16 ? 16 : token_columns(T), nct = T > 16 ? 2 : 1;
+    long one;
+    switch (fmt) {
+        case ZT_WIDE_Q4_0: one = blkt_ws_bytes<BlkFmt::Q4_0>(M, K, N); break;
+        case ZT_WIDE_Q8_0:
+        case ZT_WIDE_Q8_GGUF: one = blkt_ws_bytes<BlkFmt::Q8_0>(M, K, N); break;
+        case ZT_WIDE_Q5_0: one = blkt_ws_bytes<BlkFmt::Q5_0>(M, K, N); break;
+        case ZT_WIDE_Q4_K: one = blkt_ws_bytes<BlkFmt::Q4_K>(M, K, N); break;
+        case ZT_WIDE_Q5_K: one = blkt_ws_bytes<BlkFmt::Q5_K>(M, K, N); break;
+        case ZT_WIDE_Q6_K: one = blkt_ws_bytes<BlkFmt::Q6_K>(M, K, N); break;
+        default: return -1;
+    }
+    return one < 0 ? -1 : one * nct;
+}
+
 ZT_EXPORT int zt_gemm_blkt_tokens_f32(int fmt, const void* W_tiled, const void* S_tiled, const void* aux,
                                       const float* X, float* C, int M, int K, int T, void* ws, long ws_bytes,
                                       hipStream_t stream) {
-    if (T < 1 || T > 16 || K >= 1 << 25) return (int)hipErrorInvalidValue;
-    const int N = (T + 3) & ~3;
+    if (T < 1 || T > 32 || K >= 1 << 24) return (int)hipErrorInvalidValue;
+    const int N = token_columns(T);
     switch (fmt) {
         case ZT_WIDE_Q4_0: return gemm_blkt<BlkFmt::Q4_0>(W_tiled, S_tiled, X, C, M, K, N, ws, ws_bytes, stream, aux, 0, T);
         case ZT_WIDE_Q8_0:

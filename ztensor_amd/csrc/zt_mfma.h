@@ -153,6 +153,12 @@ static __global__ void __launch_bounds__(64) tiled_reduce_kernel(const float* __
     // consecutive threads on consecutive floats of the partial tiles
     const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (long)ntiles * 16 * N) return;
+    const bool by_token = tokens > 0;
+    if (by_token) {  // blockIdx.y: the 16-column tile, each with partials of its own
+        ws += (long)blockIdx.y * splits * ntiles * 256;
+        y += (long)blockIdx.y * 16 * rows;
+        tokens -= 16 * blockIdx.y;
+    }
     const long rt = q / (16 * N);
     const int r = (int)(q % (16 * N)), lg = r / (4 * N), li = (r / 4) % N, e = r % 4;
     const long p = (rt * 64 + 16 * lg + li) * 4 + e, stride = (long)ntiles * 256;
@@ -166,7 +172,7 @@ static __global__ void __launch_bounds__(64) tiled_reduce_kernel(const float* __
         for (int j = 0; j < 32; j++) s += v[j];
     }
     const long row = rt * 16 + 4 * lg + e;
-    if (tokens > 0) {
+    if (by_token) {
         if (row < rows && li < tokens) y[(long)li * rows + row] = s;
     } else if (row < rows) {
         y[row * N + li] = s;
@@ -179,9 +185,9 @@ __host__ __forceinline__ long tiled_ws_bytes(int rows, int splits) {
 
 __host__ __forceinline__ void tiled_reduce(const void* ws, float* y, int rows, int N, int splits, hipStream_t st,
                                                int tokens = 0) {
-    const int ntiles = (rows + 15) / 16;
-    tiled_reduce_kernel<<<(int)(((long)ntiles * 16 * N + 63) / 64), 64, 0, st>>>(
-        static_cast<const float*>(ws), y, rows, N, ntiles, splits, tokens);
+    const int ntiles = (rows + 15) / 16, n = N < 16 ? N : 16;
+    tiled_reduce_kernel<<<dim3((unsigned)(((long)ntiles * 16 * n + 63) / 64), N > 16 ? 2 : 1), 64, 0, st>>>(
+        static_cast<const float*>(ws), y, rows, n, ntiles, splits, tokens);
 }
 
 static __global__ void mfma_zero_kernel(float* __restrict__ y, long n) {

@@ -279,10 +279,12 @@ class ROCmEngine:
             m = a.numel() // k
             if m > 1:
                 x, ct = a.reshape(m, k), None
-                if _wide_tokens(m) or _few_tokens(b.storage, nout, k, x):
+                if _few_tokens(b.storage, nout, k, x):
                     ct = self._wide_times(b.storage, nout, k, x)
-                if ct is None and m <= 16:
+                if ct is None and m <= 32:
                     ct = self._tiled_tokens(b.storage, nout, k, x)
+                if ct is None and _wide_tokens(m):
+                    ct = self._wide_times(b.storage, nout, k, x)
                 if ct is not None:
                     return ct.reshape(*a.shape[:-1], nout)
             if m == 1:  # a vector is its own transpose
@@ -348,17 +350,22 @@ class ROCmEngine:
 
     def _tiled_tokens(self, s: Any, rows: int, k: int, x: torch.Tensor) -> torch.Tensor | None:
         """x[t, k] @ dequant(W)[rows, k]^T -> fp32 [t, rows] for 2 to 16 tokens
-        on the tiled copy, the token-major form of the tiled GEMMs: no
-        transposes and no padding around the call.  None for a type or size
-        that has no tiled copy; and where columns run without one (the
-        row-block GEMMs, padded counts of a mapped file), unless it is there or can be made at no risk: with
+        (fp32 ones: to 32) on the tiled copy, the token-major form of the tiled
+        GEMMs: no transposes and no padding around the call.  Past 16 the
+        other way is the wide GEMM on the upload layout, whose packing and
+        whole-K workgroups cost more there (us at 32 tokens, against it: Q8_0
+        4096 x 4096 11.7 / 16.4, 14336 x 4096 27.4 / 30.9, 4096 x 14336 25.9 /
+        45.0; Q4_K 11.8 / 18.2, 26.8 / 28.6, 25.9 / 48.6; Q4_0 14336 x 4096
+        23.8 / 23.4).  None for a type or size that has no tiled copy; and
+        where a call needs none (the row-block GEMMs, padded counts of a
+        mapped file, more than 16 tokens), unless it is there or can be made at no risk: with
         memory to spare, and not while a graph is captured, whose pool the
         copy would be left in."""
         t = x.shape[0]
         n = -(-t // 4) * 4
         mm = s.qtype if isinstance(s, MmapStorage) else None
         half = x.dtype == torch.float16
-        if x.device != self.device or k % 128 != 0:
+        if x.device != self.device or k % 128 != 0 or (t > 16 and isinstance(s, (GPTQStorage, AWQStorage, IQ4NLStorage))):
             return None
         rowblock = False
         if isinstance(s, (GPTQStorage, AWQStorage)):
@@ -380,7 +387,7 @@ class ROCmEngine:
         if getattr(s, "_gpu", None) is None:
             self.upload_weights([s])
         buf = s.gpu_ptr()
-        if ((rowblock or (mm is not None and t != n)) and _tiled_cached(s, (f + "t", rows, k, _p(buf.tensor))) is None
+        if ((rowblock or t > 16 or (mm is not None and t != n)) and _tiled_cached(s, (f + "t", rows, k, _p(buf.tensor))) is None
                 and (torch.cuda.is_current_stream_capturing()
                      or torch.cuda.mem_get_info(self.device)[0] < 2 * rows * k + self.split_reserve_bytes)):
             return None
@@ -406,8 +413,7 @@ class ROCmEngine:
             bufs = self._q5_0_tiled(s, buf, rows, k, *o)
         else:
             bufs = self._kq_tiled(s, buf, rows, k, f)
-        size_fmt = "q8" if f == "q8gguf" else f
-        ws, wsb = self._workspace(getattr(self.lib, f"zt_gemm_{size_fmt}t_workspace_bytes")(rows, k, n))
+        ws, wsb = self._workspace(self.lib.zt_gemm_blkt_tokens_workspace_bytes(_TILED_FORMATS[f], rows, k, t))
         self.lib.call("zt_gemm_blkt_tokens_f32", _TILED_FORMATS[f], _p(bufs[0]), _p(bufs[1]),
                       _p(bufs[2]) if len(bufs) > 2 else 0, _p(x), _p(c), rows, k, t, ws, wsb, self._s)
         return c
