@@ -204,6 +204,31 @@ def test_tiled_tokens_build_a_copy_only_at_no_risk(eng, orc, fmt, rows, K, T):
     assert torch.equal(careful.matmul(xd, st.Tensor((K, rows), s)), z)  # the copy is there
 
 
+def test_graph_keeps_its_workspace(orc):
+    """A graph captured before the engine's workspace grew replays on the one it was captured with."""
+    small, w = weights("q4_0", 512, 4096, 1, orc)
+    large, _ = weights("q4_0", 4096, 4096, 2, orc)
+    side = torch.cuda.Stream()
+    e = ROCmEngine(stream=side)
+    x = activations("q4_0", 8, 4096, 3)
+    xd, xl = torch.from_numpy(x).cuda(), torch.randn(32, 4096, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        e.matmul(xd, st.Tensor((4096, 512), small))  # builds the tiled copy
+        held = e._wsbuf.data_ptr()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            y = e.matmul(xd, st.Tensor((4096, 512), small))
+        e.matmul(xl, st.Tensor((4096, 4096), large))
+        assert e._wsbuf.data_ptr() != held and any(b.data_ptr() == held for b in e._wskept)
+        junk = [torch.full((1 << 20,), 7, dtype=torch.uint8, device="cuda") for _ in range(8)]
+        for _ in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            check(y.cpu().numpy(), x, w)
+            assert all(bool((j == 7).all()) for j in junk)
+
+
 def test_tiled_tokens_entry_point_errors(eng):
     lib, p = eng.lib, 1 << 20
     for t in (0, 17):

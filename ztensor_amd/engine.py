@@ -113,13 +113,16 @@ class ROCmEngine:
     def _workspace(self, nbytes: int) -> tuple[int, int]:
         """Scratch for the split-K partials of the tiled GEMMs: one buffer per
         engine, grown on demand; calls on the engine's one stream run in
-        order, so they can share it."""
+        order, so they can share it.  A captured graph may hold the address of
+        a buffer that was outgrown, so those stay; each is at least twice the
+        one before, so together they are smaller than the last."""
         if nbytes <= 0:
             return 0, 0
         buf = getattr(self, "_wsbuf", None)
         if buf is None or buf.numel() < nbytes:
-            buf = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-            self._wsbuf = buf
+            kept = [] if buf is None else self._wskept + [buf]
+            buf = torch.empty(nbytes if buf is None else max(nbytes, 2 * buf.numel()), dtype=torch.uint8, device=self.device)
+            self._wsbuf, self._wskept = buf, kept
         return _p(buf), buf.numel()
 
     # ------------------------------------------------------ KernelRunner level
