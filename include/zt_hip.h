@@ -610,14 +610,15 @@ int zt_gemm_wide_f32(int fmt, const void* W, long offset1, long offset2, const u
                      const void* X, int x_fp16, float* C, int rows, int K, int T, void* workspace,
                      long workspace_bytes, zt_stream_t stream);
 
-/* The same product for 1 to 16 tokens (block formats: to 32) on the tiled
- * copies (zt_w4a16_tile and sz, zt_iq4nl_tile, the tile functions of the
- * ZT_WIDE_* block formats, aux = the fifth bits of Q5_0 / Q5_K): X [T, K],
- * C [T, rows], any T.  Up to 16 tokens each value is that of the column-major
- * call on the tokens padded to a multiple of 4, to the bit, and the workspace
- * that call's; zt_gemm_blkt_tokens_workspace_bytes holds for every T (-1 for a
- * call that is refused).  Alignments and errors are the column-major call's;
- * a T outside the range or an X of 2 GiB -> InvalidValue. */
+/* The same product for 1 to 32 tokens on the tiled copies (zt_w4a16_tile and
+ * sz, zt_iq4nl_tile, the tile functions of the ZT_WIDE_* block formats, aux =
+ * the fifth bits of Q5_0 / Q5_K): X [T, K], C [T, rows], any T.  Up to 16
+ * tokens each value is that of the column-major call on the tokens padded to a
+ * multiple of 4, to the bit (W4A16 and IQ4_NL past 16: of that call on each
+ * 16), and the workspace that call's; past 16 it is twice that of 16 columns.
+ * zt_gemm_blkt_tokens_workspace_bytes holds for every T (-1 for a call that is
+ * refused).  Alignments and errors are the column-major call's; a T outside
+ * the range or an X of 2 GiB -> InvalidValue. */
 int zt_gemm_w4a16t_tokens_f32(const void* W_tiled, const uint32_t* sz, const uint16_t* X, float* C, int rows, int K,
                               int T, int group_size, void* workspace, long workspace_bytes, zt_stream_t stream);
 int zt_gemm_iq4nlt_tokens_f16(const void* W_tiled, const void* S_tiled, const uint16_t* X, float* C, int rows, int K,

@@ -204,6 +204,22 @@ def test_tiled_tokens_build_a_copy_only_at_no_risk(eng, orc, fmt, rows, K, T):
     assert torch.equal(careful.matmul(xd, st.Tensor((K, rows), s)), z)  # the copy is there
 
 
+@pytest.mark.parametrize("fmt", ["gptq", "iq4_nl_f16"])
+@pytest.mark.parametrize("rows,K", [(1, 256), (130, 1280), (2060, 3328), (16400, 5120)])
+def test_tiled_fp16_tokens_to_32(eng, orc, fmt, rows, K):
+    """Two column tiles of fp16 tokens give the bits of the calls on each 16 (padded), one and several K ranges and
+    chunks."""
+    s, _ = weights(fmt, rows, K, rows + K, orc)
+    for T in (17, 30, 32):
+        x = torch.from_numpy(activations(fmt, T, K, T)).cuda()
+        y = eng._tiled_tokens(s, rows, K, x)
+        assert y.shape == (T, rows)
+        pad = torch.zeros((16, K), dtype=x.dtype, device="cuda")
+        pad[: T - 16] = x[16:]
+        assert torch.equal(y[:16], eng._tiled_tokens(s, rows, K, x[:16].contiguous()))
+        assert torch.equal(y[16:], eng._tiled_tokens(s, rows, K, pad)[: T - 16])
+
+
 def test_graph_keeps_its_workspace(orc):
     """A graph captured before the engine's workspace grew replays on the one it was captured with."""
     small, w = weights("q4_0", 512, 4096, 1, orc)
@@ -231,9 +247,9 @@ def test_graph_keeps_its_workspace(orc):
 
 def test_tiled_tokens_entry_point_errors(eng):
     lib, p = eng.lib, 1 << 20
-    for t in (0, 17):
-        assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p, p, 16, 128, t and 33, 0, 0, 0) == 1
-        assert lib.zt_gemm_blkt_tokens_workspace_bytes(1, 16, 128, t and 33) == -1
+    for t in (0, 33):
+        assert lib.zt_gemm_blkt_tokens_f32(1, p, p, 0, p, p, 16, 128, t, 0, 0, 0) == 1
+        assert lib.zt_gemm_blkt_tokens_workspace_bytes(1, 16, 128, t) == -1
         assert lib.zt_gemm_w4a16t_tokens_f32(p, p, p, p, 16, 128, t, 128, 0, 0, 0) == 1
         assert lib.zt_gemm_iq4nlt_tokens_f16(p, p, p, p, 16, 128, t, 0, 0, 0) == 1
     assert lib.zt_gemm_blkt_tokens_f32(0, p, p, 0, p, p, 16, 128, 4, 0, 0, 0) == 1  # W4A16 and IQ4_NL have their own
@@ -244,7 +260,7 @@ def test_tiled_tokens_entry_point_errors(eng):
     one, two = lib.zt_gemm_q8t_workspace_bytes(4096, 4096, 16), lib.zt_gemm_blkt_tokens_workspace_bytes(2, 4096, 4096, 17)
     assert two == 2 * one > 0 and lib.zt_gemm_blkt_tokens_workspace_bytes(2, 4096, 4096, 16) == one
     assert lib.zt_gemm_blkt_tokens_f32(2, p, p, 0, p, p, 4096, 4096, 17, p, two - 1, 0) == 1
-    assert lib.zt_gemm_w4a16t_tokens_f32(p, p, p, p, 16, 1 << 26, 4, 128, 0, 0, 0) == 1
+    assert lib.zt_gemm_w4a16t_tokens_f32(p, p, p, p, 16, 1 << 25, 4, 128, 0, 0, 0) == 1
 
 
 def test_few_tokens_special_values(eng, orc):

@@ -142,7 +142,9 @@ __device__ __forceinline__ void tiled_store_partial(const float4v& v, float* __r
 // call and the padding of T to a multiple of 4 (us, 3 / 16 tokens, with
 // those: W4A16 8192 x 8192 25.0 / 18.9 -> 11.6 / 13.3, 28672 x 8192 43.7 /
 // 40.2 -> 28.5 / 32.9; Q4_0 14336 x 4096 23.7 / 22.9 -> 12.3 / 17.8; Q6_K
-// 14336 x 4096 31.6 / 28.4 -> 18.5 / 23.5).
+// 14336 x 4096 31.6 / 28.4 -> 18.5 / 23.5).  17 to 32 tokens are two column
+// tiles against each decoded operand (32 tokens, against the wide GEMM: W4A16
+// 4096 x 14336 26.2 -> 15.7, IQ4_NL 28672 x 8192 108 -> 62).
 __device__ __forceinline__ int token_slot(int row, int piece, int KC) {
     return row * KC * 2 + ((piece & ~15) | ((piece ^ row) & 15)) * 16;
 }

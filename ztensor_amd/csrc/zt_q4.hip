@@ -1646,8 +1646,10 @@ __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __rest
     }
     const int rw0 = bxi * RW, row0 = rw0 + 32 * wave;
     const int ntiles = (rows + 15) / 16;
-    float4v acc[2];
-    acc[0] = acc[1] = (float4v){0.f, 0.f, 0.f, 0.f};
+    constexpr int NCT = N > 16 ? 2 : 1;  // 16-column tiles (32 tokens: token-major only)
+    float4v acc[NCT][2];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++) acc[ct][0] = acc[ct][1] = (float4v){0.f, 0.f, 0.f, 0.f};
     // this workgroup's K range: nch chunks of UPW units, one after another
     for (int ch = 0; ch < nch; ch++) {
     const int u0 = (byi * nch + ch) * UPW, u1 = min(nunits, u0 + UPW);
@@ -1720,10 +1722,12 @@ __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __rest
     for (int u = 0; u < UPW; u++) {
         if (u0 + u < u1) {
 #pragma unroll
-            for (int s = 0; s < 4; s++) {
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int ct = 0; ct < NCT; ct++) {
                 u32x4 bw;
                 if constexpr (TM)
-                    bw = *reinterpret_cast<const u32x4*>(smem + pb[s] + 256 * u);
+                    bw = *reinterpret_cast<const u32x4*>(smem + pb[s] + ct * (32 * KC) + 256 * u);
                 else
                     bw = __builtin_bit_cast(u32x4, mfma_b_pair(smem, lbase + (136 * u + 34 * s) * 2 * N, 8 * N));
                 // activation pairs (x0 x1), (x2 x3) each twice: k slots of the
@@ -1742,7 +1746,7 @@ __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __rest
                     // scales of rows 4 lg + i of this tile, block 4u + s
                     const uint16_t* sp = ssm + ((2 * wave + t) * UPW + u) * 64 + 16 * lg + s;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) acc[t][i] = fmaf(h2f(sp[4 * i]), d[i], acc[t][i]);
+                    for (int i = 0; i < 4; i++) acc[ct][t][i] = fmaf(h2f(sp[4 * i]), d[i], acc[ct][t][i]);
                 }
             }
         }
@@ -1751,20 +1755,24 @@ __global__ void __launch_bounds__(W * 64) iq4nlt_mfma_kernel(const uint4* __rest
     if (gy > 1) {
         // K split: partial tiles to the workspace, summed in split order by tiled_reduce_kernel
 #pragma unroll
+        for (int ct = 0; ct < NCT; ct++)
+#pragma unroll
         for (int t = 0; t < 2; t++) {
             const int rt = row0 / 16 + t;
-            if (rt < ntiles) tiled_store_partial(acc[t], ws, byi, ntiles, rt, lane, N);
+            if (rt < ntiles) tiled_store_partial(acc[ct][t], ws + (long)ct * gy * ntiles * 256, byi, ntiles, rt, lane, N);
         }
     } else if (li < N) {
+#pragma unroll
+        for (int ct = 0; ct < NCT; ct++)
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = row0 + 16 * t + 4 * lg + i;
                 if constexpr (TM) {
-                    if (row < rows && li < T) y[(long)li * rows + row] = acc[t][i];
+                    if (row < rows && 16 * ct + li < T) y[(long)(16 * ct + li) * rows + row] = acc[ct][t][i];
                 } else {
-                    if (row < rows) y[(long)row * N + li] = acc[t][i];
+                    if (row < rows) y[(long)row * N + li] = acc[0][t][i];
                 }
             }
     }
@@ -1774,7 +1782,7 @@ template <int UPW, int N, bool TM>
 static void launch_iq4t(dim3 g, hipStream_t st, const uint4* wt, const uint16_t* sc, const uint16_t* x, float* y,
                         float* ws, int M, int K, int nch, int T) {
     constexpr int W = 4;
-    const size_t lds = (size_t)mfma_chunk_xbytes(128 * UPW, N) + 16 + 2048 + (size_t)2 * W * UPW * 64 * 2;
+    const size_t lds = (size_t)(TM ? 256 * UPW * N : mfma_chunk_xbytes(128 * UPW, N)) + 16 + 2048 + (size_t)2 * W * UPW * 64 * 2;
     iq4nlt_mfma_kernel<UPW, W, N, TM><<<g, W * 64, lds, st>>>(wt, sc, x, M, K, nch, (int)g.x, (int)g.y, T, y, ws);
 }
 
@@ -1794,7 +1802,9 @@ static void launch_iq4t_any(int upw, int nch, dim3 g, hipStream_t st, const uint
         case 4: launch_iq4t_n<4, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
         case 8: launch_iq4t_n<8, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
         case 12: launch_iq4t_n<12, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
-        default: launch_iq4t_n<16, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
+        case 16: launch_iq4t_n<16, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T); break;
+        default:
+            if constexpr (TM) launch_iq4t_n<32, TM>(upw, nch, g, st, wt, sc, x, y, ws, M, K, T);
     }
 }
 
@@ -1852,7 +1862,7 @@ ZT_EXPORT long zt_gemm_iq4nlt_workspace_bytes(int M, int K, int N) {
 static int gemm_iq4nlt(const void* W_tiled, const void* S_tiled, const uint16_t* B, float* C, int M, int K, int N,
                        int tokens, void* workspace, long workspace_bytes, hipStream_t stream) {
     if (M < 0 || K < 0 || K % 128 != 0) return (int)hipErrorInvalidValue;
-    if (N != 4 && N != 8 && N != 12 && N != 16) return (int)hipErrorInvalidValue;
+    if (N != 4 && N != 8 && N != 12 && N != 16 && (N != 32 || tokens <= 0)) return (int)hipErrorInvalidValue;
     if (M == 0 || K == 0) return (int)hipSuccess;
     if (W_tiled == nullptr || S_tiled == nullptr || B == nullptr || C == nullptr) return (int)hipErrorInvalidValue;
     if (((uintptr_t)W_tiled & 15) || ((uintptr_t)S_tiled & 15) || ((uintptr_t)B & 15) || ((uintptr_t)C & 3))
@@ -1860,7 +1870,7 @@ static int gemm_iq4nlt(const void* W_tiled, const void* S_tiled, const uint16_t*
     if ((long)((M + 15) / 16) * (K / 128) * 128 >= 0x7fffffffL) return (int)hipErrorInvalidValue;  // 32-bit scale offsets
     int upw, nch;
     const dim3 g = iq4t_grid(M, K, upw, nch);
-    const long need = tiled_ws_bytes(M, (int)g.y);
+    const long need = tiled_ws_bytes(M, (int)g.y) * (N > 16 ? 2 : 1);
     if (need > 0 && (workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 15)))
         return (int)hipErrorInvalidValue;
     const uint4* wt = static_cast<const uint4*>(W_tiled);
@@ -1881,6 +1891,6 @@ ZT_EXPORT int zt_gemm_iq4nlt_f16(const void* W_tiled, const void* S_tiled, const
 
 ZT_EXPORT int zt_gemm_iq4nlt_tokens_f16(const void* W_tiled, const void* S_tiled, const uint16_t* X, float* C, int M,
                                         int K, int T, void* workspace, long workspace_bytes, hipStream_t stream) {
-    if (T < 1 || T > 16 || K >= 1 << 26) return (int)hipErrorInvalidValue;
-    return gemm_iq4nlt(W_tiled, S_tiled, X, C, M, K, (T + 3) & ~3, T, workspace, workspace_bytes, stream);
+    if (T < 1 || T > 32 || K >= 1 << 25) return (int)hipErrorInvalidValue;
+    return gemm_iq4nlt(W_tiled, S_tiled, X, C, M, K, T > 16 ? 32 : (T + 3) & ~3, T, workspace, workspace_bytes, stream);
 }

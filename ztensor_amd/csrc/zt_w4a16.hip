@@ -1148,8 +1148,10 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
     const half8v ones = (half8v){16384, 16384, 16384, 16384, 16384, 16384, 16384, 16384};  // 2^14
     uint32_t bmask = 0x03C003C0u, bexp = 0x74007400u;
     asm volatile("" : "+v"(bmask), "+s"(bexp));  // v_and_or_b32: mask in a VGPR, exponent in an SGPR
-    float4v acc[2];
-    acc[0] = acc[1] = (float4v){0.f, 0.f, 0.f, 0.f};
+    constexpr int NCT = N > 16 ? 2 : 1;  // 16-column tiles (32 tokens: token-major only)
+    float4v acc[NCT][2];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ct++) acc[ct][0] = acc[ct][1] = (float4v){0.f, 0.f, 0.f, 0.f};
     // this workgroup's K range: nch chunks of UPW units, one after another
     for (int ch = 0; ch < nch; ch++) {
     const int u0 = (byi * nch + ch) * UPW, u1 = min(nunits, u0 + UPW);
@@ -1171,7 +1173,7 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
     // (64 N bytes), so they go to LDS directly (buffer_load ... lds, the
     // lanes' bytes at consecutive 16-byte slots from the segment's base):
     // no registers held and no LDS writes for the activations
-    constexpr bool XDMA = N == 16;
+    constexpr bool XDMA = N >= 16;
     u32x4 xr[XDMA ? 1 : XP];
 #pragma unroll
     for (int i = 0; i < XP; i++) {
@@ -1246,13 +1248,16 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
 #pragma unroll
     for (int u = 0; u < UPW; u++) {
         if (u0 + u < u1) {
-            float4v d[2], dn = (float4v){0.f, 0.f, 0.f, 0.f};
-            d[0] = d[1] = (float4v){0.f, 0.f, 0.f, 0.f};
+            float4v d[NCT][2], dn[NCT];
 #pragma unroll
-            for (int s = 0; s < 4; s++) {
+            for (int ct = 0; ct < NCT; ct++) d[ct][0] = d[ct][1] = dn[ct] = (float4v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int ct = 0; ct < NCT; ct++) {
                 half8v bv;
                 if constexpr (TM) {
-                    const u32x4 o = *reinterpret_cast<const u32x4*>(smem + pb[s] + 256 * u);
+                    const u32x4 o = *reinterpret_cast<const u32x4*>(smem + pb[s] + ct * (32 * KC) + 256 * u);
                     bv = __builtin_bit_cast(half8v, XDMA ? nibble_order(o) : o);
                 } else {
                     bv = mfma_b_pair(smem, lbase + (136 * u + 8 * s) * 2 * N, 4 * N);
@@ -1262,9 +1267,9 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
                     const uint32_t dw = s == 0 ? w[u][t].x : s == 1 ? w[u][t].y : s == 2 ? w[u][t].z : w[u][t].w;
                     const u32x4 av = {((dw << 6) & bmask) | bexp, ((dw << 2) & bmask) | bexp,
                                       ((dw >> 2) & bmask) | bexp, ((dw >> 6) & bmask) | bexp};
-                    d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, av), bv, d[t], 0, 0, 0);
+                    d[ct][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, av), bv, d[ct][t], 0, 0, 0);
                 }
-                dn = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, bv, dn, 0, 0, 0);
+                dn[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, bv, dn[ct], 0, 0, 0);
             }
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -1272,7 +1277,10 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
                 const float4 qa = *reinterpret_cast<const float4*>(q), qb = *reinterpret_cast<const float4*>(q + 4);
                 const float sv[4] = {qa.x, qa.z, qb.x, qb.z}, zv[4] = {qa.y, qa.w, qb.y, qb.w};
 #pragma unroll
-                for (int i = 0; i < 4; i++) acc[t][i] = fmaf(sv[i], d[t][i], fmaf(-zv[i], dn[i], acc[t][i]));
+                for (int ct = 0; ct < NCT; ct++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        acc[ct][t][i] = fmaf(sv[i], d[ct][t][i], fmaf(-zv[i], dn[ct][i], acc[ct][t][i]));
             }
         }
     }
@@ -1280,20 +1288,24 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
     if (gy > 1) {
         // K split: partial tiles to the workspace, summed in split order by tiled_reduce_kernel
 #pragma unroll
+        for (int ct = 0; ct < NCT; ct++)
+#pragma unroll
         for (int t = 0; t < 2; t++) {
             const int rt = row0 / 16 + t;
-            if (rt < ntiles) tiled_store_partial(acc[t], ws, byi, ntiles, rt, lane, N);
+            if (rt < ntiles) tiled_store_partial(acc[ct][t], ws + (long)ct * gy * ntiles * 256, byi, ntiles, rt, lane, N);
         }
     } else if (li < N) {
+#pragma unroll
+        for (int ct = 0; ct < NCT; ct++)
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = row0 + 16 * t + 4 * lg + i;
                 if constexpr (TM) {
-                    if (row < rows && li < T) y[(long)li * rows + row] = acc[t][i];
+                    if (row < rows && 16 * ct + li < T) y[(long)(16 * ct + li) * rows + row] = acc[ct][t][i];
                 } else {
-                    if (row < rows) y[(long)row * N + li] = acc[t][i];
+                    if (row < rows) y[(long)row * N + li] = acc[0][t][i];
                 }
             }
     }
@@ -1303,7 +1315,12 @@ template <int UPW, int N, bool TM>
 static void launch_w4t(dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz, const uint16_t* x, float* y,
                        float* ws, int M, int K, int gs, int nch, int T) {
     constexpr int W = 4;
-    const size_t lds = (size_t)mfma_chunk_xbytes(128 * UPW, N) + 16 + 8 * UPW * 32 * W;
+    constexpr size_t lds = (size_t)(TM ? 256 * UPW * N : mfma_chunk_xbytes(128 * UPW, N)) + 16 + 8 * UPW * 32 * W;
+    if constexpr (lds > 65536) {  // past the default dynamic LDS limit (gfx950 has 160 KB a CU)
+        static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16t_mfma_kernel<UPW, W, N, TM>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+        if (!raised) return;
+    }
     w4a16t_mfma_kernel<UPW, W, N, TM><<<g, W * 64, lds, st>>>(wt, sz, x, M, K, gs, nch, (int)g.x, (int)g.y, T, y, ws);
 }
 
@@ -1325,7 +1342,9 @@ static void launch_w4t_any(int upw, int nch, dim3 g, hipStream_t st, const uint4
         case 4: launch_w4t_n<4, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
         case 8: launch_w4t_n<8, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
         case 12: launch_w4t_n<12, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
-        default: launch_w4t_n<16, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
+        case 16: launch_w4t_n<16, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
+        default:
+            if constexpr (TM) launch_w4t_n<32, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T);
     }
 }
 
@@ -1389,7 +1408,7 @@ static int gemm_w4a16t(const void* W_tiled, const uint32_t* sz, const uint16_t* 
                        int tokens, int group_size, void* workspace, long workspace_bytes, hipStream_t stream) {
     if (M < 0 || K < 0 || K % 128 != 0 || group_size <= 0 || group_size % 128 != 0 || K % group_size != 0)
         return (int)hipErrorInvalidValue;
-    if (N != 4 && N != 8 && N != 12 && N != 16) return (int)hipErrorInvalidValue;
+    if (N != 4 && N != 8 && N != 12 && N != 16 && (N != 32 || tokens <= 0)) return (int)hipErrorInvalidValue;
     if (M == 0 || K == 0) return (int)hipSuccess;
     if (W_tiled == nullptr || sz == nullptr || B == nullptr || C == nullptr) return (int)hipErrorInvalidValue;
     if (((uintptr_t)W_tiled & 15) || ((uintptr_t)sz & 3) || ((uintptr_t)B & 15) || ((uintptr_t)C & 3))
@@ -1397,7 +1416,7 @@ static int gemm_w4a16t(const void* W_tiled, const uint32_t* sz, const uint16_t* 
     if ((long)M * (K / group_size) >= (1L << 29)) return (int)hipErrorInvalidValue;  // 32-bit sz offsets
     int upw, nch;
     const dim3 g = w4t_grid(M, K, upw, nch);
-    const long need = tiled_ws_bytes(M, (int)g.y);
+    const long need = tiled_ws_bytes(M, (int)g.y) * (N > 16 ? 2 : 1);
     if (need > 0 && (workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 15)))
         return (int)hipErrorInvalidValue;
     const uint4* wt = static_cast<const uint4*>(W_tiled);
@@ -1418,6 +1437,6 @@ ZT_EXPORT int zt_gemm_w4a16t_f32(const void* W_tiled, const uint32_t* sz, const 
 ZT_EXPORT int zt_gemm_w4a16t_tokens_f32(const void* W_tiled, const uint32_t* sz, const uint16_t* X, float* C, int M,
                                         int K, int T, int group_size, void* workspace, long workspace_bytes,
                                         hipStream_t stream) {
-    if (T < 1 || T > 16 || K >= 1 << 26) return (int)hipErrorInvalidValue;
-    return gemm_w4a16t(W_tiled, sz, X, C, M, K, (T + 3) & ~3, T, group_size, workspace, workspace_bytes, stream);
+    if (T < 1 || T > 32 || K >= 1 << 25) return (int)hipErrorInvalidValue;
+    return gemm_w4a16t(W_tiled, sz, X, C, M, K, T > 16 ? 32 : (T + 3) & ~3, T, group_size, workspace, workspace_bytes, stream);
 }

@@ -352,14 +352,15 @@ class ROCmEngine:
         return c
 
     def _tiled_tokens(self, s: Any, rows: int, k: int, x: torch.Tensor) -> torch.Tensor | None:
-        """x[t, k] @ dequant(W)[rows, k]^T -> fp32 [t, rows] for 2 to 16 tokens
-        (fp32 ones: to 32) on the tiled copy, the token-major form of the tiled
+        """x[t, k] @ dequant(W)[rows, k]^T -> fp32 [t, rows] for 2 to 32 tokens
+        on the tiled copy, the token-major form of the tiled
         GEMMs: no transposes and no padding around the call.  Past 16 the
         other way is the wide GEMM on the upload layout, whose packing and
         whole-K workgroups cost more there (us at 32 tokens, against it: Q8_0
         4096 x 4096 11.7 / 16.4, 14336 x 4096 27.4 / 30.9, 4096 x 14336 25.9 /
         45.0; Q4_K 11.8 / 18.2, 26.8 / 28.6, 25.9 / 48.6; Q4_0 14336 x 4096
-        23.8 / 23.4).  None for a type or size that has no tiled copy; and
+        23.8 / 23.4; W4A16 8192 x 8192 18.0 / 21.5, 4096 x 14336 15.7 / 26.2;
+        IQ4_NL 22.1 / 26.5, 19.9 / 26.8).  None for a type or size that has no tiled copy; and
         where a call needs none (the row-block GEMMs, padded counts of a
         mapped file, more than 16 tokens), unless it is there or can be made at no risk: with
         memory to spare, and not while a graph is captured, whose pool the
@@ -368,12 +369,14 @@ class ROCmEngine:
         n = -(-t // 4) * 4
         mm = s.qtype if isinstance(s, MmapStorage) else None
         half = x.dtype == torch.float16
-        if x.device != self.device or k % 128 != 0 or (t > 16 and isinstance(s, (GPTQStorage, AWQStorage, IQ4NLStorage))):
+        if x.device != self.device or k % 128 != 0:
             return None
         rowblock = False
         if isinstance(s, (GPTQStorage, AWQStorage)):
             if not half or s.group_size % 128 != 0 or rows * (k // s.group_size) >= 1 << 29:
                 return None
+            if t > 16 and 8192 < rows <= 16384 and k <= 4096:
+                return None  # one nearly full round of the wide GEMM: 14336 x 4096, 32 tokens 17.5 us against 19.2
             f, rowblock = "w4a16", _w4a16_rowblock(rows, k, n)
         elif isinstance(s, IQ4NLStorage):
             if not half:
@@ -399,13 +402,13 @@ class ROCmEngine:
         c = torch.empty((t, rows), dtype=torch.float32, device=self.device)
         if f == "w4a16":
             wt, sz = self._w4a16_tiled(s, rows, k)
-            ws, wsb = self._workspace(self.lib.zt_gemm_w4a16t_workspace_bytes(rows, k, n))
+            ws, wsb = self._workspace(self.lib.zt_gemm_w4a16t_workspace_bytes(rows, k, min(n, 16)) * (2 if t > 16 else 1))
             self.lib.call("zt_gemm_w4a16t_tokens_f32", _p(wt), _p(sz), _p(x), _p(c), rows, k, t, s.group_size, ws, wsb,
                           self._s)
             return c
         if f == "iq4nl":
             wt, st = self._iq4nl_tiled(s, buf, rows, k)
-            ws, wsb = self._workspace(self.lib.zt_gemm_iq4nlt_workspace_bytes(rows, k, n))
+            ws, wsb = self._workspace(self.lib.zt_gemm_iq4nlt_workspace_bytes(rows, k, min(n, 16)) * (2 if t > 16 else 1))
             self.lib.call("zt_gemm_iq4nlt_tokens_f16", _p(wt), _p(st), _p(x), _p(c), rows, k, t, ws, wsb, self._s)
             return c
         if f in ("q4", "q8", "q8gguf"):
