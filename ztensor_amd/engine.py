@@ -984,12 +984,12 @@ def _block_wide(fmt: str, rows: int, k: int, n: int) -> bool:
 
 
 def _wide_tokens(t: int, transposed: bool = False) -> bool:
-    """Whether a batch of t tokens goes to the wide-batch GEMM: past the 16
-    columns of the tiled and row-block GEMMs, which take wider batches in
-    chunks of 16 (32 tokens of 14336 x 4096 (rows x K): Q4_0 26 us against
-    2 x 13 us and the copies of the chunks, GPTQ 18 against 2 x 13); past two
-    chunks where the activations and the result are also to be transposed
-    (a weight on the A side)."""
+    """Whether a batch of t tokens that the tiled copies do not take goes to the
+    wide-batch GEMM: past the 16 columns of the column-major GEMMs, which take
+    wider batches in chunks of 16 (32 tokens of 14336 x 4096 (rows x K): Q4_0 23
+    us against 2 x 13 us and the copies of the chunks, GPTQ 17.5 against 2 x
+    13); past two chunks where the activations and the result are also to be
+    transposed (a weight on the A side)."""
     return t > (32 if transposed else 16)
 
 
