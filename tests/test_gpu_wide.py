@@ -105,6 +105,21 @@ def test_wide_matmul_both_sides(eng, orc, fmt, rows, K, T):
     assert torch.equal(eng.matmul(off, st.Tensor((K, rows), s)), y)
 
 
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_one_token_of_any_strides(eng, orc, fmt):
+    """One token whose elements are not neighbours in memory gives the bits of its copy."""
+    rows, K = 40, 512
+    s, w = weights(fmt, rows, K, 17, orc)
+    x = torch.from_numpy(activations(fmt, 8, 2 * K, 18)).cuda()
+    t = st.Tensor((K, rows), s)
+    cols = x[:, :K].t().contiguous()  # channel-major
+    for v in (cols.t()[3:4], cols[:, 3], x[2:3, ::2], x[2, 1::2], x[2, :1].expand(K), x[2, :1].expand(1, K)):
+        y = eng.matmul(v, t)
+        assert y.shape == (*v.shape[:-1], rows)
+        assert torch.equal(y, eng.matmul(v.contiguous(), t))
+        check(y.reshape(1, rows).cpu().numpy(), v.reshape(1, K).cpu().numpy(), w)
+
+
 @pytest.mark.parametrize("fmt", ["gptq", "q4_0", "q4_k", "q6_k"])
 @pytest.mark.parametrize("rows,T", [(2304, 17), (4100, 20), (4100, 40), (4100, 100), (4100, 200), (4100, 300),
                                     (4100, 520), (9000, 500), (9000, 1030), (20000, 900)])

@@ -290,8 +290,9 @@ class ROCmEngine:
                     ct = self._wide_times(b.storage, nout, k, x)
                 if ct is not None:
                     return ct.reshape(*a.shape[:-1], nout)
-            if m == 1:  # a vector is its own transpose
-                return self._weight_times(b.storage, nout, k, a.reshape(k, 1)).reshape(*a.shape[:-1], nout)
+            if m == 1:  # a vector is its own transpose (its elements need not be neighbours: a copy then)
+                x = a.reshape(k, 1).contiguous()
+                return self._weight_times(b.storage, nout, k, x).reshape(*a.shape[:-1], nout)
             xt = a.reshape(m, k).t().contiguous()  # [K, M]
             ct = self._weight_times(b.storage, nout, k, xt)  # [Nout, M]
             return ct.t().contiguous().reshape(*a.shape[:-1], nout)
