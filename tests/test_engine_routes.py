@@ -44,3 +44,12 @@ def test_one_token_of_any_strides(name):
     y = ROCmEngine.matmul.__wrapped__(eng, x, st.Tensor((K, ROWS), object()))
     assert y.shape == (*x.shape[:-1], ROWS)
     assert torch.allclose(y.reshape(-1), w @ x.reshape(-1), rtol=1e-5, atol=1e-3)
+
+
+@pytest.mark.parametrize("name", ["vector", "column", "second of each pair", "one value for all"])
+def test_grouped_vector_of_any_strides(name):
+    x = _vectors()[name]
+    eng, w = _engine()
+    eng.device = x.device
+    for y in ROCmEngine.gemv_group.__wrapped__(eng, [st.Tensor((ROWS, K), object())] * 2, x):
+        assert torch.allclose(y, w @ x, rtol=1e-5, atol=1e-3)

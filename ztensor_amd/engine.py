@@ -829,6 +829,7 @@ class ROCmEngine:
         for w in weights:
             if not isinstance(w, Tensor) or w.shape[-1] != k:
                 raise ValueError(f"gemv_group: every weight must be a quantized [rows, {k}] Tensor")
+        x = x.contiguous()  # the kernels read K elements in a row
         if x.dtype == torch.float16 and all(isinstance(w.storage, (GPTQStorage, AWQStorage)) for w in weights):
             self.upload_weights([w.storage for w in weights])
             groups = {w.storage.group_size for w in weights}
