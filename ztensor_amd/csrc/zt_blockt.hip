@@ -688,7 +688,7 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
 }
 
 template <BlkFmt F, int UPW, int N, bool TM>
-static void launch_blkt(dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux, const float* x,
+static hipError_t launch_blkt(dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux, const float* x,
                         float* y, float* ws, int M, int K, int T) {
     constexpr int NPL = N <= 8 ? 1 : 2;
     constexpr int SB = F == BlkFmt::Q8_0 ? 4 : (F == BlkFmt::Q4_K || F == BlkFmt::Q5_K || F == BlkFmt::Q6_K) ? 8 : 2;  // LDS bytes per (row, block)
@@ -696,33 +696,33 @@ static void launch_blkt(dim3 g, hipStream_t st, const uint4* wt, const void* sc,
         (N > 16 ? (size_t)NPL * 128 * UPW * 64 : (size_t)NPL * mfma_chunk_xbytes(128 * UPW, 16) + 16) +
         (size_t)8 * UPW * 64 * SB;
     if constexpr (lds > 65536) {  // past the default dynamic LDS limit (gfx950 has 160 KB a CU)
-        static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void*>(&blkt_mfma_kernel<F, UPW, N, TM>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-        if (!raised) return;
+        static std::atomic<uint64_t> done{0};
+        const hipError_t rc = raise_lds(reinterpret_cast<const void*>(&blkt_mfma_kernel<F, UPW, N, TM>), (int)lds, done);
+        if (rc != hipSuccess) return rc;
     }
     blkt_mfma_kernel<F, UPW, N, TM><<<g, 256, lds, st>>>(wt, sc, aux, x, M, K, (int)g.x, (int)g.y, T, y, ws);
+    return hipSuccess;
 }
 
 template <BlkFmt F, int N, bool TM>
-static void launch_blkt_n(int upw, dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux,
+static hipError_t launch_blkt_n(int upw, dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux,
                           const float* x, float* y, float* ws, int M, int K, int T) {
-    if (upw >= 4)
-        launch_blkt<F, 4, N, TM>(g, st, wt, sc, aux, x, y, ws, M, K, T);
-    else
-        launch_blkt<F, 2, N, TM>(g, st, wt, sc, aux, x, y, ws, M, K, T);
+    if (upw >= 4) return launch_blkt<F, 4, N, TM>(g, st, wt, sc, aux, x, y, ws, M, K, T);
+    return launch_blkt<F, 2, N, TM>(g, st, wt, sc, aux, x, y, ws, M, K, T);
 }
 
 template <BlkFmt F, bool TM>
-static void launch_blkt_any(int upw, dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux,
+static hipError_t launch_blkt_any(int upw, dim3 g, hipStream_t st, const uint4* wt, const void* sc, const uint32_t* aux,
                             const float* x, float* y, float* ws, int M, int K, int N, int T) {
     switch (N) {
-        case 4: launch_blkt_n<F, 4, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
-        case 8: launch_blkt_n<F, 8, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
-        case 12: launch_blkt_n<F, 12, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
-        case 16: launch_blkt_n<F, 16, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T); break;
+        case 4: return launch_blkt_n<F, 4, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T);
+        case 8: return launch_blkt_n<F, 8, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T);
+        case 12: return launch_blkt_n<F, 12, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T);
+        case 16: return launch_blkt_n<F, 16, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T);
         default:
-            if constexpr (TM) launch_blkt_n<F, 32, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T);
+            if constexpr (TM) return launch_blkt_n<F, 32, TM>(upw, g, st, wt, sc, aux, x, y, ws, M, K, T);
     }
+    return hipErrorInvalidValue;
 }
 
 // Grid of a tiled block GEMM: 128 rows by the largest K range per
@@ -775,10 +775,10 @@ static int gemm_blkt(const void* W_tiled, const void* S_tiled, const float* B, f
     float* wsf = static_cast<float*>(ws);
     const uint32_t* ax = static_cast<const uint32_t*>(aux);
     // tokens > 0: B[tokens][K] and C[tokens][M], N = tokens up to a multiple of 4
-    if (tokens > 0)
-        launch_blkt_any<F, true>(upw, g, stream, wt, S_tiled, ax, B, C, wsf, M, K, N, tokens);
-    else
-        launch_blkt_any<F, false>(upw, g, stream, wt, S_tiled, ax, B, C, wsf, M, K, N, tokens);
+    const hipError_t rc = tokens > 0
+        ? launch_blkt_any<F, true>(upw, g, stream, wt, S_tiled, ax, B, C, wsf, M, K, N, tokens)
+        : launch_blkt_any<F, false>(upw, g, stream, wt, S_tiled, ax, B, C, wsf, M, K, N, tokens);
+    if (rc != hipSuccess) return (int)rc;
     if (g.y > 1) tiled_reduce(ws, C, M, N, (int)g.y, stream, tokens);
     return (int)hipGetLastError();
 }

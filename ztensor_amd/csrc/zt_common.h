@@ -15,6 +15,8 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "zt_hip.h"
 
 #define ZT_EXPORT extern "C" __attribute__((visibility("default")))
@@ -30,6 +32,22 @@ constexpr int kWave = 64;
 __device__ __forceinline__ int xcd_contiguous(int b, int G) {
     const int x = b & 7, i = b >> 3, per = G >> 3, rem = G & 7;
     return x < rem ? x * (per + 1) + i : rem * (per + 1) + (x - rem) * per + i;
+}
+
+// Raises a kernel's dynamic LDS limit past the default 64 KB (gfx950 has 160 KB
+// a CU), once on each device; done is the kernel's own.  A failure is returned
+// by every call that meets it, which then launches nothing.
+__host__ inline hipError_t raise_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
+    int dev = 0;
+    hipError_t rc = hipGetDevice(&dev);
+    const uint64_t bit = 1ull << (dev & 63);
+    if (rc == hipSuccess && dev < 64 && (done.load(std::memory_order_relaxed) & bit)) return hipSuccess;
+    if (rc == hipSuccess) rc = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (rc == hipSuccess)
+        done.fetch_or(bit, std::memory_order_relaxed);
+    else
+        (void)hipGetLastError();  // reported here, not by the next call
+    return rc;
 }
 
 // fp16 bits -> fp32, exact widening (v_cvt_f32_f16; fp16 denormals are kept).

@@ -1312,40 +1312,39 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
 }
 
 template <int UPW, int N, bool TM>
-static void launch_w4t(dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz, const uint16_t* x, float* y,
+static hipError_t launch_w4t(dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz, const uint16_t* x, float* y,
                        float* ws, int M, int K, int gs, int nch, int T) {
     constexpr int W = 4;
     constexpr size_t lds = (size_t)(TM ? 256 * UPW * N : mfma_chunk_xbytes(128 * UPW, N)) + 16 + 8 * UPW * 32 * W;
     if constexpr (lds > 65536) {  // past the default dynamic LDS limit (gfx950 has 160 KB a CU)
-        static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16t_mfma_kernel<UPW, W, N, TM>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-        if (!raised) return;
+        static std::atomic<uint64_t> done{0};
+        const hipError_t rc = raise_lds(reinterpret_cast<const void*>(&w4a16t_mfma_kernel<UPW, W, N, TM>), (int)lds, done);
+        if (rc != hipSuccess) return rc;
     }
     w4a16t_mfma_kernel<UPW, W, N, TM><<<g, W * 64, lds, st>>>(wt, sz, x, M, K, gs, nch, (int)g.x, (int)g.y, T, y, ws);
+    return hipSuccess;
 }
 
 template <int N, bool TM>
-static void launch_w4t_n(int upw, int nch, dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz,
+static hipError_t launch_w4t_n(int upw, int nch, dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz,
                          const uint16_t* x, float* y, float* ws, int M, int K, int gs, int T) {
-    if (upw == 8)
-        launch_w4t<8, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
-    else if (upw == 4)
-        launch_w4t<4, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
-    else
-        launch_w4t<2, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
+    if (upw == 8) return launch_w4t<8, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
+    if (upw == 4) return launch_w4t<4, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
+    return launch_w4t<2, N, TM>(g, st, wt, sz, x, y, ws, M, K, gs, nch, T);
 }
 
 template <bool TM>
-static void launch_w4t_any(int upw, int nch, dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz,
+static hipError_t launch_w4t_any(int upw, int nch, dim3 g, hipStream_t st, const uint4* wt, const uint32_t* sz,
                            const uint16_t* x, float* y, float* ws, int M, int K, int N, int gs, int T) {
     switch (N) {
-        case 4: launch_w4t_n<4, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
-        case 8: launch_w4t_n<8, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
-        case 12: launch_w4t_n<12, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
-        case 16: launch_w4t_n<16, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T); break;
+        case 4: return launch_w4t_n<4, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T);
+        case 8: return launch_w4t_n<8, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T);
+        case 12: return launch_w4t_n<12, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T);
+        case 16: return launch_w4t_n<16, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T);
         default:
-            if constexpr (TM) launch_w4t_n<32, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T);
+            if constexpr (TM) return launch_w4t_n<32, TM>(upw, nch, g, st, wt, sz, x, y, ws, M, K, gs, T);
     }
+    return hipErrorInvalidValue;
 }
 
 // Grid of the tiled W4A16 GEMM: 128 rows a workgroup, and a K range of 8, 4
@@ -1421,10 +1420,10 @@ static int gemm_w4a16t(const void* W_tiled, const uint32_t* sz, const uint16_t* 
         return (int)hipErrorInvalidValue;
     const uint4* wt = static_cast<const uint4*>(W_tiled);
     float* ws = static_cast<float*>(workspace);
-    if (tokens > 0)
-        launch_w4t_any<true>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, N, group_size, tokens);
-    else
-        launch_w4t_any<false>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, N, group_size, tokens);
+    const hipError_t rc = tokens > 0
+        ? launch_w4t_any<true>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, N, group_size, tokens)
+        : launch_w4t_any<false>(upw, nch, g, stream, wt, sz, B, C, ws, M, K, N, group_size, tokens);
+    if (rc != hipSuccess) return (int)rc;
     if (g.y > 1) tiled_reduce(workspace, C, M, N, (int)g.y, stream, tokens);
     return (int)hipGetLastError();
 }

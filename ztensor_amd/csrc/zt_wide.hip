@@ -954,9 +954,9 @@ template <Fmt F, int NT, int WK>
 hipError_t launch_few(const WideArgs& a, hipStream_t st) {
     constexpr int shm = WK * 4096 * (1 + NT);
     if constexpr (shm > 65536) {
-        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_gemm_kernel<F, NT, WK>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-        if (set != hipSuccess) return set;
+        static std::atomic<uint64_t> done{0};
+        const hipError_t rc = raise_lds(reinterpret_cast<const void*>(&few_gemm_kernel<F, NT, WK>), shm, done);
+        if (rc != hipSuccess) return rc;
     }
     few_gemm_kernel<F, NT, WK><<<ceil_div(a.rows, 16 * NT), 64 * WK, shm, st>>>(a);
     return hipGetLastError();
@@ -967,9 +967,10 @@ hipError_t launch_tile(const WideArgs& a, hipStream_t st) {
     constexpr int xb = 2 * WK * MT * steps_of(P) * P * 1024, rb = WK > 1 ? WK / 2 * WN * MT * NT * 1024 : 0;
     constexpr int shm = xb > rb ? xb : rb;
     if constexpr (shm > 65536) {
-        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(&wide_gemm_kernel<F, P, MT, NT, WN, WK>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-        if (set != hipSuccess) return set;
+        static std::atomic<uint64_t> done{0};
+        const hipError_t rc =
+            raise_lds(reinterpret_cast<const void*>(&wide_gemm_kernel<F, P, MT, NT, WN, WK>), shm, done);
+        if (rc != hipSuccess) return rc;
     }
     const long grid = (long)ceil_div(a.T, 16 * MT) * ceil_div(a.rows, 16 * NT * WN);
     wide_gemm_kernel<F, P, MT, NT, WN, WK><<<(int)grid, 64 * WN * WK, shm, st>>>(a);
