@@ -53,3 +53,46 @@ def test_grouped_vector_of_any_strides(name):
     eng.device = x.device
     for y in ROCmEngine.gemv_group.__wrapped__(eng, [st.Tensor((ROWS, K), object())] * 2, x):
         assert torch.allclose(y, w @ x, rtol=1e-5, atol=1e-3)
+
+
+class _Lib:
+    """Entry points that only note their calls."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        if name.endswith("_bytes"):
+            return lambda *a: 64
+        raise AttributeError(name)
+
+    def call(self, name, *args):
+        self.calls.append(name)
+
+
+@pytest.mark.parametrize("capturing", [False, True])
+def test_copies_made_in_a_capture_are_not_kept(monkeypatch, capturing):
+    """A captured copy has only been recorded: no later call may find it on the storage."""
+    from types import SimpleNamespace
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (1 << 40, 1 << 40))
+    eng = object.__new__(ROCmEngine)
+    eng.lib, eng.device, eng.stream = _Lib(), torch.device("cpu"), SimpleNamespace(cuda_stream=0)
+    eng.q6k_split, eng.split_reserve_bytes = True, 0
+    buf = SimpleNamespace(tensor=torch.zeros(64, dtype=torch.uint8), data_offset=0)
+
+    def storage():
+        return SimpleNamespace(gpu_ptr=lambda: buf, group_size=128, _gpu_scales=buf.tensor, _gpu_zeros=None)
+
+    builders = [lambda s: eng._w4a16_tiled(s, 16, 256), lambda s: eng._iq4nl_tiled(s, buf, 16, 256),
+                lambda s: eng._block_tiled(s, buf, 16, 256, "q4"), lambda s: eng._kq_tiled(s, buf, 16, 256, "q5k"),
+                lambda s: eng._q5_0_tiled(s, buf, 16, 256, 0, 0)]
+    for build in builders:
+        s = storage()
+        assert build(s) is not None
+        assert (getattr(s, "_gpu_tiled", None) is None) == capturing
+    s = storage()
+    assert (eng._q6k_split_copy(s, 0, 16, 256) is None) == capturing  # (the GEMV then reads the super-blocks)
+    assert (getattr(s, "_gpu_split", None) is None) == capturing
+    assert eng._q6k_split_copy(storage(), 0, 16, 256, for_one_call=True) is not None

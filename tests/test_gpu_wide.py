@@ -219,6 +219,39 @@ def test_tiled_tokens_build_a_copy_only_at_no_risk(eng, orc, fmt, rows, K, T):
     assert torch.equal(careful.matmul(xd, st.Tensor((K, rows), s)), z)  # the copy is there
 
 
+@pytest.mark.parametrize("fmt,rows,K,T", [
+    ("q6_k", 64, 512, 1), ("q6_k", 64, 512, 20), ("q6_k", 64, 512, 40), ("mmap_q6_k", 64, 512, 1),
+    ("mmap_q6_k", 64, 512, 20), ("mmap_q6_k", 64, 512, 40), ("q6_k", 64, 512, 8), ("q4_k", 64, 512, 7),
+    ("q5_k", 64, 512, 16), ("q5_0", 64, 512, 5), ("q4_0", 64, 512, 12), ("q8_0", 64, 512, 16),
+    ("mmap_q8_0", 64, 512, 12), ("gptq", 4100, 512, 12), ("iq4_nl_f16", 64, 8448, 8)])
+def test_a_copy_made_in_a_capture_is_the_graphs_own(eng, orc, fmt, rows, K, T):
+    """A weight's first call in a capture: nothing is kept whose kernels have only been recorded, so eager calls
+    before the first replay are right, and so is every replay after them."""
+    s, w = weights(fmt, rows, K, rows + T, orc)
+    x = activations(fmt, T, K, T)
+    xd = torch.from_numpy(x).cuda()
+    side = torch.cuda.Stream()
+    cap = ROCmEngine(stream=side)
+    cap.upload_weights([s])
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side), torch.cuda.graph(g, stream=side):
+        y = cap.matmul(xd, st.Tensor((K, rows), s))
+        a = cap.matmul(st.Tensor((rows, K), s), xd.t())
+    assert getattr(s, "_gpu_split", None) is None and getattr(s, "_gpu_tiled", None) is None
+    with torch.cuda.stream(side):
+        check(cap.matmul(xd, st.Tensor((K, rows), s)).cpu().numpy(), x, w)
+    check(eng.matmul(xd, st.Tensor((K, rows), s)).cpu().numpy(), x, w)
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            g.replay()
+        torch.cuda.synchronize()
+        check(y.cpu().numpy(), x, w)
+        check(a.t().cpu().numpy(), x, w)
+        junk = torch.full((1 << 22,), 255, dtype=torch.uint8, device="cuda")
+        del junk
+
+
 @pytest.mark.parametrize("fmt", ["gptq", "iq4_nl_f16"])
 @pytest.mark.parametrize("rows,K", [(1, 256), (130, 1280), (2060, 3328), (16400, 5120)])
 def test_tiled_fp16_tokens_to_32(eng, orc, fmt, rows, K):

@@ -84,6 +84,14 @@ def _tiled_cached(s: Any, key: tuple):
     return None
 
 
+def _keep_copy(s: Any, attr: str, copy: tuple) -> None:
+    """Caches a device copy (key, buffers ...) on its storage.  Not one made
+    while a graph is captured: its kernels have only been recorded, and its
+    memory is the graph's, so it serves the call that made it and no other."""
+    if not torch.cuda.is_current_stream_capturing():
+        setattr(s, attr, copy)
+
+
 class ROCmEngine:
     def __init__(self, device: int = 0, stream: torch.cuda.Stream | None = None, q6k_split: bool = True,
                  split_reserve_bytes: int = 1 << 30):
@@ -341,7 +349,7 @@ class ROCmEngine:
             o1, o2 = ((s._gpu_offsets["qh_offset"], s._gpu_offsets["qs_offset"]) if mm is not None
                       else (s.gpu_qh_offset(), s.gpu_qs_offset()))
         elif fmt == _WIDE["q6_k"]:
-            w = self._q6k_split_copy(s, _p(buf.tensor), rows, k)
+            w = self._q6k_split_copy(s, _p(buf.tensor), rows, k, for_one_call=True)
             if w is None:
                 return None
         x = x.contiguous()
@@ -441,7 +449,7 @@ class ROCmEngine:
         sz = torch.empty(szbytes // 4, dtype=torch.int32, device=self.device)
         zeros = _p(s._gpu_zeros) if s._gpu_zeros is not None else 0
         self.w4a16_tile(_p(s.gpu_ptr().tensor), _p(s._gpu_scales), zeros, rows, k, s.group_size, _p(wt), _p(sz))
-        s._gpu_tiled = (key, wt, sz)  # type: ignore[attr-defined]
+        _keep_copy(s, "_gpu_tiled", (key, wt, sz))
         return wt, sz
 
     def _iq4nl_tiled(self, s: Any, buf: GPUBuffer, rows: int, k: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -457,7 +465,7 @@ class ROCmEngine:
         wt = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         st = torch.empty(sbytes, dtype=torch.uint8, device=self.device)
         self.lib.call("zt_iq4nl_tile", _p(buf.tensor), rows, k, buf.data_offset, _p(wt), _p(st), self._s)
-        s._gpu_tiled = (key, wt, st)  # type: ignore[attr-defined]
+        _keep_copy(s, "_gpu_tiled", (key, wt, st))
         return wt, st
 
     def _block_tiled(self, s: Any, buf: GPUBuffer, rows: int, k: int, fmt: str) -> tuple[torch.Tensor, torch.Tensor]:
@@ -477,7 +485,7 @@ class ROCmEngine:
         wt = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         st = torch.empty(sbytes, dtype=torch.uint8, device=self.device)
         self.lib.call(f"zt_{fmt}_tile", _p(buf.tensor), rows, k, buf.data_offset, _p(wt), _p(st), self._s)
-        s._gpu_tiled = (key, wt, st)  # type: ignore[attr-defined]
+        _keep_copy(s, "_gpu_tiled", (key, wt, st))
         return wt, st
 
     @staticmethod
@@ -518,7 +526,7 @@ class ROCmEngine:
             raise ValueError(f"{f} tiled layout: unsupported shape [{rows}, {k}]")
         bufs = tuple(torch.empty(n, dtype=torch.uint8, device=self.device) for n in sizes)
         self.lib.call(f"zt_{f}_tile", _p(buf.tensor), rows, k, *(_p(b) for b in bufs), self._s)
-        s._gpu_tiled = (key,) + bufs  # type: ignore[attr-defined]
+        _keep_copy(s, "_gpu_tiled", (key,) + bufs)
         return bufs
 
     def _kq_tiled_gemm(self, s: Any, buf: GPUBuffer, rows: int, k: int, x: torch.Tensor, n: int, c: torch.Tensor,
@@ -534,31 +542,36 @@ class ROCmEngine:
         them: 35-55% faster than the raw-layout GEMV at the Llama-3-8B
         shapes.  Falls back to the raw-layout GEMV where the split kernel's
         32-bit offsets or x's alignment do not allow it, when the engine was
-        made with q6k_split=False, and when building the copy would leave less
-        than split_reserve_bytes of device memory free."""
+        made with q6k_split=False, when building the copy would leave less
+        than split_reserve_bytes of device memory free, and in a graph capture
+        before there is a copy."""
         sp = self._q6k_split_copy(s, raw_ptr, rows, k) if _p(x) % 16 == 0 else None
         if sp is None:
             self.lib.call("zt_gemv_q6k_f32", raw_ptr, _p(x), _p(c), rows, k, self._s)
             return
         self.lib.call("zt_gemv_q6ks_f32", _p(sp), _p(x), _p(c), rows, k, self._s)
 
-    def _q6k_split_copy(self, s: Any, raw_ptr: int, rows: int, k: int) -> torch.Tensor | None:
+    def _q6k_split_copy(self, s: Any, raw_ptr: int, rows: int, k: int, for_one_call: bool = False) -> torch.Tensor | None:
         """The split copy of uploaded Q6_K super-blocks, built on first use,
-        or None where it may not be built."""
+        or None where it may not be built.  In a graph capture the copy would
+        be split again by every replay, so it is only made for a call that has
+        no other way (for_one_call), and not kept."""
         key = ("q6ks", rows, k, raw_ptr)
         cached = getattr(s, "_gpu_split", None)
         if cached is not None and cached[0] != key:
             s._gpu_split = cached = None  # type: ignore[attr-defined]  # a stale copy goes before a new one
         nbytes = self.lib.zt_q6k_split_bytes(rows, k)
-        if (rows * (k // 256) * 210 >= 1 << 31 or not self.q6k_split
-                or (cached is None and torch.cuda.mem_get_info(self.device)[0] < nbytes + self.split_reserve_bytes)):
+        if rows * (k // 256) * 210 >= 1 << 31 or not self.q6k_split:
             return None
-        if cached is None:
-            sp = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-            self.lib.call("zt_q6k_split", raw_ptr, rows, k, _p(sp), self._s)
-            cached = (key, sp)
-            s._gpu_split = cached  # type: ignore[attr-defined]
-        return cached[1]
+        if cached is not None:
+            return cached[1]
+        if ((torch.cuda.is_current_stream_capturing() and not for_one_call)
+                or torch.cuda.mem_get_info(self.device)[0] < nbytes + self.split_reserve_bytes):
+            return None
+        sp = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        self.lib.call("zt_q6k_split", raw_ptr, rows, k, _p(sp), self._s)
+        _keep_copy(s, "_gpu_split", (key, sp))
+        return sp
 
     def _q5_0_tiled(self, s: Any, buf: GPUBuffer, rows: int, k: int, qh: int, qs: int) -> tuple:
         """The tiled copy of uploaded Q5_0 weights (nibbles and scales in the
@@ -574,7 +587,7 @@ class ROCmEngine:
             raise ValueError(f"Q5_0 tiled layout: unsupported shape [{rows}, {k}]")
         wt, st, ht = (torch.empty(n, dtype=torch.uint8, device=self.device) for n in sizes)
         self.lib.call("zt_q5_0_tile", _p(buf.tensor), rows, k, qh, qs, _p(wt), _p(st), _p(ht), self._s)
-        s._gpu_tiled = (key, wt, st, ht)  # type: ignore[attr-defined]
+        _keep_copy(s, "_gpu_tiled", (key, wt, st, ht))
         return wt, st, ht
 
     def _q5_0_tiled_gemm(self, s: Any, buf: GPUBuffer, rows: int, k: int, x: torch.Tensor, n: int, c: torch.Tensor,
