@@ -78,7 +78,8 @@ def test_copies_made_in_a_capture_are_not_kept(monkeypatch, capturing):
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
     monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (1 << 40, 1 << 40))
     eng = object.__new__(ROCmEngine)
-    eng.lib, eng.device, eng.stream = _Lib(), torch.device("cpu"), SimpleNamespace(cuda_stream=0)
+    eng.lib, eng.device = _Lib(), torch.device("cpu")
+    eng.stream = SimpleNamespace(cuda_stream=0, synchronize=lambda: eng.lib.calls.append("synchronize"))
     eng.q6k_split, eng.split_reserve_bytes = True, 0
     buf = SimpleNamespace(tensor=torch.zeros(64, dtype=torch.uint8), data_offset=0)
 
@@ -92,6 +93,8 @@ def test_copies_made_in_a_capture_are_not_kept(monkeypatch, capturing):
         s = storage()
         assert build(s) is not None
         assert (getattr(s, "_gpu_tiled", None) is None) == capturing
+        # a kept copy is complete: an engine on another stream may find it next
+        assert (eng.lib.calls[-1] == "synchronize") != capturing
     s = storage()
     assert (eng._q6k_split_copy(s, 0, 16, 256) is None) == capturing  # (the GEMV then reads the super-blocks)
     assert (getattr(s, "_gpu_split", None) is None) == capturing

@@ -84,14 +84,6 @@ def _tiled_cached(s: Any, key: tuple):
     return None
 
 
-def _keep_copy(s: Any, attr: str, copy: tuple) -> None:
-    """Caches a device copy (key, buffers ...) on its storage.  Not one made
-    while a graph is captured: its kernels have only been recorded, and its
-    memory is the graph's, so it serves the call that made it and no other."""
-    if not torch.cuda.is_current_stream_capturing():
-        setattr(s, attr, copy)
-
-
 class ROCmEngine:
     def __init__(self, device: int = 0, stream: torch.cuda.Stream | None = None, q6k_split: bool = True,
                  split_reserve_bytes: int = 1 << 30):
@@ -433,6 +425,17 @@ class ROCmEngine:
                       _p(bufs[2]) if len(bufs) > 2 else 0, _p(x), _p(c), rows, k, t, ws, wsb, self._s)
         return c
 
+    def _keep_copy(self, s: Any, attr: str, copy: tuple) -> None:
+        """Caches a device copy (key, buffers ...) on its storage once it is
+        there: another engine may share the storage and run on another stream,
+        which knows nothing of the kernels that write the copy (a wait of the
+        host, once a weight).  A copy made while a graph is captured is not
+        kept: its kernels have only been recorded, and its memory is the
+        graph's, so it serves the call that made it and no other."""
+        if not torch.cuda.is_current_stream_capturing():
+            self.stream.synchronize()
+            setattr(s, attr, copy)
+
     def _w4a16_tiled(self, s: Any, rows: int, k: int) -> tuple[torch.Tensor, torch.Tensor]:
         """The tiled copy of uploaded W4A16 weights for batches of 4-16
         columns, built on the device on the first batched call and kept
@@ -449,7 +452,7 @@ class ROCmEngine:
         sz = torch.empty(szbytes // 4, dtype=torch.int32, device=self.device)
         zeros = _p(s._gpu_zeros) if s._gpu_zeros is not None else 0
         self.w4a16_tile(_p(s.gpu_ptr().tensor), _p(s._gpu_scales), zeros, rows, k, s.group_size, _p(wt), _p(sz))
-        _keep_copy(s, "_gpu_tiled", (key, wt, sz))
+        self._keep_copy(s, "_gpu_tiled", (key, wt, sz))
         return wt, sz
 
     def _iq4nl_tiled(self, s: Any, buf: GPUBuffer, rows: int, k: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -465,7 +468,7 @@ class ROCmEngine:
         wt = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         st = torch.empty(sbytes, dtype=torch.uint8, device=self.device)
         self.lib.call("zt_iq4nl_tile", _p(buf.tensor), rows, k, buf.data_offset, _p(wt), _p(st), self._s)
-        _keep_copy(s, "_gpu_tiled", (key, wt, st))
+        self._keep_copy(s, "_gpu_tiled", (key, wt, st))
         return wt, st
 
     def _block_tiled(self, s: Any, buf: GPUBuffer, rows: int, k: int, fmt: str) -> tuple[torch.Tensor, torch.Tensor]:
@@ -485,7 +488,7 @@ class ROCmEngine:
         wt = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         st = torch.empty(sbytes, dtype=torch.uint8, device=self.device)
         self.lib.call(f"zt_{fmt}_tile", _p(buf.tensor), rows, k, buf.data_offset, _p(wt), _p(st), self._s)
-        _keep_copy(s, "_gpu_tiled", (key, wt, st))
+        self._keep_copy(s, "_gpu_tiled", (key, wt, st))
         return wt, st
 
     @staticmethod
@@ -526,7 +529,7 @@ class ROCmEngine:
             raise ValueError(f"{f} tiled layout: unsupported shape [{rows}, {k}]")
         bufs = tuple(torch.empty(n, dtype=torch.uint8, device=self.device) for n in sizes)
         self.lib.call(f"zt_{f}_tile", _p(buf.tensor), rows, k, *(_p(b) for b in bufs), self._s)
-        _keep_copy(s, "_gpu_tiled", (key,) + bufs)
+        self._keep_copy(s, "_gpu_tiled", (key,) + bufs)
         return bufs
 
     def _kq_tiled_gemm(self, s: Any, buf: GPUBuffer, rows: int, k: int, x: torch.Tensor, n: int, c: torch.Tensor,
@@ -570,7 +573,7 @@ class ROCmEngine:
             return None
         sp = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         self.lib.call("zt_q6k_split", raw_ptr, rows, k, _p(sp), self._s)
-        _keep_copy(s, "_gpu_split", (key, sp))
+        self._keep_copy(s, "_gpu_split", (key, sp))
         return sp
 
     def _q5_0_tiled(self, s: Any, buf: GPUBuffer, rows: int, k: int, qh: int, qs: int) -> tuple:
@@ -587,7 +590,7 @@ class ROCmEngine:
             raise ValueError(f"Q5_0 tiled layout: unsupported shape [{rows}, {k}]")
         wt, st, ht = (torch.empty(n, dtype=torch.uint8, device=self.device) for n in sizes)
         self.lib.call("zt_q5_0_tile", _p(buf.tensor), rows, k, qh, qs, _p(wt), _p(st), _p(ht), self._s)
-        _keep_copy(s, "_gpu_tiled", (key, wt, st, ht))
+        self._keep_copy(s, "_gpu_tiled", (key, wt, st, ht))
         return wt, st, ht
 
     def _q5_0_tiled_gemm(self, s: Any, buf: GPUBuffer, rows: int, k: int, x: torch.Tensor, n: int, c: torch.Tensor,
