@@ -222,7 +222,7 @@ struct WideArgs {
 // the compiler may have put right before, and the load's read of them.)
 __device__ __forceinline__ void dma_1k(const void* base, uint32_t off, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-                 : "memory");
+                 : "memory", "m0");
 }
 
 __device__ __forceinline__ uint32_t and_or(uint32_t w, uint32_t mask, uint32_t base) { return (w & mask) | base; }
