@@ -220,10 +220,15 @@ struct WideArgs {
 // base + off go to lds + 16 l.  The caller waits for vmcnt before a barrier.
 // (s_nop: 5 wait states between a vector write of the base's registers, which
 // the compiler may have put right before, and the load's read of them.)
+// m0, which the load takes its LDS address from, is a register the compiler
+// reserves: it warns of the clobber that tells it of the write.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma_1k(const void* base, uint32_t off, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
                  : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 __device__ __forceinline__ uint32_t and_or(uint32_t w, uint32_t mask, uint32_t base) { return (w & mask) | base; }
 
