@@ -189,6 +189,30 @@ def test_tiled_tokens_to_32(eng, orc, fmt, rows, K):
         check(eng._wide_times(s, rows, K, torch.from_numpy(x).cuda()).cpu().numpy(), x, w)  # the other way
 
 
+def relative_error(eng, s, w, x):
+    """2-norm of matmul's error against 64 bits, relative."""
+    rows, K = w.shape
+    xd = torch.from_numpy(x).cuda()
+    ref = xd.double() @ torch.from_numpy(w).cuda().t()
+    return float((eng.matmul(xd, st.Tensor((K, rows), s)).double() - ref).norm() / ref.norm())
+
+
+# root mean square of a rounding to fp32, relative: 2^-23 / sqrt(12) over the mean mantissa
+_ROUND = 2.4e-8
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q5_0", "q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("T", [3, 8, 16, 20, 32])
+def test_error_of_tiled_tokens(eng, orc, fmt, T):
+    """A sum of n terms of one size met in n fp32 additions is off by sqrt(n / 2) roundings.  Products are exact, so
+    what is left is one such sum over the K / 32 blocks (in K ranges, which only shortens it) and, inside a block and
+    in the activations' hi + lo, less than 6e-8."""
+    rows, K = 1024, 4096
+    s, w = weights(fmt, rows, K, 51, orc)
+    x = activations(fmt, T, K, 52)
+    assert relative_error(eng, s, w, x) <= np.sqrt(K / 32 / 2) * _ROUND + 6e-8
+
+
 @pytest.mark.parametrize("fmt,rows,K,T", [("gptq", 100, 8192, 5), ("q4_0", 100, 512, 4), ("q8_0", 300, 1024, 3),
                                           ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6), ("q4_k", 64, 512, 20),
                                           ("iq4_nl_f16", 64, 5120, 8)])

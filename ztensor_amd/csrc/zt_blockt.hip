@@ -7,19 +7,18 @@
 // and with the per-row CUDA kernels gemm_q4_f32 / gemm_q8_f32
 // (internal/cuda/kernels/gemm_q4.cu:117-201, gemm_q8.cu:121-182).  Here the
 // batched product runs on v_mfma_f32_16x16x32_f16 instead:
-//  * Weights are exact fp16 values of the normal range: a 4-bit value q
-//    (Q4_0, Q4_K) becomes 2^14 + 2^10 q (the nibble moved to mantissa bits
-//    6-9 under the exponent of 2^14: a shift and an and-or), a 5-bit value
-//    (Q5_0, Q5_K) 2^15 + 2^10 q, a Q6_K value 2^15 + 2^9 q and a Q8_0 byte
-//    2^15 + 2^7 (q + 128) (byte permutes and a shift-or).  Products with the
-//    normalised activations are exact in fp32.  (These once entered as fp16
-//    subnormals, q 2^-24; with activations spread in magnitude the gfx950
-//    MFMAs sum such small products up to 1.5e-5 off, measured against fp64
-//    products.)  The offset and the base are one more MFMA a step, every A
-//    element -(base + off 2^10) (Q6_K 2^9, Q8_0 2^7), whose result is the C
-//    input of the weight MFMAs of both tiles: each step's D is
-//    2^10 sum((q - off) x), and one v_fma_mix per output takes the block's
-//    fp16 scale straight from LDS.
+//  * Weights are the exact fp16 integers q - off: the bits go into the
+//    mantissa of 1024 (an and-or, or a byte permute) and one packed fp16 add
+//    or FMA takes base and offset off.  So each step's D is sum((q - off) x)
+//    of products that are exact in fp32, and one v_fma_mix per output takes
+//    the block's fp16 scale straight from LDS.  (Two earlier forms: fp16
+//    subnormals, q 2^-24, whose small products the gfx950 MFMAs sum up to
+//    1.5e-5 off with activations spread in magnitude; and 2^14 + 2^10 q with
+//    base and offset taken off by one more MFMA a step, as many other
+//    instructions, and roundings at the size of base times sum(x): relative
+//    error of 32 tokens, 4096 x 4096, against 64 bits, Q4_0 3.4e-7 and now
+//    1.1e-7, Q8_0 3.4e-7 and 1.2e-7, Q6_K 2.3e-7 and 1.2e-7, Q4_K 1.7e-7 and
+//    1.3e-7; 4096 x 14336 Q6_K 28.6 us and now 26.9, Q8_0 25.8 and 24.8.)
 //  * fp32 activations are split into two fp16 parts, x = hi + lo, after a
 //    power-of-two normalisation per workgroup (max |x| of the workgroup's K
 //    range maps into [2^14, 2^15)), so each activation is carried to about
@@ -53,8 +52,7 @@
 //    Q4_0 block in the Q4_0 data layout; the 16-byte super-block headers
 //    [tile][super-block][16 rows][16 B] (stl), decoded per workgroup into
 //    (d * scale, dmin * min) pairs; Q5_K adds Q5_0's fifth-bit dwords (aux).
-//    Each sub-block's min term uses the base MFMA (A all -2^14, Q5_K -2^15),
-//    -2^14 sum(x) per step, which is also the C input of its weight MFMAs.
+//    Each sub-block's min term is one more MFMA, A all -1: -sum(x) per step.
 //  * Q6_K (zt_q6k_tile): the values 0..63 as bytes in the Q8_0 tile
 //    positions, ordered so that lane group g holds values 4g .. 4g+3 of each
 //    of a block's two 16-value groups; fp32 d * sc per group [16 rows]
@@ -272,6 +270,45 @@ template <BlkFmt F>
 __device__ constexpr int blkt_token_slot(int c) {
     if (F == BlkFmt::Q8_0 || F == BlkFmt::Q6_K) return c;
     return (c & 1) * 4 + ((c & 3) >> 1) + ((c >> 2) << 1);
+}
+
+// The 8 weights q - off of block s of a 128-K unit that a lane multiplies, in
+// its A slots: q is the tile's 16 bytes that hold them, qh its fifth bits.
+template <BlkFmt F>
+__device__ __forceinline__ half8v blkt_operand(const uint4& q, uint32_t qh, int s, const uint32_t (&mask)[2], uint32_t exp) {
+    constexpr bool Q5 = F == BlkFmt::Q5_0 || F == BlkFmt::Q5_K;
+    half2v o[4];
+    if constexpr (F == BlkFmt::Q8_0 || F == BlkFmt::Q6_K) {
+        uint32_t d[2] = {(s & 1) ? q.z : q.x, (s & 1) ? q.w : q.y};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (F == BlkFmt::Q8_0) d[h] ^= 0x80808080u;  // q + 128
+            const half2v off = as_half2(F == BlkFmt::Q8_0 ? 0xE480E480u : 0xE420E420u);  // -(1024 + 128), -(1024 + 32)
+            o[2 * h] = as_half2(__builtin_amdgcn_perm(exp, d[h], 0x04010400u)) + off;
+            o[2 * h + 1] = as_half2(__builtin_amdgcn_perm(exp, d[h], 0x04030402u)) + off;
+        }
+    } else {
+        const uint32_t dw = s == 0 ? q.x : s == 1 ? q.y : s == 2 ? q.z : q.w, d8 = dw >> 8;
+        // nibbles at bits 0-3 (1024 + q) and 4-7 (1024 + 16 q) of each half, then at 8-11 and 12-15
+        uint32_t v[4] = {(dw & mask[0]) | exp, (dw & mask[1]) | exp, (d8 & mask[0]) | exp, (d8 & mask[1]) | exp};
+        if constexpr (Q5) {
+            // fifth bits to the bit above; y = byte | byte << 15 puts byte bits k and k+1 16 bits apart
+            const uint32_t xb = (qh >> (8 * s)) & 0xFFu, yb = xb | (xb << 15);
+            v[0] |= (yb << 4) & 0x00100010u;
+            v[1] |= (yb << 6) & 0x01000100u;
+            v[2] |= yb & 0x00100010u;
+            v[3] |= (yb << 2) & 0x01000100u;
+        }
+        // -(1024 + off) and, after the high nibble's 1/16, -(64 + off)
+        const half2v lo = as_half2(F == BlkFmt::Q4_0 ? 0xE408E408u : F == BlkFmt::Q5_0 ? 0xE410E410u : 0xE400E400u);
+        const half2v hi = as_half2(F == BlkFmt::Q4_0 ? 0xD480D480u : F == BlkFmt::Q5_0 ? 0xD500D500u : 0xD400D400u);
+        const half2v k16 = as_half2(0x2C002C00u);  // 1/16
+        o[0] = as_half2(v[0]) + lo;
+        o[1] = as_half2(v[1]) * k16 + hi;
+        o[2] = as_half2(v[2]) + lo;
+        o[3] = as_half2(v[3]) * k16 + hi;
+    }
+    return (half8v){o[0][0], o[0][1], o[1][0], o[1][1], o[2][0], o[2][1], o[3][0], o[3][1]};
 }
 
 // TM: token-major activations (zt_mfma.h), there also 17 to 32 tokens: two
@@ -493,20 +530,14 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
 #pragma unroll
     for (int s = 0; s < 4; s++)
         pb[s] = token_slot(NPL == 1 ? (li & 8) + min(li & 7, N - 1) : min(li, N - 1), 4 * lg + s, KC);
-    // -(base + off 2^10) in every A element: one MFMA a step gives that times
-    // sum(x), the C input of both tiles' weight MFMAs, so each step's D is
-    // 2^10 sum((q - off) x) (Q6_K: 2^9, Q8_0: 2^7).
-    // Q4_0: -(2^14 + 8 2^10) = -24576; Q5_0: -(2^15 + 16 2^10) = -49152;
-    // Q4_K: -2^14 and Q5_K: -2^15 (no offset; the MFMA's result is also the
-    // sub-block's min term); Q6_K: -(2^15 + 32 2^9); Q8_0: -(2^15 + 128 2^7).
-    const _Float16 ol = __builtin_bit_cast(
-        _Float16, (uint16_t)(F == BlkFmt::Q4_0 ? 0xF600u : F == BlkFmt::Q4_K ? 0xF400u : F == BlkFmt::Q5_K ? 0xF800u
-                             : 0xFA00u));
-    const half8v aoff = (half8v){ol, ol, ol, ol, ol, ol, ol, ol};
-    // nibble (or 5-bit value) to mantissa: mask in a VGPR, exponent in an SGPR (v_and_or_b32)
-    uint32_t nmask = Q5 ? 0x01E001E0u : 0x03C003C0u,
-             nexp = (Q5 || Q6 || F == BlkFmt::Q8_0) ? 0x78007800u : 0x74007400u;
-    asm volatile("" : "+v"(nmask), "+s"(nexp));
+    const _Float16 n1 = -1;
+    const half8v minus = (half8v){n1, n1, n1, n1, n1, n1, n1, n1};  // QK: -sum(x), for the sub-blocks' minima
+    // and-or: masks in VGPRs, the exponent of 1024 in an SGPR
+    uint32_t nmask[2] = {0x000F000Fu, 0x00F000F0u}, nexp = 0x64006400u;
+    if constexpr (F == BlkFmt::Q8_0 || F == BlkFmt::Q6_K)
+        nexp = 0x64646464u;
+    else
+        asm volatile("" : "+v"(nmask[0]), "+v"(nmask[1]), "+s"(nexp));
     float4v acc[NCT][2];
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++) acc[ct][0] = acc[ct][1] = (float4v){0.f, 0.f, 0.f, 0.f};
@@ -551,28 +582,14 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
                         bq[0][pl] = __builtin_bit_cast(half4v, (short4v){b8[0], b8[1], b8[2], b8[3]});
                         bq[1][pl] = __builtin_bit_cast(half4v, (short4v){b8[4], b8[5], b8[6], b8[7]});
                     }
-                    const half4v ao = (half4v){ol, ol, ol, ol};
-                    float4v dq[2];
-#pragma unroll
-                    for (int hq = 0; hq < 2; hq++) {
-                        dq[hq] = __builtin_amdgcn_mfma_f32_16x16x16f16(ao, bq[hq][0], (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                        if constexpr (NPL == 2) dq[hq] = __builtin_amdgcn_mfma_f32_16x16x16f16(ao, bq[hq][1], dq[hq], 0, 0, 0);
-                    }
 #pragma unroll
                     for (int t = 0; t < 2; t++) {
-                        const uint4 q = w[u][t][s >> 1];
-                        const uint32_t da = (s & 1) ? q.z : q.x, db = (s & 1) ? q.w : q.y;
-                        // values 0..63 to 2^15 + 2^9 q: byte permute, then v_lshl_or_b32
-                        auto q6h = [&](uint32_t v) { return (v << 4) | nexp; };
-                        const half4v aq[2] = {
-                            __builtin_bit_cast(half4v, (uint2){q6h(__builtin_amdgcn_perm(da, da, 0x0C010C00u)),
-                                                               q6h(__builtin_amdgcn_perm(da, da, 0x0C030C02u))}),
-                            __builtin_bit_cast(half4v, (uint2){q6h(__builtin_amdgcn_perm(db, db, 0x0C010C00u)),
-                                                               q6h(__builtin_amdgcn_perm(db, db, 0x0C030C02u))})};
+                        const half8v a8 = blkt_operand<F>(w[u][t][s >> 1], 0, s, nmask, nexp);
+                        const half4v aq[2] = {(half4v){a8[0], a8[1], a8[2], a8[3]}, (half4v){a8[4], a8[5], a8[6], a8[7]}};
                         float4v d[2];
 #pragma unroll
                         for (int hq = 0; hq < 2; hq++) {
-                            d[hq] = __builtin_amdgcn_mfma_f32_16x16x16f16(aq[hq], bq[hq][0], dq[hq], 0, 0, 0);
+                            d[hq] = __builtin_amdgcn_mfma_f32_16x16x16f16(aq[hq], bq[hq][0], (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                             if constexpr (NPL == 2)
                                 d[hq] = __builtin_amdgcn_mfma_f32_16x16x16f16(aq[hq], bq[hq][1], d[hq], 0, 0, 0);
                         }
@@ -585,55 +602,24 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
                     }
                     continue;
                 }
-                float4v dn = __builtin_amdgcn_mfma_f32_16x16x32_f16(aoff, bv[0], (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                if constexpr (NPL == 2) dn = __builtin_amdgcn_mfma_f32_16x16x32_f16(aoff, bv[1], dn, 0, 0, 0);
+                float4v dn = {0.f, 0.f, 0.f, 0.f};
+                if constexpr (QK) {
+                    dn = __builtin_amdgcn_mfma_f32_16x16x32_f16(minus, bv[0], dn, 0, 0, 0);
+                    if constexpr (NPL == 2) dn = __builtin_amdgcn_mfma_f32_16x16x32_f16(minus, bv[1], dn, 0, 0, 0);
+                }
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
-                    u32x4 av;
-                    if constexpr (F != BlkFmt::Q8_0) {
-                        const uint4 q = w[u][t][0];
-                        const uint32_t dw = s == 0 ? q.x : s == 1 ? q.y : s == 2 ? q.z : q.w;
-                        // nibbles at bits 0-3, 4-7, 8-11, 12-15 of each half to mantissa bits 6-9
-                        // (Q5: 5-8, the fifth bit then at 9)
-                        if constexpr (Q5)
-                            av = (u32x4){((dw << 5) & nmask) | nexp, ((dw << 1) & nmask) | nexp,
-                                         ((dw >> 3) & nmask) | nexp, ((dw >> 7) & nmask) | nexp};
-                        else
-                            av = (u32x4){((dw << 6) & nmask) | nexp, ((dw << 2) & nmask) | nexp,
-                                         ((dw >> 2) & nmask) | nexp, ((dw >> 6) & nmask) | nexp};
-                        if constexpr (Q5) {
-                            // fifth bits to bit 9 of each half (2^10 16 more); y = byte | byte << 15
-                            // puts byte bits k and k+1 16 bits apart
-                            const uint32_t xb = (qhw[u][t] >> (8 * s)) & 0xFFu, yb = xb | (xb << 15);
-                            av[0] |= (yb << 9) & 0x02000200u;
-                            av[1] |= (yb << 7) & 0x02000200u;
-                            av[2] |= (yb << 5) & 0x02000200u;
-                            av[3] |= (yb << 3) & 0x02000200u;
-                        }
-                    } else {
-                        const uint4 q = w[u][t][s >> 1];
-                        const uint32_t da = ((s & 1) ? q.z : q.x) ^ 0x80808080u;
-                        const uint32_t db = ((s & 1) ? q.w : q.y) ^ 0x80808080u;
-                        // bytes q + 128 to 2^15 + 2^7 (q + 128): byte permute, then v_lshl_or_b32
-                        auto q8h = [&](uint32_t v) { return (v << 2) | nexp; };
-                        av = (u32x4){q8h(__builtin_amdgcn_perm(da, da, 0x0C010C00u)),
-                                     q8h(__builtin_amdgcn_perm(da, da, 0x0C030C02u)),
-                                     q8h(__builtin_amdgcn_perm(db, db, 0x0C010C00u)),
-                                     q8h(__builtin_amdgcn_perm(db, db, 0x0C030C02u))};
-                    }
-                    float4v d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, av), bv[0], dn,
-                                                                      0, 0, 0);
-                    if constexpr (NPL == 2)
-                        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, av), bv[1], d, 0, 0, 0);
+                    const half8v av = blkt_operand<F>(w[u][t][F == BlkFmt::Q8_0 ? s >> 1 : 0], Q5 ? qhw[Q5 ? u : 0][t] : 0, s,
+                                                      nmask, nexp);
+                    float4v d = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv[0], (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    if constexpr (NPL == 2) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv[1], d, 0, 0, 0);
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         if constexpr (QK) {
-                            // D = 2^10 sum(q x) and dn = -2^14 sum(x) (Q5_K: -2^15):
-                            // 2^10 (d sc sum(q x) - dmin mn sum(x)) = sv D + (mv 2^-4) dn
+                            // d sc sum(q x) - dmin mn sum(x)
                             const SV& pr = sc[t][i][s >> 1];
                             const float sv = (s & 1) ? pr.z : pr.x, mv = (s & 1) ? pr.w : pr.y;
-                            acc[ct][t][i] = fmaf(sv, d[i], fmaf(mv * (F == BlkFmt::Q5_K ? 0.03125f : 0.0625f), dn[i],
-                                                            acc[ct][t][i]));
+                            acc[ct][t][i] = fmaf(sv, d[i], fmaf(mv, dn[i], acc[ct][t][i]));
                         } else {
                             float sv;
                             if constexpr (F == BlkFmt::Q4_0 || F == BlkFmt::Q5_0) {  // fp16 scales
@@ -649,9 +635,7 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
             }
         }
     }
-    // y = acc / (2^10 c) (Q6_K: 2^9 c; Q8_0: 2^7 c): the weight encoding's
-    // factor and the activation normalisation undone in one exact
-    // power-of-two scaling
+    // y = acc / c: the activation normalisation undone, an exact power-of-two scaling
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++)
 #pragma unroll
@@ -660,7 +644,7 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
         for (int i = 0; i < 4; i++) {
             float v = acc[ct][t][i];
             if constexpr (NPL == 1) v += __shfl_xor(v, 8);  // hi columns n + lo columns 8 + n
-            acc[ct][t][i] = ldexpf(v, (F == BlkFmt::Q8_0 ? -7 : Q6 ? -9 : -10) - sh);
+            acc[ct][t][i] = ldexpf(v, -sh);
         }
     if (gy > 1) {
 #pragma unroll
