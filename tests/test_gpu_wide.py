@@ -175,18 +175,40 @@ def test_tiled_tokens_are_the_columns(eng, orc, monkeypatch, fmt, rows, K):
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q5_0", "q4_k", "q5_k", "q6_k", "mmap_q8_0", "mmap_q4_k"])
 @pytest.mark.parametrize("rows,K", [(1, 256), (37, 768), (130, 1280), (2060, 3328)])
 def test_tiled_tokens_to_32(eng, orc, fmt, rows, K):
-    """Two column tiles: partial and whole second tiles, one and several K ranges, ragged rows; tokens of very
-    different sizes share a K range's power-of-two scale, whose absolute floor is 2^-39 of the largest value."""
+    """Two column tiles: partial and whole second tiles, one and several K ranges, ragged rows."""
     s, w = weights(fmt, rows, K, rows + K, orc)
     for T in (17, 18, 31, 32):
         x = activations(fmt, T, K, T)
         x[T - 1] *= 30.0
         y = eng._tiled_tokens(s, rows, K, torch.from_numpy(x).cuda()).cpu().numpy()
         assert y.shape == (T, rows)
-        floor = 2.0**-38 * np.abs(x).max() * np.abs(w).sum(axis=1)
-        bound = (K / 32 + 24) * 2.0**-24 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + floor
-        assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound), T
+        check(y, x, w)
         check(eng._wide_times(s, rows, K, torch.from_numpy(x).cuda()).cpu().numpy(), x, w)  # the other way
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q5_0", "q4_k", "q5_k", "q6_k", "mmap_q8_0", "mmap_q4_k"])
+@pytest.mark.parametrize("T", [3, 4, 8, 12, 16, 20, 32])
+@pytest.mark.parametrize("columns", [False, True])
+def test_tiled_tokens_keep_to_themselves(eng, orc, monkeypatch, fmt, T, columns):
+    """Tokens 40 decades apart are each as exact as alone, and infinities and NaN stay in theirs, on the tiled copies:
+    token-major, and as columns.  One and several K ranges, and a last one that is shorter."""
+    import ztensor_amd.engine as E
+
+    if columns and (T > 16 or T % 4):
+        pytest.skip("columns come in 4, 8, 12 or 16")
+    monkeypatch.setattr(E, "_block_rowblock", lambda *a: False)
+    for rows, K in ((40, 256), (70, 1280)):
+        s, w = weights(fmt, rows, K, rows + T, orc)
+        x = activations(fmt, T, K, T)
+        x *= (10.0 ** np.linspace(-20, 20, T)).astype(np.float32)[:, None]
+        x[1, 5], x[T - 2, K - 3] = np.inf, np.nan
+        xd = torch.from_numpy(x).cuda()
+        y = eng._weight_times(s, rows, K, xd.t().contiguous()).t() if columns else eng._tiled_tokens(s, rows, K, xd)
+        y = y.cpu().numpy()
+        fine = [t for t in range(T) if t not in (1, T - 2)]
+        check(y[fine], x[fine], w)
+        # (T = 3: one token holds both)
+        assert not np.isfinite(y[1]).any() and np.isnan(y[T - 2]).all()
 
 
 def relative_error(eng, s, w, x):

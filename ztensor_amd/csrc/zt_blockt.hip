@@ -311,12 +311,16 @@ __device__ __forceinline__ half8v blkt_operand(const uint4& q, uint32_t qh, int 
     return (half8v){o[0][0], o[0][1], o[1][0], o[1][1], o[2][0], o[2][1], o[3][0], o[3][1]};
 }
 
+// LDS bytes for the activations' scales: 16 token exponents, or 4 waves' 16
+// column maxima; with 32 tokens none (16 bytes more left one workgroup of the
+// K-quants a CU: Q4_K 28672 x 8192 108 against 80 us, 4096 x 14336 32.7
+// against 25.7).
+constexpr int blkt_scale_bytes(int N, bool TM) { return N > 16 ? 0 : TM ? 64 : 256; }
+
 // TM: token-major activations (zt_mfma.h), there also 17 to 32 tokens: two
 // column tiles against each decoded A operand (us, 20 tokens, against the wide
 // GEMM on the upload layout: Q8_0 4096 x 14336 25.6 / 44.6, Q4_K 28672 x 8192
-// 80 / 109).  With wmax apart from the scales the K-quants' 80 KB of LDS left
-// one workgroup a CU: Q4_K 28672 x 8192 108 against 80, 4096 x 14336 32.7
-// against 25.7.
+// 80 / 109).
 template <BlkFmt F, int UPW, int N, bool TM>
 __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict__ wt, const void* __restrict__ stl,
                                                         const uint32_t* __restrict__ aux, const float* __restrict__ x,
@@ -341,12 +345,16 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
     constexpr int SP = (SPC + W * 64 - 1) / (W * 64);
     constexpr int WL = (F == BlkFmt::Q8_0 || F == BlkFmt::Q6_K) ? 2 : 1;  // 16-byte weight loads per lane per tile-unit
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    float* wmax = reinterpret_cast<float*>(smem + NPL * XPB);  // per-wave max |x|
-    // block scales, after wmax; over it with 32 tokens, so that two workgroups
-    // of the K-quants (80 KB each) fit a CU
-    char* ssm = smem + NPL * XPB + (NCT == 2 ? 0 : 16);
+    // the tokens' scale exponents (with 32 tokens in the staged activations' place, once those are used: two
+    // workgroups of the K-quants, 80 KB each, fit a CU), or each wave's max |x| of the columns
+    int* sexp = reinterpret_cast<int*>(NCT == 2 ? smem : smem + NPL * XPB);
+    float* wmax = reinterpret_cast<float*>(smem + NPL * XPB);
+    char* ssm = smem + NPL * XPB + blkt_scale_bytes(N, TM);  // block scales
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, lg = lane >> 4;
+    auto column_exponent = [&](int c) {
+        return scale_exponent(fmaxf(fmaxf(wmax[c], wmax[16 + c]), fmaxf(wmax[32 + c], wmax[48 + c])));
+    };
     const int nunits = K / 128;
     int byi = blockIdx.y, bxi = blockIdx.x;
     // gx, gy: the grid's size, passed as arguments so they arrive in preloaded
@@ -419,71 +427,135 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
             }
         }
     }
-    // workgroup max |x| -> power-of-two normalisation c = 2^sh
-    float m = 0.0f;
-#pragma unroll
-    for (int i = 0; i < XP; i++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) m = fmaxf(m, fabsf(__uint_as_float(xr[i][c])));
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if (lane == 0) wmax[wave] = m;
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-    if constexpr (NCT == 2) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // read by every wave
-    int sh = 0;
-    if (m > 0.0f && m <= 3.402823466e38f) {
-        int e2;
-        (void)frexpf(m, &e2);  // m = f 2^e2, f in [0.5, 1)
-        sh = min(127, 15 - e2);
-    }
-    const float cs = ldexpf(1.0f, sh);
+    // activations to fp16 hi + lo, scaled for each token or column (zt_mfma.h): what
+    // one holds, an infinity too, leaves the others as they would be alone
+    // token-major: thread tid's q-th piece is one of token (tid + 256 q) / TP, whose TP pieces lie in one wave or half of one
+    constexpr int TP = KC / 8, NQ = XP / 2, NR = NQ == 3 ? 4 : NQ;
+    using Max = MaxRows<TM ? NR : 1, TP>;
+    int shp[Max::C];  // scale exponents, as MaxRows leaves them
     if constexpr (TM) {
-        // hi and lo rows of a token: planes of 16 rows, or (N <= 8) rows t and 8 + t of one plane
+        float m[NR];
+        auto largest = [&](bool all) {
 #pragma unroll
-        for (int i = 0; i < XP; i += 2) {
-            const int p = tid + (i >> 1) * W * 64, t = p / (KC / 8), e = p % (KC / 8);
-            if (p < N * (KC / 8)) {
-                uint16_t h[8], l[8];
+            for (int q = 0; q < NR; q++) {
+                m[q] = 0.0f;
+                if (q >= NQ) continue;
 #pragma unroll
                 for (int c = 0; c < 8; c++) {
-                    const float v = __uint_as_float(xr[i + (c >> 2)][c & 3]) * cs;
-                    const _Float16 hv = (_Float16)v;
-                    h[blkt_token_slot<F>(c)] = __builtin_bit_cast(uint16_t, hv);
-                    l[blkt_token_slot<F>(c)] = __builtin_bit_cast(uint16_t, (_Float16)(v - (float)hv));
+                    const float v = __uint_as_float(xr[2 * q + (c >> 2)][c & 3]);
+                    m[q] = fmaxf(m[q], fabsf(all ? v : finite(v)));
                 }
+            }
+            Max::run(m);
+        };
+        largest(true);
+        float most = m[0];
+#pragma unroll
+        for (int i = 1; i < Max::C; i++) most = fmaxf(most, m[i]);
+        if (infinite(most)) largest(false);
+        float scale[Max::C];
+#pragma unroll
+        for (int i = 0; i < Max::C; i++) {
+            shp[i] = scale_exponent(m[i]);
+            scale[i] = ldexpf(1.0f, shp[i]);
+        }
+        // hi and lo rows of a token: planes of 16 rows, or (N <= 8) rows t and 8 + t of one plane
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const int p = tid + q * W * 64, t = p / TP, e = p % TP, from = Max::first(q);
+            const float cs = TP == 64 ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(scale[q % Max::C]), from))
+                                      : __shfl(scale[q % Max::C], (lane & 32) + from);
+            if (p < N * TP) {
+                float v[8];
+                half8v h, l;
+#pragma unroll
+                for (int c = 0; c < 8; c++) v[blkt_token_slot<F>(c)] = __uint_as_float(xr[2 * q + (c >> 2)][c & 3]) * cs;
+                split_hi_lo(v, h, l);
                 const int piece = (e & ~15) + 4 * (e & 3) + ((e >> 2) & 3);
-                *reinterpret_cast<short8v*>(smem + token_slot(t, piece, KC)) = __builtin_bit_cast(short8v, h);
-                *reinterpret_cast<short8v*>(smem + (NPL == 1 ? token_slot(8 + t, piece, KC) : XPB + token_slot(t, piece, KC))) =
-                    __builtin_bit_cast(short8v, l);
+                *reinterpret_cast<half8v*>(smem + token_slot(t, piece, KC)) = h;
+                *reinterpret_cast<half8v*>(smem + (NPL == 1 ? token_slot(8 + t, piece, KC) : XPB + token_slot(t, piece, KC))) = l;
             }
         }
+    }
+    auto store_exponents = [&] {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const int t = (tid + q * W * 64) / TP;
+            if (t < N && (lane & (TP - 1)) == Max::first(q)) sexp[t] = shp[q % Max::C];
+        }
+    };
+    if constexpr (TM) {
+        if constexpr (NCT == 1) store_exponents();
     } else {
+        // piece p holds columns 4 (p % PPR) ..: the same for all of a thread's pieces, or (N = 12) in turns of 3
+        constexpr int NC = PPR == 3 ? 3 : 1;
+        const int r3 = tid % 3;
+        // the maxima over the wave, by halving: value v (column 4 g + c of group g, N = 12) ends in cm[v % NC] of the
+        // 16 lanes from 16 (v / NC) on, or (else) that of columns 4 (lane % PPR) + lane / 16
+        float cm[4 * NC];
+        auto largest = [&](bool all) {
 #pragma unroll
-        for (int i = 0; i < XP; i++) {
-            const int p = tid + i * W * 64;
-            if (p < npieces) {
-                const int r = p / PPR, c4 = (p % PPR) * 4;
-                const float cr = cs;
-                const int base = mfma_xrow(blkt_lds_row<F>(r), 16);
-                uint32_t hv[2], lv[2];
+            for (int c = 0; c < 4; c++) {
+                float m[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int c = 0; c < 4; c += 2) {
-                    const float v0 = __uint_as_float(xr[i][c]) * cr, v1 = __uint_as_float(xr[i][c + 1]) * cr;
-                    const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
-                    const _Float16 l0 = (_Float16)(v0 - (float)h0), l1 = (_Float16)(v1 - (float)h1);
-                    hv[c / 2] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-                    lv[c / 2] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
+                for (int i = 0; i < XP; i++) {
+                    const float v = __uint_as_float(xr[i][c]);
+                    m[i % NC] = fmaxf(m[i % NC], fabsf(all ? v : finite(v)));
                 }
+                cm[c] = NC == 1 || r3 == 0 ? m[0] : r3 == 1 ? m[2] : m[1];
+                if constexpr (NC == 3) {
+                    cm[4 + c] = r3 == 0 ? m[1] : r3 == 1 ? m[0] : m[2];
+                    cm[8 + c] = r3 == 0 ? m[2] : r3 == 1 ? m[1] : m[0];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 2 * NC; i++) cm[i] = max_pair<32>(cm[i], cm[2 * NC + i]);
+#pragma unroll
+            for (int i = 0; i < NC; i++) {
+                cm[i] = max_step<4>(max_step<8>(max_pair<16>(cm[i], cm[NC + i])));
+                if constexpr (PPR != 4) cm[i] = max_step<2>(cm[i]);
+                if constexpr (PPR == 1 || PPR == 3) cm[i] = max_step<1>(cm[i]);
+            }
+        };
+        largest(true);
+        if (infinite(NC == 1 ? cm[0] : fmaxf(fmaxf(cm[0], cm[NC / 2]), cm[NC - 1]))) largest(false);
+        if (li < (PPR == 3 ? 1 : PPR)) {
+#pragma unroll
+            for (int i = 0; i < NC; i++) wmax[16 * wave + (PPR == 3 ? 3 * lg + i : 4 * li + lg)] = cm[i];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        float cs[NC][4];
+#pragma unroll
+        for (int g = 0; g < NC; g++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                cs[g][c] = ldexpf(1.0f, column_exponent(4 * (PPR == 3 ? (r3 + g) % 3 : tid % PPR) + c));
+#pragma unroll
+        for (int i = 0; i < XP; i += 2) {
+            float v[8];
+            half8v h, l;
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                v[e] = __uint_as_float(xr[min(i + e / 4, XP - 1)][e % 4]) * cs[(i + e / 4) % NC][e % 4];
+            split_hi_lo(v, h, l);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int p = tid + (i + j) * W * 64;
+                if (i + j >= XP || p >= npieces) continue;
+                const int r = p / PPR, c4 = (p % PPR) * 4;
+                const int base = mfma_xrow(blkt_lds_row<F>(r), 16);
+                const uint4 ha = __builtin_bit_cast(uint4, h), la = __builtin_bit_cast(uint4, l);
+                const uint2 hv = j ? make_uint2(ha.z, ha.w) : make_uint2(ha.x, ha.y);
+                const uint2 lv = j ? make_uint2(la.z, la.w) : make_uint2(la.x, la.y);
                 const int lo_off = NPL == 1 ? 16 : XPB;
                 if (N % 8 != 0 && c4 == N - 4) {
                     // last piece of a row: it also zeroes the unused columns up to the
                     // next multiple of 8, so every lane of a transposing read reads data
-                    *reinterpret_cast<uint4*>(smem + base + 2 * c4) = make_uint4(hv[0], hv[1], 0u, 0u);
-                    *reinterpret_cast<uint4*>(smem + lo_off + base + 2 * c4) = make_uint4(lv[0], lv[1], 0u, 0u);
+                    *reinterpret_cast<uint4*>(smem + base + 2 * c4) = make_uint4(hv.x, hv.y, 0u, 0u);
+                    *reinterpret_cast<uint4*>(smem + lo_off + base + 2 * c4) = make_uint4(lv.x, lv.y, 0u, 0u);
                 } else {
-                    *reinterpret_cast<uint2*>(smem + base + 2 * c4) = make_uint2(hv[0], hv[1]);
-                    *reinterpret_cast<uint2*>(smem + lo_off + base + 2 * c4) = make_uint2(lv[0], lv[1]);
+                    *reinterpret_cast<uint2*>(smem + base + 2 * c4) = hv;
+                    *reinterpret_cast<uint2*>(smem + lo_off + base + 2 * c4) = lv;
                 }
             }
         }
@@ -635,17 +707,25 @@ __global__ void __launch_bounds__(256) blkt_mfma_kernel(const uint4* __restrict_
             }
         }
     }
-    // y = acc / c: the activation normalisation undone, an exact power-of-two scaling
+    // the activations' scales undone, exact powers of two
+    if constexpr (NCT == 2) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave is done with the activations
+        store_exponents();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
 #pragma unroll
-    for (int ct = 0; ct < NCT; ct++)
+    for (int ct = 0; ct < NCT; ct++) {
+        const int col = 16 * ct + (NPL == 1 ? min(li & 7, N - 1) : min(li, N - 1));
+        const int sh = TM ? sexp[col] : column_exponent(col);
 #pragma unroll
-    for (int t = 0; t < 2; t++)
+        for (int t = 0; t < 2; t++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float v = acc[ct][t][i];
-            if constexpr (NPL == 1) v += __shfl_xor(v, 8);  // hi columns n + lo columns 8 + n
-            acc[ct][t][i] = ldexpf(v, -sh);
-        }
+            for (int i = 0; i < 4; i++) {
+                float v = acc[ct][t][i];
+                if constexpr (NPL == 1) v += __shfl_xor(v, 8);  // hi columns n + lo columns 8 + n
+                acc[ct][t][i] = ldexpf(v, -sh);
+            }
+    }
     if (gy > 1) {
 #pragma unroll
         for (int ct = 0; ct < NCT; ct++)
@@ -677,7 +757,7 @@ static hipError_t launch_blkt(dim3 g, hipStream_t st, const uint4* wt, const voi
     constexpr int NPL = N <= 8 ? 1 : 2;
     constexpr int SB = F == BlkFmt::Q8_0 ? 4 : (F == BlkFmt::Q4_K || F == BlkFmt::Q5_K || F == BlkFmt::Q6_K) ? 8 : 2;  // LDS bytes per (row, block)
     constexpr size_t lds =
-        (N > 16 ? (size_t)NPL * 128 * UPW * 64 : (size_t)NPL * mfma_chunk_xbytes(128 * UPW, 16) + 16) +
+        (size_t)NPL * (N > 16 ? 128 * UPW * 64 : mfma_chunk_xbytes(128 * UPW, 16)) + blkt_scale_bytes(N, TM) +
         (size_t)8 * UPW * 64 * SB;
     if constexpr (lds > 65536) {  // past the default dynamic LDS limit (gfx950 has 160 KB a CU)
         static std::atomic<uint64_t> done{0};

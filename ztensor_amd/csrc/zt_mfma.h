@@ -32,6 +32,79 @@ typedef __attribute__((address_space(3))) char lds_char;
 // A dword viewed as two fp16 halves (x = bits 0-15).
 __device__ __forceinline__ half2v as_half2(uint32_t u) { return __builtin_bit_cast(half2v, u); }
 
+// fp32 activations as fp16 hi + lo: each token (column) is scaled by a power of
+// two that brings its largest finite |x| to [2^14, 2^15), and what |x - hi - lo|
+// leaves is at most 2^-23 |x| + 2^-25, after scaling.
+
+constexpr float kMaxFloat = 3.402823466e38f;
+
+// Whether a largest |x| of the wave is an infinity (a NaN is never the larger
+// one): then it is taken again, of the finite values (finite).
+__device__ __forceinline__ bool infinite(float m) { return __builtin_expect(__any(m > kMaxFloat), 0); }
+__device__ __forceinline__ float finite(float v) { return fabsf(v) <= kMaxFloat ? v : 0.0f; }
+
+// The exponent of that power of two.
+__device__ __forceinline__ int scale_exponent(float m) {
+    if (!(m > 0.0f)) return 0;
+    int e2;
+    (void)frexpf(m, &e2);  // m = f 2^e2, f in [0.5, 1)
+    return min(127, 15 - e2);
+}
+
+// 8 values in two parts.  An infinity has no second one (inf - inf): any
+// finite number will do beside it, or beside a NaN, and a maximum gives one.
+__device__ __forceinline__ void split_hi_lo(const float (&v)[8], half8v& hi, half8v& lo) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        hi[e] = (_Float16)v[e];
+        lo[e] = (_Float16)(v[e] - (float)hi[e]);
+    }
+    const _Float16 b = -65504.0f;
+    lo = __builtin_elementwise_max(lo, (half8v){b, b, b, b, b, b, b, b});
+}
+
+// The larger of a's two halves of the wave (OFF 32) or of each half (OFF 16) in
+// the lower one's lanes, and of b's in the upper one's.
+template <int OFF>
+__device__ __forceinline__ float max_pair(float a, float b) {
+    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+    auto r = (OFF == 32) ? __builtin_amdgcn_permlane32_swap(ua, ub, false, false)
+                         : __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// The largest v of the lanes of one number modulo OFF, given the steps above OFF.
+template <int OFF>
+__device__ __forceinline__ float max_step(float v) {
+    if constexpr (OFF == 32 || OFF == 16)
+        return max_pair<OFF>(v, v);
+    else  // row_ror: rotate in the row of 16 lanes
+        return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + OFF, 0xF, 0xF, false)));
+}
+
+// The largest of each of R values over S lanes (64 or 32), by halving: 20 steps
+// for 8 values of a wave, one at a time 48 and an exponent each.  Value q is
+// then in v[q % C], in the 16 lanes from S' + max_lane(q) on, S' the first of
+// those S lanes.
+template <int R, int S>
+struct MaxRows {
+    static_assert(R == 1 || R == 2 || R == 4 || (R == 8 && S == 64), "");
+    static constexpr int C = S == 64 ? (R > 4 ? R / 4 : 1) : (R > 2 ? R / 2 : 1);  // values left
+    static constexpr int first(int q) { return 16 * (S == 64 ? (R == 2 ? 2 * q : R == 1 ? 0 : q / C) : R == 1 ? 0 : q / C); }
+    static __device__ __forceinline__ void run(float (&v)[R]) {
+        constexpr int H = S == 64 && R > 1 ? R / 2 : R;
+        if constexpr (S == 64) {
+#pragma unroll
+            for (int i = 0; i < H; i++) v[i] = max_pair<32>(v[i], v[R > 1 ? H + i : i]);
+        }
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            const float m = max_pair<16>(v[i], v[H > 1 ? C + i : i]);
+            v[i] = max_step<1>(max_step<2>(max_step<4>(max_step<8>(m))));
+        }
+    }
+};
+
 constexpr int kMfmaRows = 32;                         // rows per workgroup (two 16-row tiles)
 constexpr int kMfmaTiles = kMfmaRows / 16;
 constexpr int kMfmaWaves = 8;                         // waves per workgroup

@@ -109,22 +109,14 @@ __global__ void __launch_bounds__(kPackThreads) pack_kernel(const XT* __restrict
 #pragma unroll
         for (int i = 0; i < NI; i++)
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float v = fabsf(e < 4 ? a[i][e & 3] : b[i][e & 3]);
-                m = v <= 3.402823466e38f ? fmaxf(m, v) : m;  // of the finite values
-            }
+            for (int e = 0; e < 8; e++) m = fmaxf(m, fabsf(finite(e < 4 ? a[i][e & 3] : b[i][e & 3])));
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
         if ((tid & 63) == 0) wmax[tid >> 6] = m;
         __syncthreads();
 #pragma unroll
         for (int w = 0; w < kPackThreads / 64; w++) m = fmaxf(m, wmax[w]);
-        int sh = 0;
-        if (m > 0.0f) {
-            int e2;
-            (void)frexpf(m, &e2);  // m = f 2^e2, f in [0.5, 1)
-            sh = min(127, 15 - e2);
-        }
+        const int sh = scale_exponent(m);
         const float c = ldexpf(1.0f, sh);
         if (tid == 0) inv[t] = ldexpf(1.0f, -sh);
         const int no = SUMS ? (K / 8 + 127) & ~127 : K / 8;  // sums: whole 1024-K groups, zeros past K
@@ -134,28 +126,16 @@ __global__ void __launch_bounds__(kPackThreads) pack_kernel(const XT* __restrict
             if (o >= no) break;
             int ks, g, k0, k1;
             where(o, ks, g, k0, k1);
-            float v[8];
-            uint32_t h[4], l[4];
+            float v[8], r[8];
+            half8v h, l;
 #pragma unroll
             for (int e = 0; e < 8; e++) v[e] = (e < 4 ? a[i][e & 3] : b[i][e & 3]) * c;
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                uint32_t hb[2], lb[2];
-#pragma unroll
-                for (int z = 0; z < 2; z++) {
-                    const float s = v[perm[O][2 * q + z]];
-                    const _Float16 hi = (_Float16)s;
-                    // an infinity has no second part (inf - inf)
-                    const _Float16 lo = fabsf(s) <= 3.402823466e38f ? (_Float16)(s - (float)hi) : (_Float16)0.0f;
-                    hb[z] = __builtin_bit_cast(uint16_t, hi);
-                    lb[z] = __builtin_bit_cast(uint16_t, lo);
-                }
-                h[q] = hb[0] | hb[1] << 16;
-                l[q] = lb[0] | lb[1] << 16;
-            }
+            for (int e = 0; e < 8; e++) r[e] = v[perm[O][e]];
+            split_hi_lo(r, h, l);
             if (o < K / 8) {
-                dst[at(ks, g, 0)] = make_uint4(h[0], h[1], h[2], h[3]);
-                dst[at(ks, g, 1)] = make_uint4(l[0], l[1], l[2], l[3]);
+                dst[at(ks, g, 0)] = __builtin_bit_cast(uint4, h);
+                dst[at(ks, g, 1)] = __builtin_bit_cast(uint4, l);
             }
             if constexpr (SUMS) {
                 float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
