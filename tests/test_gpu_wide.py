@@ -235,6 +235,18 @@ def test_error_of_tiled_tokens(eng, orc, fmt, T):
     assert relative_error(eng, s, w, x) <= np.sqrt(K / 32 / 2) * _ROUND + 6e-8
 
 
+@pytest.mark.parametrize("fmt", ["gptq", "awq"])
+@pytest.mark.parametrize("T", [3, 8, 16, 20, 32])
+def test_error_of_tiled_fp16_tokens(eng, orc, fmt, T):
+    """As above with two terms a unit of 128, its weights about the middle zero and the rest of its zero."""
+    rows, K = 1024, 4096
+    s, w = weights(fmt, rows, K, 61, orc)
+    x = torch.from_numpy(activations(fmt, T, K, 62)).cuda()
+    ref = x.double() @ torch.from_numpy(w).cuda().t()
+    err = float((eng._tiled_tokens(s, rows, K, x).double() - ref).norm() / ref.norm())
+    assert err <= np.sqrt(K / 64 / 2) * _ROUND + 6e-8
+
+
 @pytest.mark.parametrize("fmt,rows,K,T", [("gptq", 100, 8192, 5), ("q4_0", 100, 512, 4), ("q8_0", 300, 1024, 3),
                                           ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6), ("q4_k", 64, 512, 20),
                                           ("iq4_nl_f16", 64, 5120, 8)])

@@ -1107,17 +1107,28 @@ __device__ __forceinline__ u32x4 nibble_order(const u32x4& o) {
 //    1 KB load), and X / scales are written to LDS while the weights stream;
 //    the barrier waits for LDS only, so each unit computes as soon as its own
 //    weights arrive.
-//  * A operand: the nibble pairs (e_m, e_m+4) of a dword moved to mantissa
-//    bits 6-9 under the exponent of 2^14 (a shift and an and-or a dword):
-//    a = 2^14 + 2^10 q exactly, and the MFMA products a x are exact in fp32.
-//    (fp16 subnormal weights q 2^-24 with unscaled activations give products
-//    that the gfx950 MFMAs sum about 100 ulp low.)  With D = sum(a x) and X1
-//    = sum(2^14 x) from an MFMA whose A is all 2^14,
-//    y += (s 2^-10) D - (s (16 + z) 2^-14) X1, both factors formed once per
-//    (row, unit) in fp32.
+//  * A operand: q - 8 as exact fp16 integers (w4t_operand), so the products
+//    are exact and no larger than they are with the middle zero.  With
+//    D = sum((q - 8) x) and X1 = sum(x) from an MFMA whose A is all ones,
+//    y += s D - s (z - 8) X1, both factors formed once per (row, unit) in
+//    fp32.  (As 2^14 + 2^10 q, a shift and an and-or a dword, the roundings
+//    had the size of the 2^14: relative error 2.9e-7 against 64 bits at 14336
+//    x 4096, 8 tokens, where this leaves 7.2e-8, in the same time.  fp16 subnormal weights q 2^-24 with unscaled
+//    activations give products that the gfx950 MFMAs sum about 100 ulp low.)
 //  * Workgroups are mapped XCD-aware: workgroup id mod 8 selects the XCD,
 //    and every K range of a row block runs on one XCD, whose L2 then holds
 //    the row block's scale lines.
+
+// The 8 weights q - 8 of a dword: nibbles at bits 0-3 (1024 + q) and 4-7
+// (1024 + 16 q) of each half, then at 8-11 and 12-15.
+__device__ __forceinline__ half8v w4t_operand(uint32_t dw, const uint32_t (&mask)[2], uint32_t exp) {
+    const uint32_t d8 = dw >> 8;
+    const half2v lo = as_half2(0xE408E408u), hi = as_half2(0xD480D480u), k16 = as_half2(0x2C002C00u);  // -1032, -72, 1/16
+    const half2v a = as_half2((dw & mask[0]) | exp) + lo, b = as_half2((dw & mask[1]) | exp) * k16 + hi;
+    const half2v c = as_half2((d8 & mask[0]) | exp) + lo, d = as_half2((d8 & mask[1]) | exp) * k16 + hi;
+    return (half8v){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
 template <int UPW, int W, int N, bool TM>
 __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __restrict__ wt,
                                                              const uint32_t* __restrict__ szp,
@@ -1145,9 +1156,9 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
     }
     const int rw0 = bxi * RW, row0 = rw0 + 32 * wave;
     const int ntiles = (rows + 15) / 16;
-    const half8v ones = (half8v){16384, 16384, 16384, 16384, 16384, 16384, 16384, 16384};  // 2^14
-    uint32_t bmask = 0x03C003C0u, bexp = 0x74007400u;
-    asm volatile("" : "+v"(bmask), "+s"(bexp));  // v_and_or_b32: mask in a VGPR, exponent in an SGPR
+    const half8v ones = (half8v){1, 1, 1, 1, 1, 1, 1, 1};
+    uint32_t bmask[2] = {0x000F000Fu, 0x00F000F0u}, bexp = 0x64006400u;  // 1024
+    asm volatile("" : "+v"(bmask[0]), "+v"(bmask[1]), "+s"(bexp));  // v_and_or_b32: masks in VGPRs, exponent in an SGPR
     constexpr int NCT = N > 16 ? 2 : 1;  // 16-column tiles (32 tokens: token-major only)
     float4v acc[NCT][2];
 #pragma unroll
@@ -1226,7 +1237,7 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
         const int e = tid + i * W * 64;
         if (e < UPW * RW && u0 + e / RW < u1) {
             const float sc = h2f(sr[i] & 0xffff), zz = h2f(sr[i] >> 16);
-            szs[e] = make_float2(sc * 0x1p-10f, sc * (16.0f + zz) * 0x1p-14f);
+            szs[e] = make_float2(sc, sc * (zz - 8.0f));
         }
     }
     // LDS writes visible to the workgroup; the weight loads stay in flight.
@@ -1265,9 +1276,7 @@ __global__ void __launch_bounds__(W * 64) w4a16t_mfma_kernel(const uint4* __rest
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
                     const uint32_t dw = s == 0 ? w[u][t].x : s == 1 ? w[u][t].y : s == 2 ? w[u][t].z : w[u][t].w;
-                    const u32x4 av = {((dw << 6) & bmask) | bexp, ((dw << 2) & bmask) | bexp,
-                                      ((dw >> 2) & bmask) | bexp, ((dw >> 6) & bmask) | bexp};
-                    d[ct][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, av), bv, d[ct][t], 0, 0, 0);
+                    d[ct][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w4t_operand(dw, bmask, bexp), bv, d[ct][t], 0, 0, 0);
                 }
                 dn[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, bv, dn[ct], 0, 0, 0);
             }
