@@ -247,6 +247,15 @@ def test_error_of_tiled_fp16_tokens(eng, orc, fmt, T):
     assert err <= np.sqrt(K / 64 / 2) * _ROUND + 6e-8
 
 
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k"])
+def test_error_of_wide_kquants(eng, orc, fmt):
+    """One sum over the units of 128; inside one, eight MFMAs one after another, the activations' hi + lo and the minima:
+    less than 1e-7."""
+    rows, K, T = 2304, 4096, 2048  # all of K in one wave
+    s, w = weights(fmt, rows, K, 71, orc)
+    assert relative_error(eng, s, w, activations(fmt, T, K, 72)) <= np.sqrt(K / 128 / 2) * _ROUND + 1e-7
+
+
 @pytest.mark.parametrize("fmt,rows,K,T", [("gptq", 100, 8192, 5), ("q4_0", 100, 512, 4), ("q8_0", 300, 1024, 3),
                                           ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6), ("q4_k", 64, 512, 20),
                                           ("iq4_nl_f16", 64, 5120, 8)])

@@ -387,7 +387,7 @@ __device__ __forceinline__ void iq4_lookup(uint32_t sel, half2v (&hi)[2], half2v
 
 // Decoded weights of one row tile and 32-K step: the exact value is hi (+ lo), times the scale.
 constexpr int parts_of(Fmt f) { return f == Q6_K || f == IQ4_NL ? 2 : 1; }
-constexpr bool unit_scaled(Fmt f) { return f == W4A16 || f == Q6_K; }  // one scale per 128-K unit
+constexpr bool unit_scaled(Fmt f) { return f == W4A16 || f == Q4_K || f == Q5_K || f == Q6_K; }  // one scale per 128-K unit
 
 template <Fmt F>
 __device__ __forceinline__ void decode(const Raw& r, int b, int u, int lg, half2v z1, half2v z2, half8v (&o)[parts_of(F)]) {
@@ -420,17 +420,16 @@ __device__ __forceinline__ void decode(const Raw& r, int b, int u, int lg, half2
             w >>= 4;
             v >>= 4;
         }
-        half2v k = splat2(-1024.0f);
+        // times the block's 6-bit scale: at most 31 x 63, exact
+        const half2v c = splat2((float)((u & 1) ? kq_scale(r.s, 4 + b) : kq_scale(r.s, b))), k = c * splat2(-1024.0f);
+        constexpr uint32_t B = F == Q5_K ? 0x00FF00FFu : 0x000F000Fu;
         if constexpr (F == Q5_K) {
             const int j = 4 * (u & 1) + b;  // the block's bit in every high-bit byte
             w = (w & 0x0F0F0F0Fu) | (((r.e[0] >> j) & 0x01010101u) << 4);
             v = (v & 0x0F0F0F0Fu) | (((r.e[1] >> j) & 0x01010101u) << 4);
-            o[0] = join(as_half2(and_or(w, 0x00FF00FFu, M)) + k, as_half2(and_or(w >> 8, 0x00FF00FFu, M)) + k,
-                        as_half2(and_or(v, 0x00FF00FFu, M)) + k, as_half2(and_or(v >> 8, 0x00FF00FFu, M)) + k);
-        } else {
-            o[0] = join(as_half2(and_or(w, 0x000F000Fu, M)) + k, as_half2(and_or(w >> 8, 0x000F000Fu, M)) + k,
-                        as_half2(and_or(v, 0x000F000Fu, M)) + k, as_half2(and_or(v >> 8, 0x000F000Fu, M)) + k);
         }
+        auto scaled = [&](uint32_t q) { return __builtin_elementwise_fma(as_half2(and_or(q, B, M)), c, k); };  // c q
+        o[0] = join(scaled(w), scaled(w >> 8), scaled(v), scaled(v >> 8));
     } else if constexpr (F == Q6_K) {
         // block b of a 128-value half: nibbles of bytes (b & 1) 32 + ..., low for b < 2, and bits 2 b of the high-bit bytes
         uint32_t w = r.a[2 * (b & 1)], v = r.a[2 * (b & 1) + 1];
@@ -467,10 +466,7 @@ __device__ __forceinline__ void decode(const Raw& r, int b, int u, int lg, half2
 template <Fmt F>
 __device__ __forceinline__ float block_scale(const Raw& r, int b, int u) {
     if constexpr (F == Q8_0) return __uint_as_float(r.s[b]);
-    else if constexpr (F == Q4_K || F == Q5_K) {
-        const uint32_t sc = (u & 1) ? kq_scale(r.s, 4 + b) : kq_scale(r.s, b);
-        return h2f((uint16_t)r.s[0]) * (float)sc;
-    } else return h2f((uint16_t)(r.s[b >> 1] >> (16 * (b & 1))));
+    else return h2f((uint16_t)(r.s[b >> 1] >> (16 * (b & 1))));
 }
 
 // The whole part of a W4A16 zero that goes into the operand q - zero (exact in fp16), 0 for large or non-finite zeros.
@@ -614,7 +610,7 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideAr
                     if (h == H - 1) {
 #pragma unroll
                         for (int j = 0; j < NT; j++) {
-                            const float s = h2f((uint16_t)(F == W4A16 ? cur[j].s[0] : cur[j].s[2]));
+                            const float s = h2f((uint16_t)(F == Q6_K ? cur[j].s[2] : cur[j].s[0]));
 #pragma unroll
                             for (int i = 0; i < MT; i++)
 #pragma unroll
