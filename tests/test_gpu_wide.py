@@ -256,6 +256,15 @@ def test_error_of_wide_kquants(eng, orc, fmt):
     assert relative_error(eng, s, w, activations(fmt, T, K, 72)) <= np.sqrt(K / 128 / 2) * _ROUND + 1e-7
 
 
+@pytest.mark.parametrize("fmt,terms,inside", [("q4_0", 160, 6e-8), ("q8_0", 160, 6e-8), ("mmap_q8_0", 160, 6e-8), ("q5_0", 50, 6e-8),
+                                              ("iq4_nl_f16", 50, 6e-8), ("q4_k", 22, 1e-7), ("q5_k", 22, 1e-7)])
+def test_error_of_long_rows(eng, orc, fmt, terms, inside):
+    """Long rows: no chain of sums past 160 blocks, or two of about the root of their number."""
+    rows, K, T = 1100, 14336, 2048
+    s, w = weights(fmt, rows, K, 81, orc)
+    assert relative_error(eng, s, w, activations(fmt, T, K, 82)) <= np.sqrt(terms / 2) * _ROUND + inside
+
+
 @pytest.mark.parametrize("fmt,rows,K,T", [("gptq", 100, 8192, 5), ("q4_0", 100, 512, 4), ("q8_0", 300, 1024, 3),
                                           ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6), ("q4_k", 64, 512, 20),
                                           ("iq4_nl_f16", 64, 5120, 8)])

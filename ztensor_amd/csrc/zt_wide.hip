@@ -472,8 +472,22 @@ __device__ __forceinline__ float block_scale(const Raw& r, int b, int u) {
 // The whole part of a W4A16 zero that goes into the operand q - zero (exact in fp16), 0 for large or non-finite zeros.
 __device__ __forceinline__ float whole_zero(float z) { return fabsf(z) <= 960.0f ? rintf(z) : 0.0f; }
 
-// P: parts of the activations (2 for fp32).
-template <Fmt F, int P, int MT, int NT, int WN, int WK>
+// fp32 sums of n terms of one size, added one by one, are off by sqrt(n / 2)
+// roundings.  The terms are K / 32 scaled blocks (K / 128 units), over the
+// waves along K.  Up to kChain values of K a wave adds them up as they come;
+// past it roundings would exceed those of the tiled copies and the dequantized
+// products, so more waves lie along K or (FAR) a wave's sums go to a second
+// set of them every few units.  IQ4_NL and Q5_0, whose other paths are the
+// most exact, always have the second set, at half the waves of their largest
+// tiles.  Relative error against 64 bits, one chain and now, 1021 tokens of
+// 4096 x 14336 (rows x K): Q4_0 4.0e-7 / 2.1e-7, Q5_0 3.9e-7 / 1.4e-7, Q4_K
+// 3.0e-7 / 1.7e-7, IQ4_NL 2.8e-7 / 1.3e-7; us there: 314 / 338, 363 / 364, 361
+// / 345, 333 / 298.
+constexpr int kChain = 5120;
+constexpr bool far_sums(Fmt f) { return f == IQ4_NL || f == Q5_0; }
+
+// P: parts of the activations (2 for fp32).  FAR: sums in two steps.
+template <Fmt F, int P, int MT, int NT, int WN, int WK, bool FAR>
 __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideArgs p) {
     constexpr int KSU = steps_of(P);
     constexpr int PW = parts_of(F);
@@ -514,11 +528,11 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideAr
         for (int j = 0; j < NT; j++) W.load(next[j], off[j], u, p.gu);
     };
 
-    float4v acc[MT][NT];
+    float4v acc[MT][NT], sum[FAR ? MT : 1][NT];
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int j = 0; j < NT; j++) acc[i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NT; j++) acc[i][j] = sum[FAR ? i : 0][j] = (float4v){0.f, 0.f, 0.f, 0.f};
 
     if (kg < nu) {
         stage(kg, 0, 0);
@@ -526,7 +540,20 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideAr
     }
     constexpr int H = 4 / KSU;  // barriers a unit
     bool odd = false;           // a W4A16 zero that is no whole number was seen
-    for (int t = 0; t < nsteps; t++) {
+    auto add_up = [&] {
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                sum[FAR ? i : 0][j] += acc[i][j];
+                acc[i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
+            }
+    };
+    const int per = !FAR ? nsteps : nsteps > 64 ? 5 : nsteps > 24 ? 3 : 2;  // both chains of about sqrt(4 nsteps) terms
+    for (int t0 = 0; t0 < nsteps; t0 += per) {
+    const int t1 = min(nsteps, t0 + per);
+#pragma unroll 1
+    for (int t = t0; t < t1; t++) {
         const int u = t * WK + kg;
         Raw cur[NT];
         float4v d[MT][NT];
@@ -620,6 +647,14 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideAr
                 }
             }
         }
+    }
+    if constexpr (FAR) add_up();
+    }
+    if constexpr (FAR) {
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[i][j] = sum[i][j];
     }
     if constexpr (F == W4A16) {
         // zeros that are no integers up to 960: s * zf * sum x off (all-ones B operands give a unit's sum x)
@@ -943,18 +978,18 @@ hipError_t launch_few(const WideArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <Fmt F, int P, int MT, int NT, int WN, int WK>
+template <Fmt F, int P, int MT, int NT, int WN, int WK, bool FAR = far_sums(F)>
 hipError_t launch_tile(const WideArgs& a, hipStream_t st) {
     constexpr int xb = 2 * WK * MT * steps_of(P) * P * 1024, rb = WK > 1 ? WK / 2 * WN * MT * NT * 1024 : 0;
     constexpr int shm = xb > rb ? xb : rb;
     if constexpr (shm > 65536) {
         static std::atomic<uint64_t> done{0};
         const hipError_t rc =
-            raise_lds(reinterpret_cast<const void*>(&wide_gemm_kernel<F, P, MT, NT, WN, WK>), shm, done);
+            raise_lds(reinterpret_cast<const void*>(&wide_gemm_kernel<F, P, MT, NT, WN, WK, FAR>), shm, done);
         if (rc != hipSuccess) return rc;
     }
     const long grid = (long)ceil_div(a.T, 16 * MT) * ceil_div(a.rows, 16 * NT * WN);
-    wide_gemm_kernel<F, P, MT, NT, WN, WK><<<(int)grid, 64 * WN * WK, shm, st>>>(a);
+    wide_gemm_kernel<F, P, MT, NT, WN, WK, FAR><<<(int)grid, 64 * WN * WK, shm, st>>>(a);
     return hipGetLastError();
 }
 
@@ -984,14 +1019,34 @@ hipError_t launch_gemm(const WideArgs& a, hipStream_t st) {
     if (fits(32, 32)) return launch_tile<F, P, 2, 2, 1, 8>(a, st);
     if (fits(32, 64)) return launch_tile<F, P, 2, 2, 2, 8>(a, st);
     if (fits(64, 64)) return launch_tile<F, P, 4, 2, 2, 4>(a, st);
-    if (fits(64, 128)) return launch_tile<F, P, 4, 2, 4, F == Q6_K ? 2 : 4>(a, st);
+    constexpr bool FS = far_sums(F);
+    if constexpr (F == IQ4_NL && P == 2) {  // as the column kernel that fp32 tokens had: short chains
+        if (a.K > kChain) return launch_tile<F, P, 4, 2, 2, 4>(a, st);
+        return launch_tile<F, P, 4, 2, 4, 2>(a, st);
+    }
+    if (fits(64, 128)) return launch_tile<F, P, 4, 2, 4, F == Q6_K || FS ? 2 : 4>(a, st);
     // (two parts without minima: 64 x 256 tiles, two workgroups a CU, hold their rate below 128 x 256)
     if constexpr (P == 1 || KQ || F == Q6_K) {
+        if constexpr (KQ) {
+            if (a.K > 2 * kChain && fits(128, 128)) return launch_tile<F, P, 8, 2, 4, 2, true>(a, st);
+        }
         if (fits(128, 128)) return launch_tile<F, P, 8, 2, 4, 2>(a, st);
     }
-    if (full(128, 256, P == 1 || F == Q6_K ? 0.65 : 0.85)) return launch_tile<F, P, 8, 2, 8, 1>(a, st);
-    if constexpr (!(P == 1 || KQ || F == Q6_K)) {
+    if (full(128, 256, P == 1 || F == Q6_K ? 0.65 : 0.85)) {
+        if constexpr (F != W4A16 && F != Q6_K && !FS) {
+            if (a.K > kChain) return launch_tile<F, P, 8, 2, 8, 1, true>(a, st);
+        }
+        return launch_tile<F, P, 8, 2, 8, 1>(a, st);
+    }
+    if constexpr (F == Q5_0) {
         if (full(64, 256, 0.8)) return launch_tile<F, P, 4, 2, 8, 1>(a, st);
+    } else if constexpr (!FS && F != W4A16 && F != Q6_K) {
+        // as many waves along K as keep to kChain
+        if (a.K > (KQ ? 1 : 2) * kChain) return launch_tile<F, P, 4, 2, 4, 4>(a, st);
+        if constexpr (!KQ) {
+            if (full(64, 256, 0.8)) return launch_tile<F, P, 4, 2, 8, 2>(a, st);
+            if (a.K > kChain) return launch_tile<F, P, 4, 2, 4, 2>(a, st);
+        }
     }
     return launch_tile<F, P, 4, 2, 4, 1>(a, st);
 }
