@@ -265,6 +265,15 @@ def test_error_of_long_rows(eng, orc, fmt, terms, inside):
     assert relative_error(eng, s, w, activations(fmt, T, K, 82)) <= np.sqrt(terms / 2) * _ROUND + inside
 
 
+@pytest.mark.parametrize("K,T", [(4096, 3), (4096, 37), (14336, 9), (14336, 317)])
+def test_error_of_fp32_tokens_on_iq4nl(eng, orc, K, T):
+    """As the column kernel, in fp32 throughout: the codebook's 24 bits, two chains of at most 8 terms a wave, and the
+    activations' hi + lo."""
+    rows = 512
+    s, w = weights("iq4_nl", rows, K, 91, orc)
+    assert relative_error(eng, s, w, activations("iq4_nl", T, K, 92)) <= np.sqrt(16 / 2) * _ROUND + 6e-8
+
+
 @pytest.mark.parametrize("fmt,rows,K,T", [("gptq", 100, 8192, 5), ("q4_0", 100, 512, 4), ("q8_0", 300, 1024, 3),
                                           ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6), ("q4_k", 64, 512, 20),
                                           ("iq4_nl_f16", 64, 5120, 8)])

@@ -330,13 +330,14 @@ __device__ __forceinline__ uint32_t kq_min(const uint32_t (&h)[4], int b) {
     return b < 4 ? kq_byte(h, b + 4) & 63u : (kq_byte(h, b + 4) >> 4) | ((kq_byte(h, b) >> 6) << 4);
 }
 
-// The float codebook of DequantizeIQ4NL split into fp16 parts, as byte planes of 16 entries.
+// The float codebook of DequantizeIQ4NL, times 2^12, in fp16 parts: byte planes of 16 entries.
+template <int PW>
 struct IQ4Planes {
-    uint32_t t[4][4];  // [hi part high byte, hi part low byte, lo part high byte, lo part low byte][entry / 4]
+    uint32_t t[2 * PW][4];  // [part: its high byte, its low byte][entry / 4]
 };
 constexpr float kIQ4[16] = {-1.0f, -0.6961928f, -0.5250730f, -0.3947555f, -0.2831612f, -0.1790887f, -0.0805542f, 0.0f,
                             0.0805542f, 0.1790887f, 0.2831612f, 0.3947555f, 0.5250730f, 0.6961928f, 1.0f, 1.3312578f};
-// fp16 bits of v, rounded to nearest even (|v| below 2, normal or subnormal)
+// fp16 bits of v, rounded to nearest even (|v| below 2^15, normal or subnormal)
 constexpr uint32_t f16_bits(double v) {
     const uint32_t sign = v < 0 ? 0x8000u : 0u;
     double a = v < 0 ? -v : v;
@@ -357,40 +358,55 @@ constexpr double f16_value(uint32_t b) {
     for (int i = 25; i < (e ? e : 1); i++) m *= 2;
     return b & 0x8000u ? -m : m;
 }
-constexpr IQ4Planes iq4_planes() {
-    IQ4Planes p = {};
+// v rounded to 8 bits
+constexpr double bits8(double v) {
+    double u = 1;
+    while (u * 256 <= (v < 0 ? -v : v)) u *= 2;
+    while (u * 128 > (v < 0 ? -v : v) && v != 0) u /= 2;
+    return (double)(long)(v / u + (v < 0 ? -0.5 : 0.5)) * u;
+}
+template <int PW>
+constexpr IQ4Planes<PW> iq4_planes() {
+    IQ4Planes<PW> p = {};
     for (int i = 0; i < 16; i++) {
-        const uint32_t h = f16_bits(kIQ4[i]), l = f16_bits((double)kIQ4[i] - f16_value(h));
-        const uint32_t by[4] = {h >> 8, h & 255, l >> 8, l & 255};
-        for (int q = 0; q < 4; q++) p.t[q][i >> 2] |= by[q] << (8 * (i & 3));
+        double v = 4096.0 * kIQ4[i];
+        for (int z = 0; z < PW; z++) {
+            const uint32_t h = f16_bits(PW == 3 && z == 0 ? bits8(v) : v);
+            p.t[2 * z][i >> 2] |= (h >> 8) << (8 * (i & 3));
+            p.t[2 * z + 1][i >> 2] |= (h & 255) << (8 * (i & 3));
+            v -= f16_value(h);
+        }
     }
     return p;
 }
 static_assert(f16_bits(1.0) == 0x3c00 && f16_bits(-0.5) == 0xb800 && f16_value(0x3c01) == 1.0009765625, "fp16");
 
-// Four codebook entries (selectors 0-15 in a dword's bytes): the hi and lo parts, two dwords of halves each.
-__device__ __forceinline__ void iq4_lookup(uint32_t sel, half2v (&hi)[2], half2v (&lo)[2]) {
-    constexpr IQ4Planes T = iq4_planes();
+// Four codebook entries (selectors 0-15 in a dword's bytes): two dwords of halves of each part.
+template <int PW>
+__device__ __forceinline__ void iq4_lookup(uint32_t sel, half2v (&o)[PW][2]) {
+    constexpr IQ4Planes<PW> T = iq4_planes<PW>();
     const uint32_t s7 = sel & 0x07070707u;
     const uint32_t up = ((sel >> 3) & 0x01010101u) * 255u;  // byte mask of the entries 8-15
-    uint32_t pl[4];
+    uint32_t pl[2 * PW];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
+    for (int q = 0; q < 2 * PW; q++) {
         const uint32_t a = __builtin_amdgcn_perm(T.t[q][1], T.t[q][0], s7), b = __builtin_amdgcn_perm(T.t[q][3], T.t[q][2], s7);
         pl[q] = (b & up) | (a & ~up);
     }
-    hi[0] = as_half2(__builtin_amdgcn_perm(pl[0], pl[1], 0x05010400u));
-    hi[1] = as_half2(__builtin_amdgcn_perm(pl[0], pl[1], 0x07030602u));
-    lo[0] = as_half2(__builtin_amdgcn_perm(pl[2], pl[3], 0x05010400u));
-    lo[1] = as_half2(__builtin_amdgcn_perm(pl[2], pl[3], 0x07030602u));
+#pragma unroll
+    for (int z = 0; z < PW; z++) {
+        o[z][0] = as_half2(__builtin_amdgcn_perm(pl[2 * z], pl[2 * z + 1], 0x05010400u));
+        o[z][1] = as_half2(__builtin_amdgcn_perm(pl[2 * z], pl[2 * z + 1], 0x07030602u));
+    }
 }
 
-// Decoded weights of one row tile and 32-K step: the exact value is hi (+ lo), times the scale.
-constexpr int parts_of(Fmt f) { return f == Q6_K || f == IQ4_NL ? 2 : 1; }
+// Decoded weights of one row tile and 32-K step: the exact value is the sum of the parts (P: the activations'), times
+// the scale.  (IQ4_NL: 24 bits; to 22 with fp16 activations.)
+constexpr int parts_of(Fmt f, int P) { return f == IQ4_NL ? P + 1 : f == Q6_K ? 2 : 1; }
 constexpr bool unit_scaled(Fmt f) { return f == W4A16 || f == Q4_K || f == Q5_K || f == Q6_K; }  // one scale per 128-K unit
 
-template <Fmt F>
-__device__ __forceinline__ void decode(const Raw& r, int b, int u, int lg, half2v z1, half2v z2, half8v (&o)[parts_of(F)]) {
+template <Fmt F, int PW>
+__device__ __forceinline__ void decode(const Raw& r, int b, int u, int lg, half2v z1, half2v z2, half8v (&o)[PW]) {
     constexpr uint32_t M = 0x64006400u;  // 1024 in both halves: M | n is 1024 + n
     const half2v k16 = splat2(0.0625f);
     if constexpr (F == W4A16 || F == Q4_0) {
@@ -454,11 +470,11 @@ __device__ __forceinline__ void decode(const Raw& r, int b, int u, int lg, half2
         o[0] = join(h[0], h[1], h[2], h[3]);
         o[1] = join(l[0], l[1], l[2], l[3]);
     } else {  // IQ4_NL: byte j's elements 2 j and 2 j + 1
-        half2v h0[2], l0[2], h1[2], l1[2];
-        iq4_lookup(r.a[b] & 0x0F0F0F0Fu, h0, l0);
-        iq4_lookup((r.a[b] >> 4) & 0x0F0F0F0Fu, h1, l1);
-        o[0] = join(h0[0], h0[1], h1[0], h1[1]);
-        o[1] = join(l0[0], l0[1], l1[0], l1[1]);
+        half2v e[PW][2], f[PW][2];
+        iq4_lookup<PW>(r.a[b] & 0x0F0F0F0Fu, e);
+        iq4_lookup<PW>((r.a[b] >> 4) & 0x0F0F0F0Fu, f);
+#pragma unroll
+        for (int z = 0; z < PW; z++) o[z] = join(e[z][0], e[z][1], f[z][0], f[z][1]);
     }
 }
 
@@ -466,7 +482,7 @@ __device__ __forceinline__ void decode(const Raw& r, int b, int u, int lg, half2
 template <Fmt F>
 __device__ __forceinline__ float block_scale(const Raw& r, int b, int u) {
     if constexpr (F == Q8_0) return __uint_as_float(r.s[b]);
-    else return h2f((uint16_t)(r.s[b >> 1] >> (16 * (b & 1))));
+    else return h2f((uint16_t)(r.s[b >> 1] >> (16 * (b & 1)))) * (F == IQ4_NL ? 0x1p-12f : 1.0f);
 }
 
 // The whole part of a W4A16 zero that goes into the operand q - zero (exact in fp16), 0 for large or non-finite zeros.
@@ -490,7 +506,7 @@ constexpr bool far_sums(Fmt f) { return f == IQ4_NL || f == Q5_0; }
 template <Fmt F, int P, int MT, int NT, int WN, int WK, bool FAR>
 __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideArgs p) {
     constexpr int KSU = steps_of(P);
-    constexpr int PW = parts_of(F);
+    constexpr int PW = parts_of(F, P);
     constexpr int UB = MT * KSU * P * 1024;  // bytes of one K group's stage
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -620,10 +636,20 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideAr
                             ao[q] = *reinterpret_cast<const half8v*>(xs + (i * P + q) * (KSU * 1024) + xo[s]);
 #pragma unroll
                         for (int j = 0; j < NT; j++) {
-                            float4v v = unit_scaled(F) && blk > 0 ? d[i][j] : (float4v){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                            for (int q = 0; q < P; q++) v = __builtin_amdgcn_mfma_f32_16x16x32_f16(ao[q], bo[j][0], v, 0, 0, 0);
-                            if constexpr (PW == 2) v = __builtin_amdgcn_mfma_f32_16x16x32_f16(ao[0], bo[j][PW - 1], v, 0, 0, 0);
+                            auto times = [&](int q, int w, float4v c) {
+                                return __builtin_amdgcn_mfma_f32_16x16x32_f16(ao[q < P ? q : 0], bo[j][w < PW ? w : 0], c, 0, 0, 0);
+                            };
+                            constexpr float4v none = {0.f, 0.f, 0.f, 0.f};
+                            float4v v;
+                            if constexpr (PW == 3) {
+                                // 11 x 8 bits: sums of these are (nearly) exact, and the others, of 2^-8 of it and
+                                // less, join them in one rounding
+                                v = times(0, 0, none) + times(0, 1, times(1, 0, times(0, 2, times(1, 1, none))));
+                            } else {
+                                v = times(0, 0, unit_scaled(F) && blk > 0 ? d[i][j] : none);
+                                if constexpr (P == 2) v = times(1, 0, v);
+                                if constexpr (PW == 2) v = times(0, 1, v);
+                            }
                             if constexpr (unit_scaled(F)) {
                                 d[i][j] = v;
                             } else {
@@ -784,7 +810,7 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) wide_gemm_kernel(const WideAr
 template <Fmt F, int NT, int WK>
 __global__ void __launch_bounds__(64 * WK, 2) few_gemm_kernel(const WideArgs p) {
     static_assert(F == W4A16 || F == IQ4_NL, "16-byte blocks, fp16 activations");
-    constexpr int PW = parts_of(F), SD = F == W4A16 ? 1 : 2;  // 16-byte scale loads of a row and quad
+    constexpr int PW = parts_of(F, 1), SD = F == W4A16 ? 1 : 2;  // 16-byte scale loads of a row and quad
     constexpr int RB = 4096 * (1 + NT);                       // LDS of a wave: one activation unit, NT weight quads
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
