@@ -278,14 +278,15 @@ def test_error_of_fp32_tokens_on_iq4nl(eng, orc, K, T):
                                           ("mmap_q4_0", 64, 512, 8), ("mmap_q5_k", 64, 512, 6), ("q4_k", 64, 512, 20),
                                           ("iq4_nl_f16", 64, 5120, 8)])
 def test_tiled_tokens_build_a_copy_only_at_no_risk(eng, orc, fmt, rows, K, T):
-    """Where the columns need no tiled copy the tokens make one, but neither in a capture nor at the memory limit;
-    both ways give the result."""
+    """Where the columns need no tiled copy the tokens make one, but neither in a capture nor at the memory limit, nor
+    where the engine was told not to; both ways give the result."""
     s, w = weights(fmt, rows, K, rows + T, orc)
     x = activations(fmt, T, K, T)
     xd = torch.from_numpy(x).cuda()
     careful = ROCmEngine(split_reserve_bytes=1 << 60)
-    check(careful.matmul(xd, st.Tensor((K, rows), s)).cpu().numpy(), x, w)
-    assert getattr(s, "_gpu_tiled", None) is None
+    for e in (careful, ROCmEngine(token_copies=False)):
+        check(e.matmul(xd, st.Tensor((K, rows), s)).cpu().numpy(), x, w)
+        assert getattr(s, "_gpu_tiled", None) is None
     side = torch.cuda.Stream()
     cap = ROCmEngine(stream=side)
     torch.cuda.synchronize()

@@ -86,12 +86,15 @@ def _tiled_cached(s: Any, key: tuple):
 
 class ROCmEngine:
     def __init__(self, device: int = 0, stream: torch.cuda.Stream | None = None, q6k_split: bool = True,
-                 split_reserve_bytes: int = 1 << 30):
+                 split_reserve_bytes: int = 1 << 30, token_copies: bool = True):
         """q6k_split: Q6_K batch 1 on a split copy of the super-blocks (35-55%
         faster; it doubles the resident Q6_K bytes).  The copy is built only
         while at least split_reserve_bytes of device memory stay free after
         it; otherwise, or with q6k_split=False, batch 1 reads the raw
-        super-blocks."""
+        super-blocks.  token_copies: 2 to 32 tokens on a tiled copy also where
+        another GEMM runs them on the upload layout (faster from the second
+        call on; the copy is as large as the weight); with token_copies=False
+        such a call makes none, and a copy that is there is used."""
         if not torch.cuda.is_available():
             raise RuntimeError("ROCmEngine needs a ROCm GPU (torch.cuda.is_available() is False)")
         self.device = torch.device("cuda", device)
@@ -99,6 +102,7 @@ class ROCmEngine:
         self.lib = _lib.load()
         self.q6k_split = q6k_split
         self.split_reserve_bytes = split_reserve_bytes
+        self.token_copies = token_copies
 
     @property
     def _s(self) -> int:
@@ -363,9 +367,9 @@ class ROCmEngine:
         23.8 / 23.4; W4A16 8192 x 8192 18.0 / 21.5, 4096 x 14336 15.7 / 26.2;
         IQ4_NL 22.1 / 26.5, 19.9 / 26.8).  None for a type or size that has no tiled copy; and
         where a call needs none (the row-block GEMMs, padded counts of a
-        mapped file, more than 16 tokens), unless it is there or can be made at no risk: with
-        memory to spare, and not while a graph is captured, whose pool the
-        copy would be left in."""
+        mapped file, more than 16 tokens), unless it is there or may be made
+        (token_copies) at no risk: with memory to spare, and not while a graph
+        is captured, whose pool the copy would be left in."""
         t = x.shape[0]
         n = -(-t // 4) * 4
         mm = s.qtype if isinstance(s, MmapStorage) else None
@@ -395,7 +399,7 @@ class ROCmEngine:
             self.upload_weights([s])
         buf = s.gpu_ptr()
         if ((rowblock or t > 16 or (mm is not None and t != n)) and _tiled_cached(s, (f + "t", rows, k, _p(buf.tensor))) is None
-                and (torch.cuda.is_current_stream_capturing()
+                and (not self.token_copies or torch.cuda.is_current_stream_capturing()
                      or torch.cuda.mem_get_info(self.device)[0] < 2 * rows * k + self.split_reserve_bytes)):
             return None
         x = x.contiguous()
