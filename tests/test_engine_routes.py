@@ -99,3 +99,16 @@ def test_copies_made_in_a_capture_are_not_kept(monkeypatch, capturing):
     assert (eng._q6k_split_copy(s, 0, 16, 256) is None) == capturing  # (the GEMV then reads the super-blocks)
     assert (getattr(s, "_gpu_split", None) is None) == capturing
     assert eng._q6k_split_copy(storage(), 0, 16, 256, for_one_call=True) is not None
+
+
+@pytest.mark.parametrize("rows,k,wide", [(1024, 1024, True), (20480, 1024, True), (6144, 1536, True), (8448, 1536, False),
+                                         (4096, 2048, True), (10240, 2048, False), (16384, 2048, True), (20480, 2048, False),
+                                         (4096, 3072, False), (8448, 4096, False), (14336, 4096, False)])
+def test_w4a16_tokens_on_the_faster_gemm(rows, k, wide):
+    """17 to 32 tokens: the side that measured faster, at both ends of the rule's rows and K."""
+    from ztensor_amd.engine import _few_tokens
+
+    s = object.__new__(st.GPTQStorage)
+    for t in (17, 32):
+        assert _few_tokens(s, rows, k, torch.empty(t, k, dtype=torch.float16)) == wide
+        assert not _few_tokens(s, rows, k, torch.empty(t, k))

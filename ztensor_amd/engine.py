@@ -380,8 +380,6 @@ class ROCmEngine:
         if isinstance(s, (GPTQStorage, AWQStorage)):
             if not half or s.group_size % 128 != 0 or rows * (k // s.group_size) >= 1 << 29:
                 return None
-            if t > 16 and 8192 < rows <= 16384 and k <= 4096:
-                return None  # one nearly full round of the wide GEMM: 14336 x 4096, 32 tokens 17.5 us against 19.2
             f, rowblock = "w4a16", _w4a16_rowblock(rows, k, n)
         elif isinstance(s, IQ4NLStorage):
             if not half:
@@ -968,6 +966,22 @@ def _block_rowblock(fmt: str, rows: int, k: int, n: int) -> bool:
     return rows * k <= 4096 * 4096 and (fmt == "q4" or n == 4)
 
 
+def _w4a16_wide(rows: int, k: int) -> bool:
+    """Whether 17 to 32 W4A16 tokens run faster on the wide GEMM than on the
+    tiled copy. Its workgroups walk all of K and spread rows over tiles of 16,
+    32 or 64, the smallest that the 256 CUs take at once, so it wins while K is
+    short, up to 2048 the more of the CUs those tiles fill. Measured (us, 24
+    tokens, wide against tiled): K = 512: 1024 rows 5.2 / 5.8, 8192 6.5 / 8.6,
+    28672 10.3 / 14.7; 1024: 5.9 / 6.0, 7.6 / 9.2, 14.1 / 16.5; 1536: 1024 rows
+    6.3 / 6.1, 6144 8.1 / 8.6, 8448 9.7 / 9.5, 10240 10.0 / 10.3, 12288 10.5 /
+    12.1, 20480 16.0 / 14.4; 2048: 1024 rows 7.0 / 6.4, 4096 7.6 / 8.1, 6144
+    9.3 / 9.1, 8192 9.5 / 10.6, 10240 13.0 / 12.2, 14336 13.4 / 13.7, 16384
+    13.5 / 14.7, 20480 20.4 / 17.1; 3072: 4096 rows 9.0 / 8.6, 16384 17.9 /
+    16.8; 4096: 8448 rows 20.1 / 13.5, 14336 21.2 / 18.9, 16384 21.6 / 20.9."""
+    tiles = next((-(-rows // r) for r in (16, 32, 64) if rows <= 256 * r), 0)
+    return k <= 1024 or (k <= 2048 and 32 * tiles > 3 * k)
+
+
 def _w4a16_rowblock(rows: int, k: int, n: int) -> bool:
     """Whether a batch of 4-16 W4A16 columns runs faster on the single-launch
     row-block GEMM over the row-major upload (zt_gemm_w4a16sz_f32) than on the
@@ -1016,19 +1030,22 @@ def _wide_tokens(t: int, transposed: bool = False) -> bool:
 
 
 def _few_tokens(s: Any, rows: int, k: int, x: torch.Tensor) -> bool:
-    """Whether 2 to 16 tokens x[t, k] go to the token-major GEMM on the upload
-    layout before the tiled copy's is tried.  fp16 tokens (one launch, against
-    a GEMM and the sum of its K ranges): while K is short enough for one
-    workgroup's walk and the matrix small (us, against the tiled copy: W4A16
-    4096 x 4096 6.0 / 7.0, 8192 x 4096 8.1 / 8.6, 2048 x 8192 9.1 / 6.8, 14336
-    x 4096 14.4 / 12.9; IQ4_NL 8192 x 2048 8.5 / 9.0, 6144 x 4096 11.4 / 10.4),
-    and past 8 tokens up to 4096 rows (more have a tiled copy from the
-    columns).  fp32 tokens on IQ4_NL, which has no other kernel of that shape:
-    the counts the column kernel is slow at (14336 x 4096, us against it: 3
-    tokens 27 / 63, 4 28 / 21, 8 28 / 31, 16 28 / 56)."""
+    """Whether 2 to 32 tokens x[t, k] go to the token-major GEMM on the upload
+    layout before the tiled copy's is tried. Past 16: W4A16 by _w4a16_wide.
+    fp16 tokens (one launch, against a GEMM and the sum of its K ranges): while
+    K is short enough for one workgroup's walk and the matrix small (us,
+    against the tiled copy: W4A16 4096 x 4096 6.0 / 7.0, 8192 x 4096 8.1 / 8.6,
+    2048 x 8192 9.1 / 6.8, 14336 x 4096 14.4 / 12.9; IQ4_NL 8192 x 2048 8.5 /
+    9.0, 6144 x 4096 11.4 / 10.4), and past 8 tokens up to 4096 rows (more have
+    a tiled copy from the columns). fp32 tokens on IQ4_NL, which has no other
+    kernel of that shape: the counts the column kernel is slow at (14336 x
+    4096, us against it: 3 tokens 36 / 63, 4 36 / 21, 8 36 / 31, 16 36 /
+    56)."""
     t = x.shape[0]
-    if not 2 <= t <= 16 or not isinstance(s, (GPTQStorage, AWQStorage, IQ4NLStorage)):
+    if not 2 <= t <= 32 or not isinstance(s, (GPTQStorage, AWQStorage, IQ4NLStorage)):
         return False
+    if t > 16:
+        return not isinstance(s, IQ4NLStorage) and x.dtype == torch.float16 and _w4a16_wide(rows, k)
     if x.dtype != torch.float16:
         return isinstance(s, IQ4NLStorage) and (t % 4 != 0 or t > 8)
     return (k <= 4096 and rows * k <= 1 << (24 if isinstance(s, IQ4NLStorage) else 25)
