@@ -360,7 +360,7 @@ int zt_gemm_w4a16t_f32(const void* W_tiled, const uint32_t* sz, const uint16_t* 
  *   [16 rows][4 blocks].  Rows past M, to the next multiple of 16, are zero.
  * K % 128 == 0, W_tiled / S_tiled / B 16-byte aligned, N in {4, 8, 12, 16},
  * else InvalidValue.  Activations are split into two fp16 parts after a
- * power-of-two normalisation (about 2^-22 relative precision each).  When
+ * power-of-two normalisation of their column (2^-23 relative precision).  When
  * K is split across workgroups the partial tiles go to the caller's
  * workspace (16-byte aligned, at least zt_gemm_q{4,8}t_workspace_bytes(M,
  * K, N) bytes, which is 0 when K is not split; a smaller or NULL workspace
@@ -587,9 +587,10 @@ void zt_q5_0_raw_to_gpu(const void* raw, long nblk, void* out);
  *   ZT_WIDE_Q4_K, ZT_WIDE_Q5_K   the raw super-blocks;
  *   ZT_WIDE_Q6_K     zt_q6k_split;
  *   ZT_WIDE_IQ4_NL   zt_iq4nl_raw_to_gpu, offset1 = the data offset, fp16 or fp32 X.
- * The others take fp32 X.  Weights enter as exact fp16 integers (IQ4_NL's
- * codebook and Q6_K's scaled values as fp16 hi + lo), fp32 activations as
- * fp16 hi + lo after a power-of-two scale per token, sums are fp32; every
+ * The others take fp32 X.  Weights enter as exact fp16 integers (Q6_K's scaled
+ * values as fp16 hi + lo; IQ4_NL's codebook to 22 bits, with fp32 X to all 24),
+ * fp32 activations as fp16 hi + lo after a power-of-two scale per token, within
+ * 2^-23 of each value and 2^-39 of the token's largest; sums are fp32.  Every
  * output is written once and repeats bit for bit.  Up to 16 tokens of fp16 X
  * are multiplied as they are, in one launch; the others are packed first.  K
  * % 128 == 0 (K-quants: 256), K <= 32768, bulk data below 2^31 bytes; W, X, the offsets and the

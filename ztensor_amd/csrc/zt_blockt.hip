@@ -20,9 +20,10 @@
 //    1.1e-7, Q8_0 3.4e-7 and 1.2e-7, Q6_K 2.3e-7 and 1.2e-7, Q4_K 1.7e-7 and
 //    1.3e-7; 4096 x 14336 Q6_K 28.6 us and now 26.9, Q8_0 25.8 and 24.8.)
 //  * fp32 activations are split into two fp16 parts, x = hi + lo, after a
-//    power-of-two normalisation per workgroup (max |x| of the workgroup's K
-//    range maps into [2^14, 2^15)), so each activation is carried to about
-//    2^-22 relative precision over the whole fp32 range; the normalisation
+//    power-of-two normalisation per token or column (max |x| of its finite
+//    values in the workgroup's K range maps into [2^14, 2^15)), so each
+//    activation is carried to 2^-23 over the whole fp32 range whatever the
+//    others of the batch are (zt_mfma.h); the normalisation
 //    is undone exactly at the end.  For N <= 8 the hi parts sit in B columns
 //    0..N-1 and the lo parts in columns 8..8+N-1 of the same MFMA, and the
 //    two column halves are added once at the end; for N > 8 hi and lo are

@@ -105,6 +105,12 @@ struct MaxRows {
     }
 };
 
+// 8 halves in the A operand's order of a dword's nibbles: e0 e4 e1 e5 e2 e6 e3 e7
+__device__ __forceinline__ u32x4 nibble_order(const u32x4& o) {
+    return (u32x4){__builtin_amdgcn_perm(o[2], o[0], 0x05040100u), __builtin_amdgcn_perm(o[2], o[0], 0x07060302u),
+                   __builtin_amdgcn_perm(o[3], o[1], 0x05040100u), __builtin_amdgcn_perm(o[3], o[1], 0x07060302u)};
+}
+
 constexpr int kMfmaRows = 32;                         // rows per workgroup (two 16-row tiles)
 constexpr int kMfmaTiles = kMfmaRows / 16;
 constexpr int kMfmaWaves = 8;                         // waves per workgroup

@@ -1091,12 +1091,6 @@ __global__ void w4t_sz_kernel(const uint16_t* __restrict__ scales, const uint16_
     sz[e] = (uint32_t)s | ((uint32_t)z << 16);
 }
 
-// 8 halves in the A operand's order of a dword's nibbles: e0 e4 e1 e5 e2 e6 e3 e7
-__device__ __forceinline__ u32x4 nibble_order(const u32x4& o) {
-    return (u32x4){__builtin_amdgcn_perm(o[2], o[0], 0x05040100u), __builtin_amdgcn_perm(o[2], o[0], 0x07060302u),
-                   __builtin_amdgcn_perm(o[3], o[1], 0x05040100u), __builtin_amdgcn_perm(o[3], o[1], 0x07060302u)};
-}
-
 // Small-batch W4A16 GEMM on the tiled layout (N in {4, 8, 12, 16}, K % 128 == 0,
 // group size % 128 == 0).  A workgroup of W waves owns 32 W rows (two 16-row
 // tiles a wave) and a K range of UPW 128-K units; K ranges are split across

@@ -8,18 +8,21 @@
 // stages them with direct global-to-LDS loads of 1 KB and reads them back
 // with conflict-free ds_read_b128.  fp16 activations are one part, exact;
 // fp32 activations are scaled by a power of two of their token (max |x| in
-// [2^14, 2^15)) and split into fp16 hi + lo, |x - hi - lo| <= 2^-24 |x| +
-// 2^-25 after scaling.
+// [2^14, 2^15)) and split into fp16 hi + lo, |x - hi - lo| <= 2^-23 |x| +
+// 2^-25 after scaling (zt_mfma.h).
 //
 // The GEMM's MFMA A operand is the activations (16 tokens) and the B operand
 // the weights (16 rows), so D lane 16 g + i holds 4 tokens of weight row i:
 // one register per lane scales the 4 values, and the lane that decodes a
 // row's weights is the lane that uses the row's scale.  Weights go from
 // global memory to registers and are decoded there to exact fp16 integers
-// (q - 8, q - zero, sc * q as hi + lo, ...): the products are exact, only the
-// fp32 sums round.  A wave covers MT token tiles by NT row tiles, so that a
-// decoded operand feeds MT x parts MFMAs; WN waves lie along the rows and WK
-// along K (their sums meet through LDS at the end).
+// (q - 8, q - zero, q times a 6-bit scale, ...), so that only the activations'
+// split and the fp32 sums round.  Two formats need parts: Q6_K's scale times q
+// (hi + lo; the product of both second parts, at most 2^-22 of the whole, is
+// left out) and IQ4_NL's float codebook (22 bits of it with fp16 activations,
+// all 24 with fp32 ones).  A wave covers MT token tiles by NT row tiles, so
+// that a decoded operand feeds MT x parts MFMAs; WN waves lie along the rows
+// and WK along K (their sums meet through LDS at the end).
 #include <type_traits>
 
 #include "zt_common.h"
@@ -899,8 +902,7 @@ __global__ void __launch_bounds__(64 * WK, 2) few_gemm_kernel(const WideArgs p) 
                 for (int b = 0; b < 4; b++) {
                     const u32x4 o = *reinterpret_cast<const u32x4*>(xs + get[b]);
                     const u32x4 e = F == W4A16
-                        ? (u32x4){__builtin_amdgcn_perm(o[2], o[0], 0x05040100u), __builtin_amdgcn_perm(o[2], o[0], 0x07060302u),
-                                  __builtin_amdgcn_perm(o[3], o[1], 0x05040100u), __builtin_amdgcn_perm(o[3], o[1], 0x07060302u)}
+                        ? nibble_order(o)
                         : (u32x4){__builtin_amdgcn_perm(o[1], o[0], 0x05040100u), __builtin_amdgcn_perm(o[3], o[2], 0x05040100u),
                                   __builtin_amdgcn_perm(o[1], o[0], 0x07060302u), __builtin_amdgcn_perm(o[3], o[2], 0x07060302u)};
                     ao[b] = __builtin_bit_cast(half8v, e);
@@ -1023,9 +1025,9 @@ hipError_t launch_tile(const WideArgs& a, hipStream_t st) {
 // the chain of loads and barriers along K, so the smallest tile whose
 // workgroups still fit the 256 CUs wins, with as many waves along K as the
 // registers and LDS allow (16 waves against 8 in 64 x 128 tiles, K = 4096 /
-// 14336, 512 tokens of 4096 rows: Q4_0 54 / 159 us against 61 / 179, Q4_K
-// 64 / 183 against 78 / 234, W4A16 35 / 91 against 37 / 106; Q6_K's decode
-// would spill there and stays at 8 waves).  Past one round the tile that
+// 14336, 512 tokens of 4096 rows: Q4_0 54 / 159 us against 61 / 179, W4A16 35
+// / 91 against 37 / 106; Q6_K's decode and the second sums of IQ4_NL and Q5_0
+// would spill there and stay at 8 waves).  Past one round the tile that
 // feeds most MFMAs a decoded weight and stage wins, as long as its last round
 // is full enough: 128 x 256 in 8 waves (14336 x 4096 rows x K, us against 64
 // x 128 in 4 waves: 512 tokens W4A16 76 / 104, Q4_0 147 / 152, Q6_K 183 /
